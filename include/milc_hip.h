@@ -41,7 +41,9 @@ extern "C" {
  * mixed_precision: 0 = solve entirely in internal precision; 1 = FP32 sloppy
  * iterations with FP64 reliable updates; 2 = 16-bit (per-site normed) sloppy
  * iterations with FP64 reliable updates (MILC's HALF_MIXED / MAX_MIXED,
- * Makefile:463-466). */
+ * Makefile:463-466).  On lattices of at most 49152 sites per parity a CG runs
+ * in FP64 throughout whatever mixed_precision asks for (it is the fastest form
+ * there), to the same FP64 true residual. */
 typedef struct {
   int max_iter;
   int evenodd;
@@ -390,7 +392,8 @@ int milc_hip_dev_invert(int slot_b, int slot_x, double mass, int parity, double 
  * milc_hip_dev_write, milc_hip_dev_source or an earlier solve) and the links of
  * the sloppy precision are resident (one milc_hip_dev_invert with the same
  * mixed_precision after the links were loaded builds them).  Work vectors
- * needing more than 256 MiB (FP64: 4 x 48 B, mixed: 200 B per site of one
+ * needing more than 256 MiB (FP64: 4 x 48 B (5 x 48 B up to 131072 sites per
+ * parity), mixed: 200 B per site of one
  * parity, i.e. up to about 2.6M lattice sites mixed, 2.8M FP64) return -6
  * with a message.  parity must be EVEN or ODD (else -2).  Same results and
  * stats as milc_hip_dev_invert.  Calls share the array, so calls that overlap

@@ -13,6 +13,7 @@
 #include "../../include/milc_hip.h"
 #include "mh_batch.h"
 #include "mh_internal.h"
+#include "mh_persist.h"
 
 using namespace mh;
 
@@ -167,6 +168,7 @@ int milc_hip_init(const int dims[4], int device) {
   rc = dev_alloc((void**)&c.ws.partials, (size_t)c.ws.max_blocks * 4 * 2 * sizeof(double));
   if (rc) return rc;
   if ((rc = dev_alloc((void**)&c.ws.scal, sizeof(CGScalars)))) return rc;
+  if ((rc = dev_alloc((void**)&c.ws.flags, kPersistFlagBytes))) return rc;
   MH_CHECK(hipHostMalloc((void**)&c.ws.scal_host, sizeof(CGScalars), hipHostMallocDefault));
   // pinned read-back space for one partial record per block (vec_norm2)
   if (!pinned_scratch((size_t)c.ws.max_blocks * 4 * sizeof(double))) return -5;
@@ -194,6 +196,7 @@ int milc_hip_finalize(void) {
   c.thin_valid = false;
   dev_free(c.ws.partials);
   dev_free(c.ws.scal);
+  dev_free(c.ws.flags);
   if (c.ws.scal_host) (void)hipHostFree(c.ws.scal_host);
   if (c.ws.pinned) (void)hipHostFree(c.ws.pinned);
   dev_free(c.staging);
@@ -311,7 +314,7 @@ static int dev_invert_impl(int slot_b, int slot_x, double mass, int parity, doub
   if (noalloc) {
     if (parity != EVEN && parity != ODD) return -2;
     if (!g_slots[slot_x].data || !c.links[P_F64].valid || !c.links[ps].valid) return -3;
-    size_t need = cg_scratch_bytes(ps, c.stride);
+    size_t need = cg_scratch_bytes(ps, c.Vh, c.stride);
     if (need > kScratchBytes) {
       fprintf(stderr, "milc_hip_dev_invert_noalloc: %zu bytes of work vectors needed, scratch holds %zu\n", need,
               kScratchBytes);

@@ -14,6 +14,7 @@
 
 #include "mh_dslash.h"
 #include "mh_internal.h"
+#include "mh_persist.h"
 
 namespace mh {
 
@@ -1053,7 +1054,9 @@ static double batch_rate(double log_rate, double rsq_before, double rsq_now, int
 // with the optional Fermilab relative residual: its target is met when
 // my_relative_residue < relresid^2 (relrsqmin, :92), tested beside the
 // residual at every restart block (:213-220) and after every update (:351-354).
-static int cg_solve_f64(const VecField& src, VecField& x, double mass, const SolveParams& sp, SolveStats& st) {
+// niter: iterations between restarts; max_cg, max_restarts: limits of the solve.
+static int cg_solve_f64(const VecField& src, VecField& x, double mass, const SolveParams& sp, int niter, long max_cg,
+                        int max_restarts, SolveStats& st) {
   Context& c = ctx();
   const DevLinks& L = c.links[P_F64];
   if (!L.valid) return -3;
@@ -1062,8 +1065,6 @@ static int cg_solve_f64(const VecField& src, VecField& x, double mass, const Sol
   double rsqmin = sp.resid * sp.resid;
   double relrsqmin = sp.relresid * sp.relresid;
   const bool rel = relrsqmin > 0;
-  int niter = sp.max_iters, max_restarts = sp.max_restarts;
-  long max_cg = (long)max_restarts * niter;
   st = SolveStats();
   double source_norm;
   int rc = vec_norm2(src, P_F64, &source_norm);
@@ -1072,10 +1073,12 @@ static int cg_solve_f64(const VecField& src, VecField& x, double mass, const Sol
     st.converged = 1;
     return vec_zero(x, P_F64);
   }
-  VecField ttt, p, r, tmp;
-  VecScope owned{&ttt, &p, &r, &tmp};
+  const bool one_kernel = !rel && persist_shape(c.Vh).lps > 0;
+  VecField ttt, p, r, tmp, extra;
+  VecScope owned{&ttt, &p, &r, &tmp, &extra};
   if ((rc = alloc_vec(ttt, P_F64, c.stride)) || (rc = alloc_vec(p, P_F64, c.stride)) ||
-      (rc = alloc_vec(r, P_F64, c.stride)) || (rc = alloc_vec(tmp, P_F64, c.stride)))
+      (rc = alloc_vec(r, P_F64, c.stride)) || (rc = alloc_vec(tmp, P_F64, c.stride)) ||
+      (one_kernel && (rc = alloc_vec(extra, P_F64, c.stride))))
     return rc;
   CGScalars h;
   memset(&h, 0, sizeof h);
@@ -1105,6 +1108,18 @@ static int cg_solve_f64(const VecField& src, VecField& x, double mass, const Sol
     long left = niter - (iteration % niter);
     if (left == niter) left = 0;
     left = std::min(left, max_cg - iteration);
+    if (one_kernel) {
+      VecField work[4] = {p, tmp, ttt, extra};
+      if ((rc = cg_persist(x, r, work, pb, msq_x4, (int)std::min<long>(left, 1L << 30)))) break;
+      if ((rc = read_scalars(&h))) break;
+      if (h.iters < 0) {
+        rc = -8;
+        break;
+      }
+      iteration += h.iters;
+      size_r = h.rsq / source_norm;
+      continue;
+    }
     int nb_next = next_batch(batch, log_rate, h.rsq, h.rsq_stop, 16);
     while (left > 0) {
       int nb = (int)std::min<long>(nb_next, left);
@@ -1128,6 +1143,7 @@ static int cg_solve_f64(const VecField& src, VecField& x, double mass, const Sol
   st.size_r = size_r;
   st.iters = (int)iteration;
   st.restarts = nrestart;
+  st.reliable_updates = nrestart;
   // converged = the FP64 true residuals met the targets (the GPU glue's test,
   // d_congrad5_fn_gpu.c:153, with the relative residual of :92 when asked for)
   st.converged = met(final_rsq, final_relrsq) ? 1 : 0;
@@ -1310,16 +1326,21 @@ int cg_iteration_profile(const VecField& src, double mass, int parity, int reps,
 }
 
 // The work vectors cg_solve_f64 / cg_solve_mixed allocate, 256-byte aligned.
-size_t cg_scratch_bytes(int ps, int stride) {
+size_t cg_scratch_bytes(int ps, int Vh, int stride) {
   auto a = [&](int prec) { return (vec_bytes(prec, stride) + 255) & ~(size_t)255; };
-  if (ps == P_F64) return 4 * a(P_F64);
+  if (ps == P_F64 || Vh <= kPersistMixedSites) return (persist_shape(Vh).lps ? 5 : 4) * a(P_F64);
   return 2 * a(P_F64) + 2 * a(ps) + 3 * a(ps == P_H16 ? kH16Arith : P_F32);
 }
 
 int cg_solve(const VecField& src, VecField& x, double mass, const SolveParams& sp, SolveStats& st) {
   auto t0 = std::chrono::steady_clock::now();
   int rc;
-  if (sp.sloppy_prec == P_F64) rc = cg_solve_f64(src, x, mass, sp, st);
+  const long max_cg = (long)sp.max_restarts * sp.max_iters;
+  if (sp.sloppy_prec == P_F64) rc = cg_solve_f64(src, x, mass, sp, sp.max_iters, max_cg, sp.max_restarts, st);
+  // on a small lattice the FP64 loop in one kernel is the fastest solve for
+  // any sloppy precision: it restarts until the true residual meets the target
+  else if (sp.relresid <= 0 && ctx().Vh <= kPersistMixedSites && persist_shape(ctx().Vh).lps)
+    rc = cg_solve_f64(src, x, mass, sp, (int)std::min<long>(max_cg, 1L << 30), max_cg, 1 << 30, st);
   else if (sp.sloppy_prec == P_F32) rc = cg_solve_mixed<P_F32, P_F32>(src, x, mass, sp, st);
   else rc = cg_solve_mixed<P_H16, kH16Arith>(src, x, mass, sp, st);
   (void)hipStreamSynchronize(ctx().stream);

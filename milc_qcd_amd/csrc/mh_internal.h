@@ -38,6 +38,7 @@ struct Workspace {
   int max_blocks = 0;
   CGScalars* scal = nullptr;   // device
   CGScalars* scal_host = nullptr;  // pinned host mirror
+  unsigned* flags = nullptr;       // barrier words of the one-kernel solvers
   void* pinned = nullptr;          // pinned host scratch for small read-backs
   size_t pinned_bytes = 0;
 };
@@ -117,7 +118,7 @@ struct ScratchArena {
 // Work-vector bytes cg_solve takes from the arena for sloppy precision ps.
 // per-kernel times of the 16-bit mixed CG iteration in its own sequence (us[5])
 int cg_iteration_profile(const VecField& src, double mass, int parity, int reps, double us[5]);
-size_t cg_scratch_bytes(int ps, int stride);
+size_t cg_scratch_bytes(int ps, int Vh, int stride);
 // hand the pooled free blocks back to the device (end of context)
 void dev_pool_release();
 int alloc_vec(VecField& v, int prec, int stride);

@@ -1,0 +1,59 @@
+"""The Krylov loops that run in one kernel on small lattices (mh_persist.hip):
+every shape of the dispatch (lanes per site, threads per workgroup) at ragged
+sizes and at the edges of its range, on both parities.
+
+The FP64 CG is compared with the oracle's CG on the same links where that is
+quick: iteration counts within one, solutions within the residual times the
+condition number of the operator, 1 / (4 m^2) (times 10); everywhere its true
+residual, which other kernels compute, has to meet the target.  A mixed solve
+on a lattice above the one-kernel range of the mixed CG still goes through the
+sloppy iterations."""
+import numpy as np
+import pytest
+
+import ks_oracle as ko
+import milc_qcd_amd as mq
+
+pytestmark = pytest.mark.gpu
+
+# Vh = 128, 648, 4096 | 6000, 8192 | 13824, 16384 | 21168, 65536 | 68040, 131072
+SIZES = [(4, 4, 4, 4), (6, 6, 6, 6), (8, 8, 8, 16), (10, 10, 10, 12), (8, 8, 16, 16), (12, 12, 12, 16),
+         (16, 8, 16, 16), (18, 6, 14, 28), (16, 16, 16, 32), (18, 18, 14, 30), (16, 16, 32, 32)]
+
+
+@pytest.mark.parametrize("dims", SIZES)
+@pytest.mark.parametrize("parity", [mq.EVEN, mq.ODD])
+def test_cg_one_kernel(dims, parity):
+    mass, resid = 0.1, 1e-10
+    print(f"one-kernel CG {dims} parity {parity}", flush=True)
+    with mq.Lattice(dims) as G:
+        G.dev_gauge_hisq(1400)
+        G.dev_source(1401, parity, 0)
+        it, st = G.dev_invert(0, 1, mass, parity, resid, 0)
+        assert st["converged"] and st["resid"] < resid
+        # the same solve again, bit for bit
+        G.dev_invert(0, 2, mass, parity, resid, 0)
+        assert G.dev_diff(1, 2) == 0.0
+        itm, stm = G.dev_invert(0, 3, mass, parity, resid, 2)
+        assert stm["converged"] and stm["resid"] < resid
+        if G.V > 30000:
+            return
+        fat, lng = G.dev_read_links()
+        src, x = G.dev_read(0, parity), G.dev_read(1, parity)
+        L = ko.Lattice(dims)
+        ref, it_ref, _ = L.congrad(fat, lng, src, mass, resid, parity=parity, max_iters=20000)
+        s = L.parity_slice(parity)
+        assert abs(it - it_ref) <= 1
+        assert np.linalg.norm(x[s] - ref[s]) < 10 * resid / (4 * mass ** 2) * np.linalg.norm(ref[s])
+
+
+def test_mixed_cg_above_the_one_kernel_range():
+    dims = (16, 16, 16, 32)  # Vh = 65536
+    with mq.Lattice(dims) as G:
+        G.dev_gauge_hisq(1402)
+        G.dev_source(1403, mq.EVEN, 0)
+        _, ref = G.dev_invert(0, 1, 0.05, mq.EVEN, 1e-11, 0)
+        for mixed in (1, 2):
+            _, st = G.dev_invert(0, 2, 0.05, mq.EVEN, 1e-10, mixed)
+            assert st["converged"] and st["resid"] < 1e-10
+            assert G.dev_diff(2, 1) < 10 * 1e-10 / (4 * 0.05 ** 2)

@@ -619,8 +619,10 @@ extern "C" int milc_hip_multishift_invert(int external_precision, int internal_p
   if (rc) return rc;
   int pb = pbit(parity);
   bool mixed = args.mixed_precision != 0;
+  bool small = mixed && multishift_is_small() && args.max_iter != 1;
+  for (int j = 0; j < num_offsets; j++) small = small && (target_resid[j] > 0 ? target_resid[j] : target_resid[0]) > 0;
   int bulk = (internal_precision == 1 || mixed) ? P_F32 : P_F64;
-  if ((rc = ensure_links(bulk))) return rc;
+  if (!small && (rc = ensure_links(bulk))) return rc;
   VecField b;
   std::vector<VecField> xs(num_offsets);
   VecScope owned{&b};
@@ -639,24 +641,26 @@ extern "C" int milc_hip_multishift_invert(int external_precision, int internal_p
   mp.prec = bulk;
   mp.batch = 16;
   SolveStats st;
-  if ((rc = multicg_solve(b, xs, offs, mp, st))) return rc;
-  int total_iters = st.iters;
-  std::vector<double> fres(num_offsets, 0.0);
-  if (mixed) {
+  std::vector<double> fres(num_offsets, 0.0), res(num_offsets);
+  for (int j = 0; j < num_offsets; j++) res[j] = target_resid[j] > 0 ? target_resid[j] : target_resid[0];
+  long it = 0;
+  int conv = 1;
+  if (small) {
+    if ((rc = multishift_small(b, xs, offs, res.data(), parity, mp.max_iters, &it, fres.data(), &conv))) return rc;
+  } else if ((rc = multicg_solve(b, xs, offs, mp, st))) {
+    return rc;
+  }
+  if (mixed && !small) {
     // per-shift refinement: (offset_j - D D) x_j = b with mass = sqrt(offset_j)/2
     // (the mass <-> offset relation of ks_multicg.c:142,222), FP32 sloppy
     // operator (16-bit with mixed_precision 2), up to four shifts per batched CG
-    std::vector<double> res(num_offsets);
-    for (int j = 0; j < num_offsets; j++) res[j] = target_resid[j] > 0 ? target_resid[j] : target_resid[0];
-    long it = 0;
-    int conv = 1;
     const int sloppy = args.mixed_precision == 2 ? P_H16 : P_F32;
     if ((rc = refine_shifts(b, xs, offs.data(), res.data(), parity, mp.max_iters, sloppy, &it, fres.data(), &conv)))
       return rc;
-    total_iters += (int)it;
-  } else {
+  } else if (!mixed) {
     for (int j = 0; j < num_offsets; j++) fres[j] = std::sqrt(st.final_rsq);
   }
+  const int total_iters = st.iters + (int)it;
   for (int j = 0; j < num_offsets; j++)
     if ((rc = host_vec_out(external_precision, xs[j], pb, solutions[j]))) return rc;
   for (int j = 0; j < num_offsets; j++) {

@@ -1010,6 +1010,47 @@ static int true_residual(const VecField& src, const VecField& x, VecField& tmp_o
   return 0;
 }
 
+// rec[0] = the summed |resid|^2 of one k_dslash_resid
+__global__ void k_resid_sum(const double* __restrict__ partials_rr, int nblocks, double* rec) {
+  double t[1];
+  reduce_records<1>(partials_rr, nblocks, t);
+  if (threadIdx.x == 0) rec[0] = t[0];
+}
+
+// |b - (offset_j - D D) x_j| / |b| for every shift, read back together.
+int shift_residuals(const VecField& b, const std::vector<VecField>& x, const double* offsets, int parity, double* rel) {
+  Context& c = ctx();
+  const DevLinks& L = c.links[P_F64];
+  if (!L.valid) return -3;
+  const int n = (int)x.size(), pb = pbit(parity);
+  double norm = 0;
+  int rc = vec_norm2(b, P_F64, &norm);
+  if (rc) return rc;
+  VecField tmp, res, none{};
+  VecScope owned{&tmp, &res};
+  double* sums = nullptr;
+  OnExit scratch([&] {
+    (void)hipStreamSynchronize(c.stream);
+    dev_free(sums);
+  });
+  double* h = (double*)pinned_scratch(n * sizeof(double));
+  if (!h) return -5;
+  if ((rc = alloc_vec(tmp, P_F64, c.stride)) || (rc = alloc_vec(res, P_F64, c.stride)) ||
+      (rc = dev_alloc((void**)&sums, n * sizeof(double))))
+    return rc;
+  for (int j = 0; j < n; j++) {
+    launch_dslash<P_F64>(L, x[j], tmp, pb ^ 1, nullptr);
+    hipLaunchKernelGGL(k_dslash_resid<P_F64>, dim3(dslash_grid()), dim3(256), 0, c.stream, c.geom, L.fat, L.lng, tmp,
+                       x[j], b, res, none, 0, pb, offsets[j], partials_rr());
+    hipLaunchKernelGGL(k_resid_sum, dim3(1), dim3(1024), 0, c.stream, partials_rr(), dslash_grid(), sums + j);
+  }
+  MH_CHECK(hipGetLastError());
+  MH_CHECK(hipMemcpyAsync(h, sums, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+  MH_CHECK(hipStreamSynchronize(c.stream));
+  for (int j = 0; j < n; j++) rel[j] = norm > 0 ? std::sqrt(h[j] / norm) : 0.0;
+  return 0;
+}
+
 template <int PL, int PP, int PA>
 static void enqueue_cg_iteration(const DevLinks& L, VecField& p, VecField& tmp, VecField& r, VecField& ttt,
                                  VecField& x, int pb, double msq_x4, bool rel = false) {

@@ -219,9 +219,21 @@ struct MultiParams {
   double resid;        // base-system target |r|/|b|
   int prec;            // P_F64 or P_F32 bulk
   int batch;
+  // one-kernel solve only: |r_j|/|b| below which a shift is left as it is
+  // (nullptr: all shifts run to the end, as MILC's do)
+  const double* shift_resid = nullptr;
 };
 int multicg_solve(const VecField& src, std::vector<VecField>& x, const std::vector<double>& offsets,
                   const MultiParams& mp, SolveStats& st);
+// Whether the mixed multi-shifts of `sources` sources run as multishift_small.
+bool multishift_is_small(int sources = 1);
+// Multi-shift of a small lattice to each shift's own FP64 true residual
+// target resid[j] (what the FP32 stage and refine_shifts do on larger ones):
+// FP64 in one kernel, every true residual checked, a shift that misses its
+// target finished by its own CG.  iters, fres and converged as refine_shifts.
+int multishift_small(const VecField& b, std::vector<VecField>& x, const std::vector<double>& offsets,
+                     const double* resid, int parity, int max_iters, long* iters, double* fres, int* converged);
+int shift_residuals(const VecField& b, const std::vector<VecField>& x, const double* offsets, int parity, double* rel);
 
 // ---- force outer products ---------------------------------------------------
 int force_oprod(const std::vector<VecField>& xe, const std::vector<VecField>& xo,

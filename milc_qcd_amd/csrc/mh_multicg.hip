@@ -22,11 +22,9 @@
 
 #include "mh_dslash.h"
 #include "mh_internal.h"
+#include "mh_persist.h"
 
 namespace mh {
-
-#define MS_MAX 32
-#define MS_KW 8
 
 struct MSScalars {
   double zeta_i[MS_MAX], zeta_im1[MS_MAX], zeta_ip1[MS_MAX];
@@ -415,13 +413,131 @@ static int multicg_run(const VecField& src64, std::vector<VecField>& x64, const 
   return 0;
 }
 
+// The FP64 solve of a small lattice in one kernel.
+static int multicg_one_kernel(const VecField& src64, std::vector<VecField>& x64, const std::vector<double>& offsets,
+                              const MultiParams& mp, SolveStats& st) {
+  Context& c = ctx();
+  const int n = (int)offsets.size();
+  if (!c.links[P_F64].valid) return -3;
+  if (n <= 0 || n > MS_MAX) return -2;
+  double source_norm;
+  int rc = vec_norm2(src64, P_F64, &source_norm);
+  if (rc) return rc;
+  st = SolveStats();
+  if (source_norm == 0.0) {
+    for (int j = 0; j < n; j++)
+      if ((rc = vec_zero(x64[j], P_F64))) return rc;
+    st.converged = 1;
+    return 0;
+  }
+  constexpr int kTab = 2 * MS_MAX + MS_KW;
+  VecField tab[kTab]{}, work[4];
+  VecScope owned{&work[0], &work[1], &work[2], &work[3]};
+  for (int l = MS_MAX; l < kTab; l++) owned.add(&tab[l]);
+  char* dev = nullptr;
+  OnExit scalars([&] {
+    (void)hipStreamSynchronize(c.stream);
+    dev_free(dev);
+  });
+  auto take = [&](VecField& v) {
+    v.stride = c.stride;
+    return dev_alloc(&v.data, vec_bytes(P_F64, c.stride));
+  };
+  for (auto& v : work)
+    if ((rc = take(v))) return rc;
+  for (int j = 0; j < n; j++) {
+    tab[j] = x64[j];
+    if ((rc = take(tab[MS_MAX + j]))) return rc;
+  }
+  for (int l = 0; l < MS_KW; l++)
+    if ((rc = take(tab[2 * MS_MAX + l]))) return rc;
+  const size_t head = (sizeof(MSPersist) + 15) & ~(size_t)15, bytes = head + sizeof tab;
+  char* hp = (char*)pinned_scratch(bytes);
+  if (!hp) return -5;
+  if ((rc = dev_alloc((void**)&dev, bytes))) return rc;
+  MSPersist& h = *(MSPersist*)hp;
+  memset(&h, 0, sizeof h);
+  memcpy(hp + head, tab, sizeof tab);
+  h.n = n;
+  for (int j = 0; j < n; j++) {
+    h.shifts[j] = offsets[j];
+    if (offsets[j] < offsets[h.j_low]) h.j_low = j;
+    if (mp.shift_resid) h.stop[j] = mp.shift_resid[j] * mp.shift_resid[j] * source_norm;
+  }
+  h.source_norm = source_norm;
+  h.rsqstop = mp.resid * mp.resid * source_norm;
+  h.max_iter = (int)std::min<long>(mp.max_iters, 1L << 30);
+  MH_CHECK(hipMemcpyAsync(dev, hp, bytes, hipMemcpyHostToDevice, c.stream));
+  if ((rc = ms_persist(src64, (const VecField*)(dev + head), work, pbit(mp.parity), (MSPersist*)dev))) return rc;
+  MH_CHECK(hipMemcpyAsync(&h, dev, sizeof h, hipMemcpyDeviceToHost, c.stream));
+  MH_CHECK(hipStreamSynchronize(c.stream));
+  if (h.iters < 0) return -8;
+  st.iters = 1 + h.iters;
+  st.converged = h.converged;
+  st.final_rsq = st.size_r = h.rsq / source_norm;
+  return 0;
+}
+
 int multicg_solve(const VecField& src, std::vector<VecField>& x, const std::vector<double>& offsets,
                   const MultiParams& mp, SolveStats& st) {
   auto t0 = std::chrono::steady_clock::now();
-  int rc = mp.prec == P_F64 ? multicg_run<P_F64>(src, x, offsets, mp, st) : multicg_run<P_F32>(src, x, offsets, mp, st);
+  int rc = mp.prec == P_F64 && mp.max_iters > 1 && persist_shape(ctx().Vh).lps
+               ? multicg_one_kernel(src, x, offsets, mp, st)
+           : mp.prec == P_F64 ? multicg_run<P_F64>(src, x, offsets, mp, st) : multicg_run<P_F32>(src, x, offsets, mp, st);
   (void)hipStreamSynchronize(ctx().stream);
   st.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   return rc;
+}
+
+bool multishift_is_small(int sources) {
+  return ctx().Vh <= persist_mixed_shift_sites(sources) && persist_shape(ctx().Vh).lps && ctx().links[P_F64].valid;
+}
+
+int multishift_small(const VecField& b, std::vector<VecField>& x, const std::vector<double>& offsets,
+                     const double* resid, int parity, int max_iters, long* iters, double* fres, int* converged) {
+  const int n = (int)offsets.size();
+  if (n <= 0 || n > MS_MAX) return -2;
+  int low = 0;
+  for (int j = 1; j < n; j++)
+    if (offsets[j] < offsets[low]) low = j;
+  MultiParams mp;
+  mp.parity = parity;
+  mp.max_iters = max_iters;
+  // a little below the target, so that rounding does not leave the true
+  // residual just above it
+  mp.resid = 0.999 * resid[low];
+  mp.prec = P_F64;
+  mp.batch = 16;
+  std::vector<double> stop(n);
+  for (int j = 0; j < n; j++) stop[j] = 0.5 * resid[j];
+  mp.shift_resid = stop.data();
+  SolveStats st;
+  int rc = multicg_solve(b, x, offsets, mp, st);
+  if (rc) return rc;
+  *iters += st.iters;
+  *converged = 1;
+  std::vector<double> rel(n);
+  if ((rc = shift_residuals(b, x, offsets.data(), parity, rel.data()))) return rc;
+  for (int j = 0; j < n; j++) {
+    if (!(rel[j] < resid[j])) {
+      SolveParams sp;
+      sp.parity = parity;
+      sp.max_iters = max_iters;
+      sp.max_restarts = 1;
+      sp.resid = resid[j];
+      sp.relresid = 0;
+      sp.sloppy_prec = P_H16;
+      sp.delta = kReliableDelta;
+      sp.batch = 16;
+      SolveStats s2;
+      if ((rc = ensure_links(P_H16)) || (rc = cg_solve(b, x[j], 0.5 * std::sqrt(offsets[j]), sp, s2))) return rc;
+      *iters += s2.iters;
+      rel[j] = std::sqrt(s2.final_rsq);
+      *converged &= s2.converged;
+    }
+    if (fres) fres[j] = rel[j];
+  }
+  return 0;
 }
 
 }  // namespace mh

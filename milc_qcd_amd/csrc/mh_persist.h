@@ -26,4 +26,31 @@ constexpr int kPersistMixedSites = 49152;
 // waiting), the work fields are scratch.
 int cg_persist(VecField& x, VecField& r, VecField (&work)[4], int pb, double msq_x4, int max_it);
 
+// Multi-shift CG: most shifts of a solve, iterations of a window of deferred
+// updates.
+#define MS_MAX 32
+#define MS_KW 8
+// Sites per parity up to which the mixed multi-shift of `sources` sources runs
+// in FP64 in one kernel, one source after another (ms of one source, 12 shifts
+// to 1e-9, here / FP32 stage and refinement: Vh = 2048 1.3 / 7.6; 20736
+// 5.4 / 16.8; 65536 10.5 / 24; 131072 22.6 / 36; three shifts at 131072
+// 20.3 / 20.8).  Against the batched solve of up to four sources (all solves
+// of one HISQ trajectory step pair, two sources): 20736 28 / 50, 65536
+// 49 / 84, 131072 113 / 133, so that four sources break even near 16384.
+constexpr int persist_mixed_shift_sites(int sources) {
+  return sources <= 2 ? 131072 : (sources == 3 ? 65536 : (sources == 4 ? 16384 : (sources <= 6 ? 4096 : 0)));
+}
+
+// What one FP64 multi-shift solve in one kernel takes and gives back (device memory).
+struct MSPersist {
+  double shifts[MS_MAX];  // the offsets, as given
+  double stop[MS_MAX];    // |r_j|^2 below which shift j (not the smallest) is done; 0: never
+  double source_norm, rsqstop, rsq;
+  int n, j_low, max_iter, iters, converged;
+};
+// tab (device memory): psim_j in [0, n), pm_j in [MS_MAX, MS_MAX + n), the
+// residuals of a window in [2 MS_MAX, 2 MS_MAX + MS_KW); iters = -1 in io: a
+// workgroup gave up waiting.
+int ms_persist(const VecField& src, const VecField* tab, VecField (&work)[4], int pb, MSPersist* io);
+
 }  // namespace mh

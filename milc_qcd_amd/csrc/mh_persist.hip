@@ -211,8 +211,17 @@ struct SiteStencil {
     return h;
   }
   __device__ __forceinline__ static int at(const Geom& g, const Coord& c, int cb, const Hop& h) {
+    // scalar copies of the extents: an indexed g.X would move to memory
+    const int X0 = __builtin_amdgcn_readfirstlane(g.X[0]), X1 = __builtin_amdgcn_readfirstlane(g.X[1]);
+    const int X2 = __builtin_amdgcn_readfirstlane(g.X[2]), X3 = __builtin_amdgcn_readfirstlane(g.X[3]);
+    const int x = h.mu == 0 ? c.x : (h.mu == 1 ? c.y : (h.mu == 2 ? c.z : c.t));
+    const int L = h.mu == 0 ? X0 : (h.mu == 1 ? X1 : (h.mu == 2 ? X2 : X3));
+    const int stride = h.mu == 1 ? g.sy : (h.mu == 2 ? g.sz : g.st);
     const int dist = h.three ? 3 : 1;
-    return neighbour(g, c, cb, h.mu, h.back ? -dist : dist);
+    int y = x + (h.back ? -dist : dist);
+    y += y < 0 ? L : 0;
+    y -= y >= L ? L : 0;
+    return h.mu == 0 ? c.rowbase + (y >> 1) : cb + (y - x) * stride;
   }
   // the hop's matrix as it multiplies the neighbour: F, or -F^dag of the back link
   __device__ __forceinline__ static void link(const LinkField& fat, const LinkField& lng, int cb, int pb, const Hop& h,
@@ -419,6 +428,210 @@ k_cg_persist(Geom g, LinkField fat, LinkField lng, VecField x, VecField r, Excha
   }
 }
 
+// Multi-shift CG (ks_multicg_offset_field_cpu, ks_multicg_offset.c:291-460) in
+// one kernel: the recurrences and deferred updates of mh_multicg.hip, the
+// scalars of all shifts in LDS, computed alike by every workgroup (thread j has
+// shift j).  tab: psim_j (MS_MAX), pm_j (MS_MAX), then the MS_KW residuals of
+// the window, all touched by the lanes of their own site only; lane `sub` of a
+// site brings shifts sub, sub + LPS ... up to date.  pm_j and psim_j start as
+// the source and zero without being read.  A shift with a target of its own is
+// left as it is once its residual zeta_j |r| is below it (zeta_j set to zero,
+// as when it underflows).
+template <int LPS, int BS>
+__global__ void __launch_bounds__(BS, 1)
+k_ms_persist(Geom g, LinkField fat, LinkField lng, VecField src, const VecField* __restrict__ tab, Exchange ex, int pb,
+             MSPersist* io) {
+  constexpr int LDSM = Resident<LPS, BS>::lds;
+  __shared__ double sm[1][BS / 64];
+  __shared__ int lds_dead;
+  __shared__ nat_d2 lds[LDSM ? LDSM : 1][9][LDSM ? BS : 1];
+  __shared__ double zi[MS_MAX], zm1[MS_MAX], zp1[MS_MAX], bi[MS_MAX], shf[MS_MAX], wa[MS_MAX], wx[MS_MAX];
+  __shared__ double wc[MS_MAX][MS_KW], wb[MS_MAX][MS_KW];
+  __shared__ int done[MS_MAX];  // nothing left to bring up to date in this window
+  auto ldsp = (nat_d2(*)[9][BS])lds;
+  const int nb = gridDim.x, tid = threadIdx.x;
+  const int t = xcd_block(blockIdx.x, nb) * BS + tid;
+  const int cb = t / LPS, sub = t % LPS;
+  const bool on = cb < g.Vh;
+  const int n = io->n, jl = io->j_low, max_iter = io->max_iter;
+  const double rsqstop = io->rsqstop, shift0 = -io->shifts[jl];
+  if (tid < n) {
+    zi[tid] = zm1[tid] = 1.0;
+    shf[tid] = tid == jl ? io->shifts[tid] : io->shifts[tid] - io->shifts[jl];
+  }
+  const double stop_shift = tid < n && tid != jl ? io->stop[tid] : 0.0;
+  Vec3<double> rv, pv, tv;
+  SiteStencil<LPS, BS> st;
+  Waiter w{ex.gone, false};
+  zero(rv);
+  if (on) {
+    load_vec<P_F64>(src, cb, rv);
+    st.init(g, fat, lng, cb, pb ^ 1, sub, ldsp);
+    empty_vec<LPS>(ex.p[1], cb, sub);
+    empty_vec<LPS>(ex.tmp[1], cb, sub);
+  }
+  pv = rv;
+  double rsq = io->source_norm, alpha_low = 0.0, beta_low_1 = -1.0;
+  int it = 0, now = n, now_ws = n, m = 0, halt = 0, converged = 0;
+  bool first = true, ok = true;
+  __syncthreads();
+  while (!halt) {
+    const int e = it & 1;
+    if (m == 0) {
+      now_ws = now;
+      if (tid < n) {
+        wa[tid] = 1.0;
+        wx[tid] = 0.0;
+        for (int l = 0; l < MS_KW; l++) wc[tid][l] = wb[tid][l] = 0.0;
+        done[tid] = zi[tid] == 0.0;
+      }
+    }
+    double s[1] = {0.0};
+    if (on) {
+      put_vec<LPS>(ex.p[e], cb, sub, pv);
+      st.template apply<0>(g, fat, lng, ex.p[e], cb, pb ^ 1, sub, ldsp, w, tv);
+      put_vec<LPS>(ex.tmp[e], cb, sub, tv);
+      st.template apply<1>(g, fat, lng, ex.tmp[e], cb, pb, sub, ldsp, w, tv);
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        tv.c[k].re += shift0 * pv.c[k].re;
+        tv.c[k].im += shift0 * pv.c[k].im;
+        s[0] += pv.c[k].re * tv.c[k].re + pv.c[k].im * tv.c[k].im;
+      }
+      if (LPS > 1 && sub != 0) s[0] = 0.0;
+    }
+    // records: <p, ttt> in buffers 0 and 1, |r|^2 in 2 and 3
+    double* const rec_a = ex.rec + (size_t)e * 4 * nb;
+    double* const rec_b = ex.rec + (size_t)(2 + e) * 4 * nb;
+    publish_sums<1, BS>(s, rec_a, sm);
+    if (!(ok = collect_sums<1, BS>(s, rec_a, nb, sm, &lds_dead, w))) break;
+    if (on) {
+      empty_vec<LPS>(ex.p[e], cb, sub);
+      empty_vec<LPS>(ex.tmp[e], cb, sub);
+    }
+    if (it > 0 && tid == 0) st_empty(ex.rec + (size_t)(2 + (e ^ 1)) * 4 * nb + 4 * blockIdx.x);
+    // beta and zeta (ks_multicg_offset.c:322-356)
+    const double beta_low = -rsq / s[0];
+    it++;
+    m++;
+    const int last = now - 1;
+    const bool retire = last > jl && zi[last] == 0.0;
+    if (tid < now) {
+      if (tid == jl) {
+        bi[tid] = beta_low;
+        zp1[tid] = 1.0;
+      } else {
+        double z = zi[tid] * zm1[tid] * beta_low_1;
+        const double c1 = beta_low * alpha_low * (zm1[tid] - zi[tid]);
+        const double c2 = zm1[tid] * beta_low_1 * (1.0 + shf[tid] * beta_low);
+        z = c1 + c2 != 0.0 ? z / (c1 + c2) : 0.0;
+        if (zi[tid] != 0.0) {
+          bi[tid] = beta_low * z / zi[tid];
+        } else {
+          z = 0.0;
+          bi[tid] = 0.0;
+        }
+        zp1[tid] = z;
+      }
+    }
+    if (retire) now--;
+    if (tid < now) {
+      const double b = bi[tid];
+      wx[tid] += b * wa[tid];
+      for (int l = 0; l < m - 1; l++) wb[tid][l] += b * wc[tid][l];
+    }
+    s[0] = 0.0;
+    if (on) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        rv.c[k].re += beta_low * tv.c[k].re;
+        rv.c[k].im += beta_low * tv.c[k].im;
+        s[0] += rv.c[k].re * rv.c[k].re + rv.c[k].im * rv.c[k].im;
+      }
+      if (sub == 0) store_vec<P_F64>(tab[2 * MS_MAX + m - 1], cb, rv);
+      if (LPS > 1 && sub != 0) s[0] = 0.0;
+    }
+    publish_sums<1, BS>(s, rec_b, sm);
+    if (!(ok = collect_sums<1, BS>(s, rec_b, nb, sm, &lds_dead, w))) break;
+    if (tid == 0) st_empty(rec_a + 4 * blockIdx.x);
+    const double oldrsq = rsq;
+    rsq = s[0];
+    if (rsqstop > 0 && rsq <= rsqstop) {
+      halt = converged = 1;
+    } else {
+      // alpha, the coefficients of the window, scroll (:358-463)
+      alpha_low = rsq / oldrsq;
+      if (tid < now) {
+        double a = alpha_low;
+        if (tid != jl)
+          a = zi[tid] * beta_low != 0.0 ? alpha_low * zp1[tid] * bi[tid] / (zi[tid] * beta_low) : 0.0;
+        wa[tid] *= a;
+        for (int l = 0; l < m - 1; l++) wc[tid][l] *= a;
+        wc[tid][m - 1] = zp1[tid];
+        zm1[tid] = zi[tid];
+        zi[tid] = zp1[tid] * zp1[tid] * rsq < stop_shift ? 0.0 : zp1[tid];
+      }
+      beta_low_1 = beta_low;
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        pv.c[k].re = rv.c[k].re + alpha_low * pv.c[k].re;
+        pv.c[k].im = rv.c[k].im + alpha_low * pv.c[k].im;
+      }
+      if (1 + it >= max_iter) halt = 1;
+    }
+    if (m < MS_KW && !halt) continue;
+    // psim_j and pm_j from the window's residuals
+    __syncthreads();
+    if (on) {
+      Vec3<double> ring[MS_KW];
+#pragma unroll
+      for (int l = 0; l < MS_KW; l++) {
+        if (l < m) load_vec<P_F64>(tab[2 * MS_MAX + l], cb, ring[l]);
+        else zero(ring[l]);
+      }
+      for (int j = sub; j < now_ws; j += LPS) {
+        Vec3<double> d, x;
+        if (done[j]) continue;
+        if (first) {
+          load_vec<P_F64>(src, cb, d);
+          zero(x);
+        } else {
+          load_vec<P_F64>(tab[MS_MAX + j], cb, d);
+          load_vec<P_F64>(tab[j], cb, x);
+        }
+        const double cx = wx[j], ca = wa[j];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+          double xr = x.c[k].re + cx * d.c[k].re, xi = x.c[k].im + cx * d.c[k].im;
+          double qr = ca * d.c[k].re, qi = ca * d.c[k].im;
+#pragma unroll
+          for (int l = 0; l < MS_KW; l++) {
+            const double b = wb[j][l], cc = wc[j][l];
+            xr += b * ring[l].c[k].re;
+            xi += b * ring[l].c[k].im;
+            qr += cc * ring[l].c[k].re;
+            qi += cc * ring[l].c[k].im;
+          }
+          x.c[k].re = xr;
+          x.c[k].im = xi;
+          d.c[k].re = qr;
+          d.c[k].im = qi;
+        }
+        store_vec<P_F64>(tab[j], cb, x);
+        if (!halt) store_vec<P_F64>(tab[MS_MAX + j], cb, d);
+      }
+    }
+    first = false;
+    m = 0;
+    __syncthreads();
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    io->rsq = rsq;
+    io->iters = ok ? it : -1;
+    io->converged = converged;
+  }
+}
+
 int cu_count() {
   static int n[64] = {0};
   const int dev = ctx().device;
@@ -460,13 +673,9 @@ PersistShape persist_shape(int Vh) {
   return PersistShape{0, 0, 0};
 }
 
-int cg_persist(VecField& x, VecField& r, VecField (&work)[4], int pb, double msq_x4, int max_it) {
+// The exchange of a launch, all words empty.
+static int start_exchange(const VecField (&work)[4], int nb, int records, Exchange& ex) {
   Context& c = ctx();
-  const DevLinks& L = c.links[P_F64];
-  const PersistShape sh = persist_shape(c.Vh);
-  if (!L.valid || !sh.lps) return -3;
-  const int nb = sh.blocks;
-  Exchange ex;
   int rc;
   for (int k = 0; k < 4; k++) {
     (k < 2 ? ex.p[k] : ex.tmp[k - 2]) = work[k];
@@ -474,18 +683,49 @@ int cg_persist(VecField& x, VecField& r, VecField (&work)[4], int pb, double msq
   }
   ex.rec = c.ws.partials;
   ex.gone = c.ws.flags;
-  if ((rc = empty_words(ex.rec, (size_t)3 * 4 * nb * sizeof(double)))) return rc;
+  if ((rc = empty_words(ex.rec, (size_t)records * 4 * nb * sizeof(double)))) return rc;
   MH_CHECK(hipMemsetAsync(ex.gone, 0, kPersistFlagBytes, c.stream));
+  return 0;
+}
+
+// Kernel K<lanes, threads> of a shape.
+#define PERSIST_KERNEL(K, sh)                                                            \
+  ((sh).lps == 16  ? (const void*)K<16, 256>                                             \
+   : (sh).lps == 8 ? (const void*)K<8, 256>                                              \
+   : (sh).lps == 4 ? (const void*)K<4, 256>                                              \
+                   : ((sh).threads == 256 ? (const void*)K<1, 256> : (const void*)K<1, 512>))
+
+int cg_persist(VecField& x, VecField& r, VecField (&work)[4], int pb, double msq_x4, int max_it) {
+  Context& c = ctx();
+  const DevLinks& L = c.links[P_F64];
+  const PersistShape sh = persist_shape(c.Vh);
+  if (!L.valid || !sh.lps) return -3;
+  const int nb = sh.blocks;
+  Exchange ex;
+  int rc = start_exchange(work, nb, 3, ex);
+  if (rc) return rc;
   Geom g = c.geom;
   LinkField fat = L.fat, lng = L.lng;
   CGScalars* sc = c.ws.scal;
   void* args[] = {&g, &fat, &lng, &x, &r, &ex, &pb, &msq_x4, &max_it, &sc};
-  const void* k = nullptr;
-#define SHAPE(l, b) if (sh.lps == l && sh.threads == b) k = (const void*)k_cg_persist<l, b>
-  SHAPE(16, 256); SHAPE(8, 256); SHAPE(4, 256); SHAPE(1, 256); SHAPE(1, 512);
-#undef SHAPE
-  if (!k) return -3;
-  MH_CHECK(hipLaunchCooperativeKernel(k, dim3(nb), dim3(sh.threads), args, 0, c.stream));
+  MH_CHECK(hipLaunchCooperativeKernel(PERSIST_KERNEL(k_cg_persist, sh), dim3(nb), dim3(sh.threads), args, 0, c.stream));
+  return 0;
+}
+
+int ms_persist(const VecField& src, const VecField* tab, VecField (&work)[4], int pb, MSPersist* io) {
+  Context& c = ctx();
+  const DevLinks& L = c.links[P_F64];
+  const PersistShape sh = persist_shape(c.Vh);
+  if (!L.valid || !sh.lps) return -3;
+  Exchange ex;
+  int rc = start_exchange(work, sh.blocks, 4, ex);
+  if (rc) return rc;
+  Geom g = c.geom;
+  LinkField fat = L.fat, lng = L.lng;
+  VecField s = src;
+  void* args[] = {&g, &fat, &lng, &s, &tab, &ex, &pb, &io};
+  MH_CHECK(hipLaunchCooperativeKernel(PERSIST_KERNEL(k_ms_persist, sh), dim3(sh.blocks), dim3(sh.threads), args, 0,
+                                      c.stream));
   return 0;
 }
 

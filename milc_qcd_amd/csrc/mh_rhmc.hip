@@ -101,6 +101,13 @@ static int rational_solve(const VecField& phi, int n, const double* offsets, dou
   for (int t = 0; t < n; t++)
     if ((rc = alloc_vec(x[t], P_F64, c.stride))) return rc;
   std::vector<double> offs(offsets, offsets + n);
+  if (mixed && resid > 0 && multishift_is_small()) {
+    std::vector<double> res(n, resid);
+    long it = 0;
+    if ((rc = multishift_small(phi, x, offs, res.data(), parity, 20000, &it, nullptr, &st.converged))) return rc;
+    st.iters = (int)it;
+    return 0;
+  }
   MultiParams mp;
   mp.parity = parity;
   mp.max_iters = 20000;
@@ -135,6 +142,19 @@ static int rational_solve_all(const std::vector<const VecField*>& src, const std
   for (auto& o : offs) {
     if (o.empty() || (int)o.size() > BMS_MAX) return -2;
     n = std::max(n, (int)o.size());
+  }
+  if (multishift_is_small(ns) && *std::min_element(resid.begin(), resid.end()) > 0) {
+    // one source after another: no padding sources, no refinement
+    x.assign(ns, {});
+    long it = 0;
+    for (int r = 0; r < ns; r++) {
+      SolveStats st;
+      int rc = rational_solve(*src[r], (int)offs[r].size(), offs[r].data(), resid[r], 1, EVEN, x[r], st);
+      if (rc) return rc;
+      it += st.iters;
+    }
+    if (iters) *iters = it;
+    return 0;
   }
   // a source with fewer shifts repeats its last one; the padding sources are
   // zero and halt at once

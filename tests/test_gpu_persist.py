@@ -57,3 +57,51 @@ def test_mixed_cg_above_the_one_kernel_range():
             _, st = G.dev_invert(0, 2, 0.05, mq.EVEN, 1e-10, mixed)
             assert st["converged"] and st["resid"] < 1e-10
             assert G.dev_diff(2, 1) < 10 * 1e-10 / (4 * 0.05 ** 2)
+
+
+OFFSETS = [4 * 0.05 ** 2 + 1e-4 * 10 ** (4 * i / 11) for i in range(12)]
+
+
+@pytest.mark.parametrize("dims", SIZES)
+@pytest.mark.parametrize("mixed", [0, 1])
+def test_multishift_one_kernel(dims, mixed):
+    """Three and twelve shifts against single-mass solves to a hundredth of the
+    target; a repeat is bit-identical."""
+    resid = 1e-9
+    print(f"one-kernel multi-shift {dims} mixed {mixed}", flush=True)
+    with mq.Lattice(dims) as G:
+        G.dev_gauge_hisq(1404)
+        G.dev_source(1405, mq.EVEN, 0)
+        for offs in (OFFSETS[5:2:-1], OFFSETS):
+            n = len(offs)
+            _, _, conv = G.dev_multishift(0, offs, resid, mixed, out_slot0=1)
+            assert conv
+            G.dev_multishift(0, offs, resid, mixed, out_slot0=20)
+            for j in (0, 1, n - 1):
+                assert G.dev_diff(1 + j, 20 + j) == 0.0
+                G.dev_invert(0, 40, 0.5 * offs[j] ** 0.5, mq.EVEN, resid / 100, 0)
+                assert G.dev_diff(1 + j, 40) < 10 * resid / offs[j]
+
+
+@pytest.mark.parametrize("n", [1, 2, 31, 32])
+def test_multishift_one_kernel_shift_counts_and_retirement(n):
+    """Shift counts at the ends of the table, the smallest offset last or first,
+    heavy shifts whose zeta underflows (retired), and iteration caps inside and
+    at the edge of a window, against the oracle's multi-shift CG."""
+    dims = (6, 4, 8, 6)
+    L = ko.Lattice(dims)
+    U = L.rephase(L.gauge_random(1406))
+    fat, lng, _ = L.hisq_links(U)
+    src = L.gaussian_vector(1407, ko.EVEN)
+    offs = [0.04 * 1.9 ** (j if n % 2 else n - 1 - j) for j in range(n)]
+    s = L.parity_slice(ko.EVEN)
+    with mq.Lattice(dims) as G:
+        G.set_links(fat, lng)
+        for cap in (3000, 2, 9, 10):
+            ref, it_ref, _ = L.multicg_offset(fat, lng, src, offs, 1e-10, max_iters=cap, nrestart=1)
+            ksp = [mq.KsParam(offset=o) for o in offs]
+            qic = [mq.QuarkInvertControl(max=cap, nrestart=1, resid=1e-10) for _ in offs]
+            x = G.ks_multicg_offset_field(src, ksp, qic, mixed=0)
+            assert qic[0].final_iters == it_ref
+            for a, b in zip(x, ref):
+                assert np.linalg.norm(a[s] - b[s]) < 1e-9 * max(np.linalg.norm(b[s]), 1e-300)

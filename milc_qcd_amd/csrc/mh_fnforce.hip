@@ -1635,6 +1635,22 @@ __global__ void __launch_bounds__(256) k_link_axpy(LinkField y, LinkField x, dou
   store_link<P_F64, double>(y, pb, mu, cb, my, 1.0f);
 }
 
+template <typename R>
+__global__ void __launch_bounds__(256) k_add_increments(R* __restrict__ m, const double* __restrict__ inc, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    m[i] += (R)inc[i];
+}
+// m (precision 1 float, 2 double) += inc, n numbers
+int add_increments_dev(int prec, const double* inc, void* m, size_t n) {
+  const unsigned nb = (unsigned)std::min<size_t>((n + 255) / 256, 8192);
+  if (prec == 2)
+    hipLaunchKernelGGL(k_add_increments<double>, dim3(nb), dim3(256), 0, ctx().stream, (double*)m, inc, n);
+  else
+    hipLaunchKernelGGL(k_add_increments<float>, dim3(nb), dim3(256), 0, ctx().stream, (float*)m, inc, n);
+  MH_CHECK(hipGetLastError());
+  return 0;
+}
+
 int link_axpy_dev(LinkField& y, const LinkField& x, double a, double b, int signed_odd) {
   Context& c = ctx();
   hipLaunchKernelGGL(k_link_axpy, dim3((c.Vh + 255) / 256, 8), dim3(256), 0, c.stream, y, x, a, b, signed_odd,

@@ -248,6 +248,7 @@ constexpr double kForceFilter = 5.0e-5;  // HISQ_FORCE_FILTER of ks_imp_rhmc/Mak
 int hisq_force_from_oprod(const LinkField& U, const LinkField& V, const LinkField& W, const LinkField& o1,
                           const LinkField& o3, const double coeff2[6], const double coeff1[6], double scale,
                           double filter, double* mom_dev, const LinkField* one_link_extra = nullptr);
+int add_increments_dev(int prec, const double* inc, void* m, size_t n);
 // y = b y + a x on FP64 link fields (x negated on odd sites when signed_odd)
 int link_axpy_dev(LinkField& y, const LinkField& x, double a, double b, int signed_odd);
 // "1-link + Naik" table of a second Naik set (imp_actions/hisq/hisq_u3_action.h:86-101)

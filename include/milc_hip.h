@@ -312,11 +312,11 @@ int milc_hip_link_compression(int prec);
 
 /* Evaluation form of the thin-link force adjoints (FN and HISQ): 0 = gather
  * over the path table for every smearing; 1 (default) = reverse mode through
- * the generalised staples of the fattening wherever that is exact for any
- * links (no Lepage term, or the U(3)-projected HISQ links), path table
- * otherwise; 2 = staple form for every smearing (exact for unitary links: the
- * optimised Lepage term retraces U U^+).  Returns -2 for another value.  No
- * counterpart in the reference (MILC's CPU code walks sorted paths). */
+ * the staples of the fattening, for any links (the Lepage paths taken as they
+ * are unless the links are the U(3)-projected HISQ ones); 2 = the same with the
+ * Lepage term as a double staple for every smearing (exact for unitary links:
+ * it retraces U U^+).  Returns -2 for another value.  No counterpart in the
+ * reference (MILC's CPU code walks sorted paths). */
 int milc_hip_set_force_form(int form);
 
 /* ---- many right-hand sides ------------------------------------------------- */

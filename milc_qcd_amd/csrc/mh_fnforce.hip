@@ -107,11 +107,21 @@ static void build_entries(const std::vector<FnPath>& paths, const std::vector<in
   start[4] = (int)ent.size();
 }
 
+// Element e of a matrix lies e planes after the first: a base that is the same
+// for the whole block plus the site's 32-bit byte offset, so that a load takes a
+// scalar base and one offset register instead of a 64-bit address of its own
+// (with those kept, k_sf_adj5 took 306 registers).
+__device__ __forceinline__ unsigned site_off(int cb) { return (unsigned)cb * (unsigned)sizeof(double2); }
+__device__ __forceinline__ const char* plane_base(const void* data, size_t plane, int stride) {
+  return (const char*)data + plane * (size_t)stride * sizeof(double2);
+}
 __device__ __forceinline__ void mload(const LinkField& f, int pb, int mu, int cb, Mat3<double>& m) {
-  const double2* p = (const double2*)f.data + (size_t)((pb * 4 + mu) * 9) * f.stride + cb;
+  const char* p = plane_base(f.data, (size_t)((pb * 4 + mu) * 9), f.stride);
+  const size_t step = (size_t)f.stride * sizeof(double2);
+  const unsigned off = site_off(cb);
 #pragma unroll
   for (int e = 0; e < 9; e++) {
-    double2 a = p[(size_t)e * f.stride];
+    double2 a = *(const double2*)(p + e * step + off);
     m.e[e / 3][e % 3].re = a.x;
     m.e[e / 3][e % 3].im = a.y;
   }
@@ -429,11 +439,8 @@ __global__ void __launch_bounds__(128) k_u3_adjoint(Geom g, LinkField Vf, LinkFi
 // (c5 S2 + sum_sig c7 S_sig(S2))], S1 = S_nu(U_mu), S2 = S_rho(S1),
 //   S_nu(A)(x) = U_nu(x) A(x+nu) U_nu(x+mu)^dag + U_nu(x-nu)^dag A(x-nu) U_nu(x-nu+mu),
 // plus the Naik product.  Every step is a gather over one lattice of 3x3
-// matrices (no atomics), 38 launches per direction mu instead of the path
-// walk per (path, position).  For unitary links the result differs from the
-// path-table gather only by components the traceless anti-Hermitian part (or
-// the U(3) projection derivative) removes: the retracing Lepage terms are
-// constant on the group.
+// matrices (no atomics), 22 launches per direction mu instead of the path
+// walk per (path, position).
 // ---------------------------------------------------------------------------
 // a matrix per site and parity: element e of site (pb, cb) at
 // data[(pb * pstride + off + e) * stride + cb]  (pstride 36 / off 9 mu for one
@@ -446,61 +453,74 @@ __host__ inline MF mf_link(const LinkField& f, int mu) { return MF{(double2*)f.d
 __host__ inline MF mf_site(double2* d, int stride) { return MF{d, stride, 9, 0}; }
 
 __device__ __forceinline__ void mfl(const MF& f, int pb, int cb, Mat3<double>& m) {
-  const double2* p = f.data + (size_t)(pb * f.pstride + f.off) * f.stride + cb;
+  const char* p = plane_base(f.data, (size_t)(pb * f.pstride + f.off), f.stride);
+  const size_t step = (size_t)f.stride * sizeof(double2);
+  const unsigned off = site_off(cb);
 #pragma unroll
   for (int e = 0; e < 9; e++) {
-    double2 a = p[(size_t)e * f.stride];
+    double2 a = *(const double2*)(p + e * step + off);
     m.e[e / 3][e % 3].re = a.x;
     m.e[e / 3][e % 3].im = a.y;
   }
 }
 __device__ __forceinline__ void mfs(const MF& f, int pb, int cb, const Mat3<double>& m) {
-  double2* p = f.data + (size_t)(pb * f.pstride + f.off) * f.stride + cb;
+  char* p = (char*)plane_base(f.data, (size_t)(pb * f.pstride + f.off), f.stride);
+  const size_t step = (size_t)f.stride * sizeof(double2);
+  const unsigned off = site_off(cb);
 #pragma unroll
-  for (int e = 0; e < 9; e++) p[(size_t)e * f.stride] = make_double2(m.e[e / 3][e % 3].re, m.e[e / 3][e % 3].im);
+  for (int e = 0; e < 9; e++)
+    *(double2*)(p + e * step + off) = make_double2(m.e[e / 3][e % 3].re, m.e[e / 3][e % 3].im);
 }
 // f += c m
 __device__ __forceinline__ void mfa(const MF& f, int pb, int cb, double c, const Mat3<double>& m) {
-  double2* p = f.data + (size_t)(pb * f.pstride + f.off) * f.stride + cb;
+  char* p = (char*)plane_base(f.data, (size_t)(pb * f.pstride + f.off), f.stride);
+  const size_t step = (size_t)f.stride * sizeof(double2);
+  const unsigned off = site_off(cb);
 #pragma unroll
   for (int e = 0; e < 9; e++) {
-    double2 a = p[(size_t)e * f.stride];
+    double2 a = *(double2*)(p + e * step + off);
     a.x += c * m.e[e / 3][e % 3].re;
     a.y += c * m.e[e / 3][e % 3].im;
-    p[(size_t)e * f.stride] = a;
+    *(double2*)(p + e * step + off) = a;
   }
 }
 // Non-temporal forms for the own-site accumulators of the staple kernels,
 // which no other site reads in the same pass: their lines are not kept in L2,
 // leaving it to the neighbour-read links and forces.
 __device__ __forceinline__ void mfl_nt(const MF& f, int pb, int cb, Mat3<double>& m) {
-  const double2* p = f.data + (size_t)(pb * f.pstride + f.off) * f.stride + cb;
+  const char* p = plane_base(f.data, (size_t)(pb * f.pstride + f.off), f.stride);
+  const size_t step = (size_t)f.stride * sizeof(double2);
+  const unsigned off = site_off(cb);
 #pragma unroll
   for (int e = 0; e < 9; e++) {
-    const nat_d2 a = ldnt(p + (size_t)e * f.stride);
+    const nat_d2 a = ldnt((const double2*)(p + e * step + off));
     m.e[e / 3][e % 3].re = a.x;
     m.e[e / 3][e % 3].im = a.y;
   }
 }
 __device__ __forceinline__ void mfs_nt(const MF& f, int pb, int cb, const Mat3<double>& m) {
-  double2* p = f.data + (size_t)(pb * f.pstride + f.off) * f.stride + cb;
+  char* p = (char*)plane_base(f.data, (size_t)(pb * f.pstride + f.off), f.stride);
+  const size_t step = (size_t)f.stride * sizeof(double2);
+  const unsigned off = site_off(cb);
 #pragma unroll
   for (int e = 0; e < 9; e++) {
     nat_d2 a;
     a.x = m.e[e / 3][e % 3].re;
     a.y = m.e[e / 3][e % 3].im;
-    __builtin_nontemporal_store(a, (nat_d2*)(p + (size_t)e * f.stride));
+    __builtin_nontemporal_store(a, (nat_d2*)(p + e * step + off));
   }
 }
 // f += c m, non-temporal
 __device__ __forceinline__ void mfa_nt(const MF& f, int pb, int cb, double c, const Mat3<double>& m) {
-  double2* p = f.data + (size_t)(pb * f.pstride + f.off) * f.stride + cb;
+  char* p = (char*)plane_base(f.data, (size_t)(pb * f.pstride + f.off), f.stride);
+  const size_t step = (size_t)f.stride * sizeof(double2);
+  const unsigned off = site_off(cb);
 #pragma unroll
   for (int e = 0; e < 9; e++) {
-    nat_d2 a = ldnt(p + (size_t)e * f.stride);
+    nat_d2 a = ldnt((const double2*)(p + e * step + off));
     a.x += c * m.e[e / 3][e % 3].re;
     a.y += c * m.e[e / 3][e % 3].im;
-    __builtin_nontemporal_store(a, (nat_d2*)(p + (size_t)e * f.stride));
+    __builtin_nontemporal_store(a, (nat_d2*)(p + e * step + off));
   }
 }
 __device__ __forceinline__ void mmul_na(const Mat3<double>& a, const Mat3<double>& b, Mat3<double>& c) {
@@ -522,13 +542,30 @@ __device__ __forceinline__ void madd(Mat3<double>& a, const Mat3<double>& b) {
       a.e[i][j].im += b.e[i][j].im;
     }
 }
-__device__ __forceinline__ void madd_adj(Mat3<double>& a, const Mat3<double>& b) {
+__device__ __forceinline__ void mzero(Mat3<double>& a) {
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++) a.e[i][j].re = a.e[i][j].im = 0.0;
+}
+// a += c b
+__device__ __forceinline__ void maxpy(Mat3<double>& a, double c, const Mat3<double>& b) {
 #pragma unroll
   for (int i = 0; i < 3; i++)
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-      a.e[i][j].re += b.e[j][i].re;
-      a.e[i][j].im -= b.e[j][i].im;
+      a.e[i][j].re += c * b.e[i][j].re;
+      a.e[i][j].im += c * b.e[i][j].im;
+    }
+}
+// a += c b^dag
+__device__ __forceinline__ void maxpy_adj(Mat3<double>& a, double c, const Mat3<double>& b) {
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      a.e[i][j].re += c * b.e[j][i].re;
+      a.e[i][j].im -= c * b.e[j][i].im;
     }
 }
 
@@ -601,32 +638,42 @@ __host__ inline bool sf_tiled(const Geom& g, int mu, int nu) {
   return (mu == 3 || nu == 3) && g.st % 16 == 0 && g.X[3] % 4 == 0;
 }
 
-// out = S_nu(A) for the mu link
+// The staple in direction nu is the sum of an upper half, through y+nu, and a
+// lower one, through y-nu; `which` picks them (bit 0 upper, bit 1 lower).
+enum { SF_UPPER = 1, SF_LOWER = 2, SF_BOTH = 3 };
+
+// out = S_nu(A) for the mu link (or one half of it)
 template <int MU, int NU, int TT>
-__global__ void __launch_bounds__(128) k_sf_fwd(Geom g, LinkField U, MF A, MF out) {
+__global__ void __launch_bounds__(128) k_sf_fwd(Geom g, LinkField U, MF A, MF out, int which) {
   int cb, pb;
   if (!sf_site<TT>(g, cb, pb)) return;
   const int po = pb ^ 1;
   const SfSites n = sf_sites<MU, NU>(g, cb, pb);
   Mat3<double> a, b, t, up, lo;
-  mfl(A, po, n.ypn, a);
-  mload(U, po, NU, n.ypm, b);
-  mmul_na(a, b, t);
-  mload(U, pb, NU, cb, b);
-  mmul(b, t, up);
-  mload(U, po, NU, n.ymn, a);
-  mfl(A, po, n.ymn, b);
-  mmul_an(a, b, t);
-  mload(U, pb, NU, n.ymnpm, b);
-  mmul(t, b, lo);
-  madd(up, lo);
+  mzero(up);
+  if (which & SF_UPPER) {
+    mfl(A, po, n.ypn, a);
+    mload(U, po, NU, n.ypm, b);
+    mmul_na(a, b, t);
+    mload(U, pb, NU, cb, b);
+    mmul(b, t, up);
+  }
+  if (which & SF_LOWER) {
+    mload(U, po, NU, n.ymn, a);
+    mfl(A, po, n.ymn, b);
+    mmul_an(a, b, t);
+    mload(U, pb, NU, n.ymnpm, b);
+    mmul(t, b, lo);
+    madd(up, lo);
+  }
   mfs(out, pb, cb, up);
 }
 
-// out = S_P(AP) + S_Q(AQ) for the mu link: the two 5-staples of one 7-staple
-// direction in one pass
+// out = S_P(AP) + S_Q(AQ) + ce E for the mu link: the two 5-staples of one
+// 7-staple direction in one pass (E: the 3-staple whose Lepage term takes the
+// same FU pass; ce = 0: none)
 template <int MU, int P, int Q, int TT>
-__global__ void __launch_bounds__(128) k_sf_fwd2(Geom g, LinkField U, MF AP, MF AQ, MF out) {
+__global__ void __launch_bounds__(128) k_sf_fwd2(Geom g, LinkField U, MF AP, MF AQ, MF E, double ce, MF out) {
   int cb, pb;
   if (!sf_site<TT>(g, cb, pb)) return;
   const int po = pb ^ 1;
@@ -660,9 +707,13 @@ __global__ void __launch_bounds__(128) k_sf_fwd2(Geom g, LinkField U, MF AP, MF 
     mmul(t, b, lo);
     madd(up, lo);
   }
+  if (ce != 0.0) {
+    mfl_nt(E, pb, cb, a);
+    maxpy(up, ce, a);
+  }
   mfs(out, pb, cb, up);
 }
-typedef void (*SfFwd2Fn)(Geom, LinkField, MF, MF, MF);
+typedef void (*SfFwd2Fn)(Geom, LinkField, MF, MF, MF, double, MF);
 template <int MU, int P, int Q>
 static SfFwd2Fn sf_fwd2_pick(bool tt) {
   return tt ? k_sf_fwd2<MU, P, Q, 1> : k_sf_fwd2<MU, P, Q, 0>;
@@ -686,91 +737,194 @@ static SfFwd2Fn sf_fwd2_kernel(const Geom& g, int mu, int p, int q) {
   }
 }
 
-// reverse of O = S_nu(A) for the force Gs on O scaled by cg:
-//   FA(y)    += cg [U_nu(y-nu+mu)^dag G(y-nu) U_nu(y-nu) + U_nu(y+mu) G(y+nu) U_nu(y)^dag]
-//   FU_nu(y) += cg [A(y+nu) U_nu(y+mu)^dag G(y) + (G(y-mu) U_nu(y-mu) A(y-mu+nu))^dag
-//                   + (A(y) U_nu(y+mu) G(y+nu))^dag + G(y-mu+nu) U_nu(y-mu)^dag A(y-mu)]
-// With fa_init the FA term is not accumulated but initialised:
-//   FA(y) = ci FI(y) + cg [...]
-// which stands for a preceding FA = ci FI pass (the scaled staple force).
-// MODE 0 computes both terms; MODE 1 only the FA term, MODE 2 only the FU term
-// (FA depends on Gs alone, FU is linear in A: the 7-staple driver forms each
-// FA once per direction pair and the FU of two 5-staples from their sum).
-template <int MU, int NU, int TT, int MODE>
-__global__ void __launch_bounds__(128) k_sf_adj(Geom g, LinkField U, MF A, MF Gs, double cg, MF FA, MF FU,
-                                                int fa_init, MF FI, double ci) {
-  int cb, pb;
-  if (!sf_site<TT>(g, cb, pb)) return;
+// Reverse of O = S_nu(A) for the force G on O:
+//   FA(y)    = U_nu(y-nu+mu)^dag G(y-nu) U_nu(y-nu) + U_nu(y+mu) G(y+nu) U_nu(y)^dag
+//   FU_nu(y) = A(y+nu) U_nu(y+mu)^dag G(y) + (G(y-mu) U_nu(y-mu) A(y-mu+nu))^dag
+//              + (A(y) U_nu(y+mu) G(y+nu))^dag + G(y-mu+nu) U_nu(y-mu)^dag A(y-mu)
+// The first FA term and the first two FU terms belong to the upper half of the
+// staple, the others to the lower half; the halves may have arguments (Ap, Am)
+// and forces (Gp, Gm) of their own.
+template <int NU>
+__device__ __forceinline__ void sf_fa(const LinkField& U, const SfSites& n, int cb, int pb, const MF& Gp, const MF& Gm,
+                                      int which, Mat3<double>& acc) {
   const int po = pb ^ 1;
-  const SfSites n = sf_sites<MU, NU>(g, cb, pb);
-  Mat3<double> a, b, t, u, acc;
-  if (MODE != 2) {
+  Mat3<double> b, t, u;
+  mzero(acc);
+  if (which & SF_UPPER) {
     mload(U, pb, NU, n.ymnpm, u);
-    mfl(Gs, po, n.ymn, b);
+    mfl(Gp, po, n.ymn, b);
     mmul_an(u, b, t);
     mload(U, po, NU, n.ymn, u);
     mmul(t, u, acc);
+  }
+  if (which & SF_LOWER) {
     mload(U, po, NU, n.ypm, u);
-    mfl(Gs, po, n.ypn, b);
+    mfl(Gm, po, n.ypn, b);
     mmul(u, b, t);
     mload(U, pb, NU, cb, u);
-    mmul_na(t, u, a);
-    madd(acc, a);
-    if (fa_init) {
-      mfl_nt(FI, pb, cb, a);
-#pragma unroll
-      for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-          double re = ci * a.e[i][j].re, im = ci * a.e[i][j].im;
-          a.e[i][j].re = re + cg * acc.e[i][j].re;
-          a.e[i][j].im = im + cg * acc.e[i][j].im;
-        }
-      mfs_nt(FA, pb, cb, a);
-    } else {
-      mfa_nt(FA, pb, cb, cg, acc);
-    }
+    mmul_na(t, u, b);
+    madd(acc, b);
   }
-  if (MODE == 1) return;
+}
+// fu += c FU
+template <int NU>
+__device__ __forceinline__ void sf_fu(const LinkField& U, const SfSites& n, int cb, int pb, const MF& Ap, const MF& Am,
+                                      const MF& Gp, const MF& Gm, double c, Mat3<double>& fu) {
+  const int po = pb ^ 1;
+  Mat3<double> a, b, t, u;
   // A(y+nu) U_nu(y+mu)^dag G(y)
-  mfl(A, po, n.ypn, a);
+  mfl(Ap, po, n.ypn, a);
   mload(U, po, NU, n.ypm, u);
   mmul_na(a, u, t);
-  mfl(Gs, pb, cb, b);
-  mmul(t, b, acc);
+  mfl(Gp, pb, cb, b);
+  mmul(t, b, a);
+  maxpy(fu, c, a);
+  // (A(y) U_nu(y+mu) G(y+nu))^dag
+  mfl(Am, pb, cb, a);
+  mmul(a, u, t);
+  mfl(Gm, po, n.ypn, b);
+  mmul(t, b, a);
+  maxpy_adj(fu, c, a);
   // (G(y-mu) U_nu(y-mu) A(y-mu+nu))^dag
-  mfl(Gs, po, n.ymm, b);
+  mfl(Gp, po, n.ymm, b);
   mload(U, po, NU, n.ymm, u);
   mmul(b, u, t);
-  mfl(A, pb, n.ymmpn, a);
+  mfl(Ap, pb, n.ymmpn, a);
   mmul(t, a, b);
-  madd_adj(acc, b);
-  // (A(y) U_nu(y+mu) G(y+nu))^dag
-  mfl(A, pb, cb, a);
-  mload(U, po, NU, n.ypm, u);
-  mmul(a, u, t);
-  mfl(Gs, po, n.ypn, b);
-  mmul(t, b, a);
-  madd_adj(acc, a);
+  maxpy_adj(fu, c, b);
   // G(y-mu+nu) U_nu(y-mu)^dag A(y-mu)
-  mfl(Gs, pb, n.ymmpn, b);
-  mload(U, po, NU, n.ymm, u);
+  mfl(Gm, pb, n.ymmpn, b);
   mmul_na(b, u, t);
-  mfl(A, po, n.ymm, a);
+  mfl(Am, po, n.ymm, a);
   mmul(t, a, b);
-  madd(acc, b);
-  mfa_nt(FU, pb, cb, cg, acc);
+  maxpy(fu, c, b);
+}
+// Keeps the loads of one part from being carried over into the next: the
+// staple kernels run two wavefronts per SIMD only while a part's matrices fit
+// the registers, and the links it shares with the next part are still in L2.
+__device__ __forceinline__ void sf_part() { asm volatile("" ::: "memory"); }
+
+// FA = ci FI + cg FA_nu(Gs) (the halves `which` of it)
+template <int MU, int NU, int TT>
+__global__ void __launch_bounds__(128) k_sf_fa(Geom g, LinkField U, MF Gs, double cg, MF FI, double ci, MF FA,
+                                               int which) {
+  int cb, pb;
+  if (!sf_site<TT>(g, cb, pb)) return;
+  const SfSites n = sf_sites<MU, NU>(g, cb, pb);
+  Mat3<double> acc, o, f;
+  sf_fa<NU>(U, n, cb, pb, Gs, Gs, which, acc);
+  mfl_nt(FI, pb, cb, f);
+  mzero(o);
+  maxpy(o, ci, f);
+  maxpy(o, cg, acc);
+  mfs_nt(FA, pb, cb, o);
 }
 
-typedef void (*SfFwdFn)(Geom, LinkField, MF, MF);
-typedef void (*SfAdjFn)(Geom, LinkField, MF, MF, double, MF, MF, int, MF, double);
+// FU += cg FU_nu(Ap / Am, Gs)
+template <int MU, int NU, int TT>
+__global__ void __launch_bounds__(128) k_sf_fu(Geom g, LinkField U, MF Ap, MF Am, MF Gs, double cg, MF FU) {
+  int cb, pb;
+  if (!sf_site<TT>(g, cb, pb)) return;
+  const SfSites n = sf_sites<MU, NU>(g, cb, pb);
+  Mat3<double> fu;
+  mzero(fu);
+  sf_fu<NU>(U, n, cb, pb, Ap, Am, Gs, Gs, cg, fu);
+  mfa_nt(FU, pb, cb, 1.0, fu);
+}
+
+// The 3-staple: both halves of the reverse, FA += cg FA_nu, FU += cg FU_nu
+template <int MU, int NU, int TT>
+__global__ void __launch_bounds__(128) k_sf_adj(Geom g, LinkField U, MF A, MF Gp, MF Gm, double cg, MF FA, MF FU) {
+  int cb, pb;
+  if (!sf_site<TT>(g, cb, pb)) return;
+  const SfSites n = sf_sites<MU, NU>(g, cb, pb);
+  Mat3<double> acc;
+  sf_fa<NU>(U, n, cb, pb, Gp, Gm, SF_BOTH, acc);
+  mfa_nt(FA, pb, cb, cg, acc);
+  sf_part();
+  mzero(acc);
+  sf_fu<NU>(U, n, cb, pb, A, A, Gp, Gm, cg, acc);
+  mfa_nt(FU, pb, cb, 1.0, acc);
+}
+
+// One 5-staple of direction nu and what is pulled back through it: argument A,
+// force Gs, and where the force on A goes, FA (+)= ... cg FA_nu(Gs); with
+// init FA starts as ci F + cj FJ (cj = 0: ci F).
+struct SfTerm {
+  MF A, Gs, FA, FJ;  // site fields of one stride
+  double cj;
+  int init;
+};
+template <int NU>
+__device__ __forceinline__ void sf_term(const LinkField& U, const SfSites& n, int cb, int pb, const SfTerm& s, double cg,
+                                        const MF& F, double ci, Mat3<double>& fu) {
+  {
+    Mat3<double> acc, f;
+    sf_fa<NU>(U, n, cb, pb, s.Gs, s.Gs, SF_BOTH, acc);
+    if (s.init) {
+      Mat3<double> o;
+      mzero(o);
+      maxpy(o, cg, acc);
+      mfl(F, pb, cb, f);
+      maxpy(o, ci, f);
+      if (s.cj != 0.0) {
+        mfl(s.FJ, pb, cb, f);
+        maxpy(o, s.cj, f);
+      }
+      mfs_nt(s.FA, pb, cb, o);
+    } else {
+      mfa_nt(s.FA, pb, cb, cg, acc);
+    }
+  }
+  sf_part();
+  sf_fu<NU>(U, n, cb, pb, s.A, s.A, s.Gs, s.Gs, cg, fu);
+  sf_part();
+}
+// The two 5-staples whose outer direction is nu and the 7-staples' FU part of
+// the same direction (argument SS, force F), one update of FU (48^3x96, pairs
+// without / with t: 6.7 / 8.1 ms against 6.9 / 8.4 in three passes, though it
+// moves a quarter less: the L2 misses of the neighbour reads bound it, and two
+// or one workgroup fewer per CU did not help):
+//   FA_k (+)= cg FA_nu(Gs_k),  FU += cg sum_k FU_nu(A_k, Gs_k) + c7 FU_nu(SS, F)
+template <int MU, int NU, int TT>
+__global__ void __launch_bounds__(128) k_sf_adj5(Geom g, LinkField U, SfTerm s0, SfTerm s1, double cg, MF F,
+                                                 double ci, MF SS, double c7, MF FU) {
+  int cb, pb;
+  if (!sf_site<TT>(g, cb, pb)) return;
+  const SfSites n = sf_sites<MU, NU>(g, cb, pb);
+  Mat3<double> fu;
+  mzero(fu);
+  // one copy of the code for both: side by side the two parts' matrices run out
+  // of registers (512 and 300 B of scratch against 176)
+#pragma unroll 1
+  for (int k = 0; k < 2; k++) {
+    SfTerm s = s0;
+    s.A.data = k ? s1.A.data : s0.A.data;
+    s.Gs.data = k ? s1.Gs.data : s0.Gs.data;
+    s.FA.data = k ? s1.FA.data : s0.FA.data;
+    s.FJ.data = k ? s1.FJ.data : s0.FJ.data;
+    s.init = k ? s1.init : s0.init;
+    // addresses formed in the pass, not kept over both (90 registers)
+    SfSites m = n;
+    int y = cb;
+    asm volatile("" : "+v"(m.ypn), "+v"(m.ymn), "+v"(m.ypm), "+v"(m.ymm), "+v"(m.ymnpm), "+v"(m.ymmpn), "+v"(y));
+    sf_term<NU>(U, m, y, pb, s, cg, F, ci, fu);
+  }
+  if (c7 != 0.0) sf_fu<NU>(U, n, cb, pb, SS, SS, F, F, c7, fu);
+  mfa_nt(FU, pb, cb, 1.0, fu);
+}
+
 struct SfKernels {
-  SfFwdFn fwd;
-  SfAdjFn adj[3];  // by MODE
+  void (*fwd)(Geom, LinkField, MF, MF, int);
+  void (*fa)(Geom, LinkField, MF, double, MF, double, MF, int);
+  void (*fu)(Geom, LinkField, MF, MF, MF, double, MF);
+  void (*adj)(Geom, LinkField, MF, MF, MF, double, MF, MF);
+  void (*adj5)(Geom, LinkField, SfTerm, SfTerm, double, MF, double, MF, double, MF);
 };
 template <int MU, int NU, int TT>
 static SfKernels sf_pick() {
-  return SfKernels{k_sf_fwd<MU, NU, TT>, {k_sf_adj<MU, NU, TT, 0>, k_sf_adj<MU, NU, TT, 1>, k_sf_adj<MU, NU, TT, 2>}};
+  return SfKernels{k_sf_fwd<MU, NU, TT>, k_sf_fa<MU, NU, TT>, k_sf_fu<MU, NU, TT>, k_sf_adj<MU, NU, TT>,
+                   k_sf_adj5<MU, NU, TT>};
 }
 // kernels of the direction pair (mu, nu), mu != nu
 static SfKernels sf_kernels(const Geom& g, int mu, int nu) {
@@ -957,29 +1111,23 @@ static int path_adjoint_launch(int mode, const LinkField& Lk, const LinkField& F
 // coefficients; scale multiplies U G (2 eps in fermion_force_fn_multi, 1 when
 // the outer products already carry 2 eps, fermion_force_asqtad_gpu.c:53-56).
 static int smear_adjoint_dev(const LinkField& L, const LinkField& F1, const LinkField& F3, int with_eps,
-                             const double coeff[6], LinkField& G);
-// Which device form the thin-link force adjoints use.  The staple form walks
-// the optimised fattening, whose Lepage term includes retracing paths
-// U_nu U_nu^+ that equal 1 only for unitary links; the path table holds the
-// fattening's paths themselves.  0: path table everywhere; 1 (default): the
-// staple form where it is exact for any links (a smearing without a Lepage
-// term, or the U(3)-projected links W, unitary by construction), the path
-// table otherwise; 2: the staple form everywhere (exact for unitary links).
+                             const double coeff[6], bool unitary, LinkField& G);
+// Which device form the thin-link force adjoints use.  0: the path table
+// everywhere; 1 (default): the staple form, with the Lepage paths taken as they
+// are where the links need not be unitary; 2: the staple form with the Lepage
+// term as a double staple everywhere (exact for unitary links).
 static int g_force_form = 1;
 void set_force_form(int form) { g_force_form = form; }
-static bool use_staple_form(const double coeff[6], bool links_unitary) {
-  return g_force_form == 2 || (g_force_form == 1 && (links_unitary || coeff[5] == 0.0));
-}
 
 int fn_force_from_oprod(const LinkField& U, const LinkField& o1, const LinkField& o3, const double coeff[6],
                         double scale, double* mom_dev) {
   LinkField none{nullptr, 1.0f, 0};
-  if (!use_staple_form(coeff, false)) return path_adjoint_launch(1, U, o1, o3, 1, coeff, none, U, scale, mom_dev);
+  if (g_force_form == 0) return path_adjoint_launch(1, U, o1, o3, 1, coeff, none, U, scale, mom_dev);
   Context& c = ctx();
   LinkField G{};
   int rc;
   if ((rc = alloc_links(G, P_F64, c.stride))) return rc;
-  rc = smear_adjoint_dev(U, o1, o3, 1, coeff, G);
+  rc = smear_adjoint_dev(U, o1, o3, 1, coeff, g_force_form == 2, G);
   if (!rc) {
     hipLaunchKernelGGL(k_mom_ta, dim3((c.Vh + 127) / 128, 8), dim3(128), 0, c.stream, c.geom, U, G, scale, mom_dev, 0);
     rc = hipGetLastError() == hipSuccess ? 0 : -1;
@@ -1509,98 +1657,127 @@ int mom_action_dev(const double* mom_dev, double* action) {
 // Per direction mu, with F = eps F1_mu:
 //   S1[nu] = S_nu(L_mu)                      (3-staples)
 //   G2[sig] = c5 F + c7 FA_sig(F)            (the 7-staple force seen by a 5-staple)
-//   G[sig] += c7 FU_sig(S_rho(S1[nu]) + S_nu(S1[rho]), F)   ({nu, rho, sig} the other three)
-//   per nu: G1 = c3 F + cl FA_nu(F)  [Lepage] + sum_rho FA_rho(G2[sig]) (or c5 FA_rho(F)),
-//           G[nu] += cl FU_nu(S1[nu], F), G[rho] += FU_rho(S1[nu], G2[sig]),
-//           G_mu += FA_nu(G1), G[nu] += FU_nu(L_mu, G1)
-// FA_nu(X) and FU_nu(A, X) are the two halves of the reverse of S_nu (k_sf_adj).
-// A 7-staple force term depends on the 5-staple only through FU, linearly,
-// and its FA part only on F and sig, so the two orders (nu, rho) and
-// (rho, nu) of one sig share one FA pass and one FU pass.
+//   per outer direction rho of the 5-staples ({nu, sig, rho} the other three):
+//     G1[nu]  += FA_rho(G2[sig]), G1[sig] += FA_rho(G2[nu]),
+//     G[rho]  += FU_rho(S1[nu], G2[sig]) + FU_rho(S1[sig], G2[nu])
+//                + c7 FU_rho(S_nu(S1[sig]) + S_sig(S1[nu]), F)
+//   per nu (G1[nu] started as c3 F):
+//     G_mu += FA_nu(G1[nu]), G[nu] += FU_nu(L_mu, G1[nu])
+// FA_nu(X) and FU_nu(A, X) are the two halves of the reverse of S_nu.  A
+// 7-staple force term depends on the 5-staple only through FU, linearly, and
+// its FA part only on F and its direction, so the two orders share one FA pass
+// and one FU pass.
+//
+// The Lepage term.  For unitary links it is cl S_nu(S_nu(L_mu)) with -6 cl on
+// the one-link term (the retracing paths of the double staple equal L_mu), and
+// takes no pass of its own beside 7-staples: its FA part is c7's, already in
+// G2[nu], so G1[nu] starts as (c3 - cl c5 / c7) F + (cl / c7) G2[nu], and its
+// FU part rides on the 7-staples' (argument + (cl / c7) S1[rho]).  For links
+// that need not be unitary it is the path itself, the upper half of S_nu of the
+// upper half plus the lower half of the lower half, with forces of their own
+// for the two halves of the 3-staple.
 static int smear_adjoint_dev(const LinkField& L, const LinkField& F1, const LinkField& F3, int with_eps,
-                             const double coeff[6], LinkField& G) {
+                             const double coeff[6], bool unitary, LinkField& G) {
   Context& c = ctx();
   const int st = c.stride;
-  const double c1 = coeff[0] - 6.0 * coeff[5], cN = coeff[1], c3 = coeff[2], c5 = coeff[3], c7 = coeff[4],
-               cl = coeff[5];
+  const double cN = coeff[1], c3 = coeff[2], c5 = coeff[3], c7 = coeff[4], cl = coeff[5];
+  const bool split = cl != 0.0 && !unitary;  // Lepage paths half by half
+  const double c1 = coeff[0] - (split ? 0.0 : 6.0 * cl);
   const bool staples = c3 != 0.0 || cl != 0.0 || c5 != 0.0 || c7 != 0.0;
   const bool five = c5 != 0.0 || c7 != 0.0, seven = c7 != 0.0;
-  // F, G1, S1[4], G2[4], SS: the mu-th entries of S1 and G2 are not used
-  double2 *F = nullptr, *G1 = nullptr, *SS = nullptr, *S1[4] = {}, *G2[4] = {};
+  const bool ride = cl != 0.0 && !split && seven;  // Lepage term on the 7-staples' passes
+  const bool double_staple = cl != 0.0 && !split && !seven;
+  // buffers by slot of the three other directions
+  double2 *F = nullptr, *SS = nullptr, *S1[3] = {}, *G1[3] = {}, *G2[3] = {}, *H[4] = {};
   OnExit bufs([&] {
     dev_free(F);
-    dev_free(G1);
     dev_free(SS);
-    for (int d = 0; d < 4; d++) {
+    for (int d = 0; d < 3; d++) {
       dev_free(S1[d]);
+      dev_free(G1[d]);
       dev_free(G2[d]);
     }
+    for (auto* h : H) dev_free(h);
   });
   const size_t bytes = (size_t)2 * 9 * st * sizeof(double2);
   int rc;
   if ((rc = dev_alloc((void**)&F, bytes))) return rc;
   if (staples) {
-    if ((rc = dev_alloc((void**)&G1, bytes))) return rc;
     for (int d = 0; d < 3; d++)
-      if ((rc = dev_alloc((void**)&S1[d], bytes))) return rc;
+      if ((rc = dev_alloc((void**)&S1[d], bytes)) || (rc = dev_alloc((void**)&G1[d], bytes))) return rc;
     if (seven) {
       if ((rc = dev_alloc((void**)&SS, bytes))) return rc;
       for (int d = 0; d < 3; d++)
         if ((rc = dev_alloc((void**)&G2[d], bytes))) return rc;
     }
+    if (split)
+      for (auto& h : H)
+        if ((rc = dev_alloc((void**)&h, bytes))) return rc;
   }
   MH_CHECK(hipMemsetAsync(G.data, 0, link_bytes(P_F64, st), c.stream));
-  const MF mF = mf_site(F, st), mG1 = mf_site(G1, st), mSS = mf_site(SS, st);
+  const MF mF = mf_site(F, st), mSS = mf_site(SS, st);
   // init: plain grid; the neighbour-reading kernels: XCD block order
   dim3 grid((c.Vh + 127) / 128, 2), xgrid = xcd_grid((c.Vh + 127) / 128, 2), blk(128);
-  const MF none{};
-  auto adj = [&](int mode, int mu, int nu, const MF& A, const MF& Gs, double cg, const MF& FA, const MF& FU, int init,
-                 double ci) {
-    const SfKernels k = sf_kernels(c.geom, mu, nu);
-    hipLaunchKernelGGL(k.adj[mode], xgrid, blk, 0, c.stream, c.geom, L, A, Gs, cg, FA, FU, init, mF, ci);
-  };
-  auto fwd = [&](int mu, int nu, const MF& A, const MF& out) {
-    const SfKernels k = sf_kernels(c.geom, mu, nu);
-    hipLaunchKernelGGL(k.fwd, xgrid, blk, 0, c.stream, c.geom, L, A, out);
-  };
   for (int mu = 0; mu < 4; mu++) {
-    const MF Gmu = mf_link(G, mu);
+    const MF Gmu = mf_link(G, mu), Lmu = mf_link(L, mu);
     hipLaunchKernelGGL(k_sf_init, grid, blk, 0, c.stream, c.geom, mf_link(F1, mu), with_eps, mF, Gmu, c1);
     if (staples) {
-      // the three other directions and their buffers
       int od[3], k = 0;
+      SfKernels sk[3];
+      MF mS1[3], mG1[3], mG2[3];
       for (int d = 0; d < 4; d++)
-        if (d != mu) od[k++] = d;
-      MF mS1[4], mG2[4];
-      for (int i = 0; i < 3; i++) {
-        mS1[od[i]] = mf_site(S1[i], st);
-        mG2[od[i]] = mf_site(G2[i], st);
-      }
-      for (int i = 0; i < 3; i++) fwd(mu, od[i], mf_link(L, mu), mS1[od[i]]);
+        if (d != mu) {
+          sk[k] = sf_kernels(c.geom, mu, d);
+          mS1[k] = mf_site(S1[k], st);
+          mG1[k] = mf_site(G1[k], st);
+          mG2[k] = mf_site(G2[k], st);
+          od[k++] = d;
+        }
+      bool g1_set[3] = {false, false, false};
+      if (five || double_staple)
+        for (int i = 0; i < 3; i++)
+          hipLaunchKernelGGL(sk[i].fwd, xgrid, blk, 0, c.stream, c.geom, L, Lmu, mS1[i], (int)SF_BOTH);
       if (seven)
+        for (int i = 0; i < 3; i++)
+          hipLaunchKernelGGL(sk[i].fa, xgrid, blk, 0, c.stream, c.geom, L, mF, c7, mF, c5, mG2[i], (int)SF_BOTH);
+      if (double_staple)
         for (int i = 0; i < 3; i++) {
-          const int sig = od[i], nu = od[(i + 1) % 3], rho = od[(i + 2) % 3];
-          adj(1, mu, sig, none, mF, c7, mG2[sig], none, 1, c5);
-          const int p = std::min(nu, rho), q = std::max(nu, rho);
-          hipLaunchKernelGGL(sf_fwd2_kernel(c.geom, mu, p, q), xgrid, blk, 0, c.stream, c.geom, L, mS1[q], mS1[p],
-                             mSS);
-          adj(2, mu, sig, mSS, mF, c7, none, mf_link(G, sig), 0, 0.0);
+          hipLaunchKernelGGL(sk[i].fa, xgrid, blk, 0, c.stream, c.geom, L, mF, cl, mF, c3, mG1[i], (int)SF_BOTH);
+          hipLaunchKernelGGL(sk[i].fu, xgrid, blk, 0, c.stream, c.geom, L, mS1[i], mS1[i], mF, cl,
+                             mf_link(G, od[i]));
+          g1_set[i] = true;
+        }
+      if (five)
+        for (int i = 0; i < 3; i++) {
+          // outer direction od[i]; p < q the other two
+          const int p = i == 0 ? 1 : 0, q = i == 2 ? 1 : 2;
+          if (seven)
+            hipLaunchKernelGGL(sf_fwd2_kernel(c.geom, mu, od[p], od[q]), xgrid, blk, 0, c.stream, c.geom, L, mS1[q],
+                               mS1[p], mS1[i], ride ? cl / c7 : 0.0, mSS);
+          auto term = [&](int inner, int third) {
+            SfTerm t{mS1[inner], seven ? mG2[third] : mF, mG1[inner], mG2[inner], ride ? cl / c7 : 0.0,
+                     g1_set[inner] ? 0 : 1};
+            g1_set[inner] = true;
+            return t;
+          };
+          const SfTerm tp = term(p, q), tq = term(q, p);
+          hipLaunchKernelGGL(sk[i].adj5, xgrid, blk, 0, c.stream, c.geom, L, tp, tq, seven ? 1.0 : c5, mF,
+                             ride ? c3 - cl * c5 / c7 : c3, mSS, c7, mf_link(G, od[i]));
         }
       for (int i = 0; i < 3; i++) {
-        const int nu = od[i];
-        bool g1_set = false;
-        if (cl != 0.0) {
-          adj(0, mu, nu, mS1[nu], mF, cl, mG1, mf_link(G, nu), 1, c3);
-          g1_set = true;
+        const MF G1c = g1_set[i] ? mG1[i] : mF;
+        const double cg = g1_set[i] ? 1.0 : c3;
+        if (split) {
+          const MF up = mf_site(H[0], st), lo = mf_site(H[1], st), gp = mf_site(H[2], st), gm = mf_site(H[3], st);
+          hipLaunchKernelGGL(sk[i].fwd, xgrid, blk, 0, c.stream, c.geom, L, Lmu, up, (int)SF_UPPER);
+          hipLaunchKernelGGL(sk[i].fwd, xgrid, blk, 0, c.stream, c.geom, L, Lmu, lo, (int)SF_LOWER);
+          hipLaunchKernelGGL(sk[i].fu, xgrid, blk, 0, c.stream, c.geom, L, up, lo, mF, cl, mf_link(G, od[i]));
+          hipLaunchKernelGGL(sk[i].fa, xgrid, blk, 0, c.stream, c.geom, L, mF, cl, G1c, cg, gp, (int)SF_UPPER);
+          hipLaunchKernelGGL(sk[i].fa, xgrid, blk, 0, c.stream, c.geom, L, mF, cl, G1c, cg, gm, (int)SF_LOWER);
+          hipLaunchKernelGGL(sk[i].adj, xgrid, blk, 0, c.stream, c.geom, L, Lmu, gp, gm, 1.0, Gmu, mf_link(G, od[i]));
+        } else {
+          hipLaunchKernelGGL(sk[i].adj, xgrid, blk, 0, c.stream, c.geom, L, Lmu, G1c, G1c, cg, Gmu, mf_link(G, od[i]));
         }
-        if (five)
-          for (int j = 1; j < 3; j++) {
-            const int rho = od[(i + j) % 3], sig = od[(i + 3 - j) % 3];
-            adj(0, mu, rho, mS1[nu], seven ? mG2[sig] : mF, seven ? 1.0 : c5, mG1, mf_link(G, rho), g1_set ? 0 : 1,
-                c3);
-            g1_set = true;
-          }
-        adj(0, mu, nu, mf_link(L, mu), g1_set ? mG1 : mF, g1_set ? 1.0 : c3, Gmu, mf_link(G, nu), 0, 0.0);
       }
     }
     if (cN != 0.0)
@@ -1673,7 +1850,7 @@ int hisq_force_from_oprod(const LinkField& U, const LinkField& V, const LinkFiel
     return rc;
   }
   LinkField none{nullptr, 1.0f, 0};
-  if (use_staple_form(coeff2, true)) rc = smear_adjoint_dev(W, o1, o3, 1, coeff2, FW);
+  if (g_force_form) rc = smear_adjoint_dev(W, o1, o3, 1, coeff2, true, FW);  // W is U(3)-projected
   else rc = path_adjoint_launch(0, W, o1, o3, 1, coeff2, FW, none, 0.0, nullptr);
   if (!rc && one_link_extra) rc = link_axpy_dev(FW, *one_link_extra, 1.0, 1.0, 1);
   if (!rc) {
@@ -1681,8 +1858,8 @@ int hisq_force_from_oprod(const LinkField& U, const LinkField& V, const LinkFiel
     rc = hipGetLastError() == hipSuccess ? 0 : -1;
   }
   if (!rc) {
-    if (use_staple_form(coeff1, false)) {
-      rc = smear_adjoint_dev(U, FV, FV, 0, coeff1, FW);  // FW reused as F_U
+    if (g_force_form) {
+      rc = smear_adjoint_dev(U, FV, FV, 0, coeff1, g_force_form == 2, FW);  // FW reused as F_U
       if (!rc) {
         hipLaunchKernelGGL(k_mom_ta, dim3((c.Vh + 127) / 128, 8), dim3(128), 0, c.stream, c.geom, U, FW, scale,
                            mom_dev, 0);

@@ -626,8 +626,8 @@ class Lattice:
         return ne.value, md.value
 
     def set_force_form(self, form):
-        """0: path-table gather; 1 (default): staple form where exact for any
-        links, path table otherwise; 2: staple form everywhere (unitary links)"""
+        """0: path-table gather; 1 (default): staple form, for any links; 2:
+        staple form with the Lepage term as a double staple (unitary links)"""
         self._activate()
         _check(self.lib.milc_hip_set_force_form(form), "milc_hip_set_force_form")
 

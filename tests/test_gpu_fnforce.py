@@ -92,3 +92,36 @@ def test_asqtad_force_from_outer_products(l8):
         mom = np.zeros((L.V, 4, 10))
         G.asqtad_force(c, O1, O3, U, mom)
     assert rel(mom, ref) < 1e-12
+
+
+# which of {3-staple, 5-staple, 7-staple, Lepage} a path table has
+SUBSETS = [(1, 1, 1, 1), (1, 1, 0, 1), (1, 0, 0, 1), (0, 0, 0, 1), (1, 1, 1, 0), (0, 0, 1, 1), (1, 0, 0, 0), (0, 0, 0, 0)]
+
+
+@pytest.mark.parametrize("have", SUBSETS)
+@pytest.mark.parametrize("dims", [(4, 6, 4, 10), (6, 4, 8, 8), (8, 4, 4, 4)])
+def test_staple_form_against_the_path_table(have, dims):
+    """The staple form (1) follows the paths of the table (0) for links that are
+    not unitary, and with the Lepage term as a double staple (2) for links that
+    are; every subset of the smearing's terms, t-tiled site order or not.  The
+    path sums of a momentum are a few hundred products of matrices of norm
+    about one, summed in another order: 1e-13."""
+    full = ko.asqtad_coeffs(0.85)
+    c = [full[0], full[1]] + [full[2 + k] * have[k] for k in range(4)]
+    L = ko.Lattice(dims)
+    U = L.rephase(L.gauge_random(1031))
+    rng = np.random.default_rng(1032)
+    rough = np.ascontiguousarray(U * 0.9 + 0.05 * rng.standard_normal(U.shape))
+    xs = [L.gaussian_vector(1033 + t, ko.EVENANDODD) for t in range(2)]
+    with mq.Lattice(dims) as G:
+        try:
+            for links, form in ((rough, 1), (U, 1), (U, 2)):
+                mom = [np.zeros((L.V, 4, 10)), np.zeros((L.V, 4, 10))]
+                for m, f in zip(mom, (0, form)):
+                    G.set_force_form(f)
+                    G.fermion_force_fn_multi(0.1, [0.7, -0.4], xs, c, links, m)
+                err = np.linalg.norm(mom[1] - mom[0]) / np.linalg.norm(mom[0])
+                print(f"{dims} {have} form {form}: {err:.1e}", flush=True)
+                assert err < 1e-13
+        finally:
+            G.set_force_form(1)

@@ -1032,8 +1032,6 @@ extern "C" int milc_hip_fermion_force_fn_multi(int precision, double eps, const 
 // ---------------------------------------------------------------------------
 
 namespace {
-int batch_width(int nsrc) { return nsrc <= 4 ? 4 : (nsrc <= 8 ? 8 : 16); }
-
 struct BBuf {
   void* p = nullptr;
   BBuf() = default;
@@ -1094,6 +1092,7 @@ extern "C" int milc_hip_dev_block_tune(int prec, int nrhs, int* variant, double*
   if (!c.initialised || !c.links[P_F64].valid) return -1;
   int ip = block_prec(prec);
   if (ip != P_F64 && ensure_links(ip)) return -3;
+  if (nrhs != 4 && nrhs != 8 && nrhs != 16) return -2;
   int v;
   double us;
   int rc = btune(ip, nrhs, &v, &us);

@@ -412,16 +412,16 @@ struct BWork {
   double* partials = nullptr;
   float* W = nullptr;
   unsigned W_version = ~0u;
-  int tuned[3][3];      // [prec][nr index] -> variant, -1 untuned
-  double tuned_us[3][3];
+  int tuned[3][4];      // [prec][nr index] -> variant, -1 untuned
+  double tuned_us[3][4];
   BWork() {
     for (int a = 0; a < 3; a++)
-      for (int b = 0; b < 3; b++) tuned[a][b] = -1, tuned_us[a][b] = 0;
+      for (int b = 0; b < 4; b++) tuned[a][b] = -1, tuned_us[a][b] = 0;
   }
 };
 BWork g_bw;
 
-int nr_index(int nr) { return nr == 4 ? 0 : (nr == 8 ? 1 : (nr == 16 ? 2 : -1)); }
+int nr_index(int nr) { return nr == 4 ? 0 : (nr == 8 ? 1 : (nr == 16 ? 2 : (nr == 2 ? 3 : -1))); }
 
 // site-order block shapes offered to the tuner (index 0: checkerboard order)
 const int kOrders[4][4] = {{0, 0, 0, 0}, {8, 8, 8, 4}, {8, 4, 4, 4}, {4, 4, 4, 4}};
@@ -530,7 +530,8 @@ int launch_h16_tps(const BDOp& op, const BVariant& v, int* nb) {
       if constexpr (NR / 2 <= 8) return launch_h16<NR, 2>(op, v.block, v.loop, v.order, nb);
       break;
     case 4:
-      return launch_h16<NR, 4>(op, v.block, v.loop, v.order, nb);
+      if constexpr (NR >= 4) return launch_h16<NR, 4>(op, v.block, v.loop, v.order, nb);
+      break;
     case 8:
       if constexpr (NR >= 8) return launch_h16<NR, 8>(op, v.block, v.loop, v.order, nb);
       break;
@@ -583,7 +584,8 @@ int launch_valu_tps(const BDOp& op, const BVariant& v, int* nb) {
       if constexpr (NR / 2 <= RMAX) return launch_valu<P, NR, 2>(op, v.block, v.loop, v.order, nb);
       break;
     case 4:
-      return launch_valu<P, NR, 4>(op, v.block, v.loop, v.order, nb);
+      if constexpr (NR >= 4) return launch_valu<P, NR, 4>(op, v.block, v.loop, v.order, nb);
+      break;
     case 8:
       if constexpr (NR >= 8) return launch_valu<P, NR, 8>(op, v.block, v.loop, v.order, nb);
       break;
@@ -594,21 +596,24 @@ int launch_valu_tps(const BDOp& op, const BVariant& v, int* nb) {
 int launch_variant(const BDOp& op, const BVariant& v, int* nb) {
   if (op.prec == P_H16) {
     if (v.mfma) return -2;
+    if (op.nr == 2) return launch_h16_tps<2>(op, v, nb);
     if (op.nr == 4) return launch_h16_tps<4>(op, v, nb);
     if (op.nr == 8) return launch_h16_tps<8>(op, v, nb);
     return launch_h16_tps<16>(op, v, nb);
   }
   if (v.mfma) {
-    if (op.prec != P_F32) return -2;
+    if (op.prec != P_F32 || op.nr < 4) return -2;  // four columns to a block
     if (op.nr == 4) return launch_mfma<4>(op, v.block, v.loop, v.order, nb);
     if (op.nr == 8) return launch_mfma<8>(op, v.block, v.loop, v.order, nb);
     return launch_mfma<16>(op, v.block, v.loop, v.order, nb);
   }
   if (op.prec == P_F64) {
+    if (op.nr == 2) return launch_valu_tps<P_F64, 2>(op, v, nb);
     if (op.nr == 4) return launch_valu_tps<P_F64, 4>(op, v, nb);
     if (op.nr == 8) return launch_valu_tps<P_F64, 8>(op, v, nb);
     return launch_valu_tps<P_F64, 16>(op, v, nb);
   }
+  if (op.nr == 2) return launch_valu_tps<P_F32, 2>(op, v, nb);
   if (op.nr == 4) return launch_valu_tps<P_F32, 4>(op, v, nb);
   if (op.nr == 8) return launch_valu_tps<P_F32, 8>(op, v, nb);
   return launch_valu_tps<P_F32, 16>(op, v, nb);
@@ -644,7 +649,7 @@ std::vector<BVariant> bvariants(int prec, int nr) {
           v.push_back(BVariant{0, tps, block, loop, order});
         }
     }
-  if (prec == P_F32)
+  if (prec == P_F32 && nr >= 4)
     for (int order : orders)
       for (int block : {128, 256})
         for (int loop : {1, 2, 4}) {
@@ -770,15 +775,18 @@ int bpack(const VecField& in, void* batched, int prec, int nr, int r) {
   Context& c = ctx();
   dim3 grid((c.Vh + 255) / 256);
   if (prec == P_H16) {
-    if (nr == 4) hipLaunchKernelGGL((k_bpack_h16<4>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
+    if (nr == 2) hipLaunchKernelGGL((k_bpack_h16<2>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
+    else if (nr == 4) hipLaunchKernelGGL((k_bpack_h16<4>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bpack_h16<8>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
     else hipLaunchKernelGGL((k_bpack_h16<16>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
   } else if (prec == P_F64) {
-    if (nr == 4) hipLaunchKernelGGL((k_bpack<double, 4>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
+    if (nr == 2) hipLaunchKernelGGL((k_bpack<double, 2>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
+    else if (nr == 4) hipLaunchKernelGGL((k_bpack<double, 4>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bpack<double, 8>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
     else hipLaunchKernelGGL((k_bpack<double, 16>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
   } else {
-    if (nr == 4) hipLaunchKernelGGL((k_bpack<float, 4>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
+    if (nr == 2) hipLaunchKernelGGL((k_bpack<float, 2>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
+    else if (nr == 4) hipLaunchKernelGGL((k_bpack<float, 4>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bpack<float, 8>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
     else hipLaunchKernelGGL((k_bpack<float, 16>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
   }
@@ -790,15 +798,18 @@ int bunpack(const void* batched, int prec, int nr, int r, VecField& out) {
   Context& c = ctx();
   dim3 grid((c.Vh + 255) / 256);
   if (prec == P_H16) {
-    if (nr == 4) hipLaunchKernelGGL((k_bunpack_h16<4>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
+    if (nr == 2) hipLaunchKernelGGL((k_bunpack_h16<2>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
+    else if (nr == 4) hipLaunchKernelGGL((k_bunpack_h16<4>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bunpack_h16<8>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
     else hipLaunchKernelGGL((k_bunpack_h16<16>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
   } else if (prec == P_F64) {
-    if (nr == 4) hipLaunchKernelGGL((k_bunpack<double, 4>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
+    if (nr == 2) hipLaunchKernelGGL((k_bunpack<double, 2>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
+    else if (nr == 4) hipLaunchKernelGGL((k_bunpack<double, 4>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bunpack<double, 8>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
     else hipLaunchKernelGGL((k_bunpack<double, 16>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
   } else {
-    if (nr == 4) hipLaunchKernelGGL((k_bunpack<float, 4>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
+    if (nr == 2) hipLaunchKernelGGL((k_bunpack<float, 2>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
+    else if (nr == 4) hipLaunchKernelGGL((k_bunpack<float, 4>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bunpack<float, 8>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
     else hipLaunchKernelGGL((k_bunpack<float, 16>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
   }

@@ -67,13 +67,21 @@ struct FPtrs {
 // ---------------------------------------------------------------------------
 // multi-shift kernels
 // ---------------------------------------------------------------------------
+// The scalar kernels run one thread per (rhs, shift), thread 32 r + j, in one
+// workgroup (one thread per rhs walking its shifts and window coefficients took
+// tens of microseconds per iteration with 7 to 12 shifts).
+constexpr int kScalarThreads = 32 * BNR_MAX;
+static_assert(BMS_MAX == 32, "one half-wavefront of shifts per right-hand side");
+
 __global__ void k_bms_reset(BMSR* __restrict__ s, const BMSG* __restrict__ g) {
-  int r = threadIdx.x;
+  const int r = threadIdx.x >> 5, j = threadIdx.x & 31;
   if (r >= g->nr) return;
   BMSR& S = s[r];
-  S.m = 0;
-  S.now_ws = S.num_now;
-  for (int j = 0; j < g->n; j++) {
+  if (j == 0) {
+    S.m = 0;
+    S.now_ws = S.num_now;
+  }
+  if (j < g->n) {
     S.wa[j] = 1.0;
     S.wx[j] = 0.0;
     for (int l = 0; l < BKW; l++) S.wc[j][l] = S.wb[j][l] = 0.0;
@@ -82,82 +90,96 @@ __global__ void k_bms_reset(BMSR* __restrict__ s, const BMSG* __restrict__ g) {
 
 // beta/zeta recurrences (ks_multicg_offset.c:322-356) and the solution-update
 // coefficients of this iteration
-__global__ void k_bms_beta(const double* __restrict__ sums, BMSR* __restrict__ s, BMSG* __restrict__ g) {
-  int r = threadIdx.x;
+__global__ void __launch_bounds__(kScalarThreads) k_bms_beta(const double* __restrict__ sums, BMSR* __restrict__ s,
+                                                             BMSG* __restrict__ g) {
+  const int r = threadIdx.x >> 5, j = threadIdx.x & 31;
   if (g->halt_all) return;
-  if (r < g->nr && !s[r].halt) {
-    BMSR& S = s[r];
-    const int jl = S.j_low;
-    double pkp = sums[r];
+  const bool live = r < g->nr && !s[r].halt;
+  int jl = 0, m = 0, now = 0, now1 = 0;
+  double beta = 0, zip1 = 0;
+  if (live) {
+    const BMSR& S = s[r];
+    jl = S.j_low;
+    m = S.m + 1;
+    now = S.num_now;
+    const double beta_low = -S.rsq / sums[r], beta_low_1 = S.beta_im1[jl];
+    // only the last shift can retire (its zeta has underflown)
+    now1 = now - 1 > jl && S.zeta_i[now - 1] == 0.0 ? now - 1 : now;
+    if (j == jl) {
+      beta = beta_low;
+      zip1 = 1.0;
+    } else if (j < now) {
+      const double zi = S.zeta_i[j], zm = S.zeta_im1[j];
+      zip1 = zi * zm * beta_low_1;
+      const double c1 = beta_low * S.alpha[jl] * (zm - zi);
+      const double c2 = zm * beta_low_1 * (1.0 + S.shifts[j] * beta_low);
+      zip1 = c1 + c2 != 0.0 ? zip1 / (c1 + c2) : 0.0;
+      if (zi != 0.0) beta = beta_low * zip1 / zi;
+      else zip1 = 0.0;
+    }
+  }
+  __syncthreads();
+  if (!live) return;
+  BMSR& S = s[r];
+  if (j == 0) {
     S.iters += 1;
-    int m = S.m + 1;
     S.m = m;
-    S.beta_i[jl] = -S.rsq / pkp;
-    S.zeta_ip1[jl] = 1.0;
-    int now = S.num_now;
-    for (int j = 0; j < now; j++) {
-      if (j == jl) continue;
-      S.zeta_ip1[j] = S.zeta_i[j] * S.zeta_im1[j] * S.beta_im1[jl];
-      double c1 = S.beta_i[jl] * S.alpha[jl] * (S.zeta_im1[j] - S.zeta_i[j]);
-      double c2 = S.zeta_im1[j] * S.beta_im1[jl] * (1.0 + S.shifts[j] * S.beta_i[jl]);
-      if (c1 + c2 != 0.0) S.zeta_ip1[j] /= c1 + c2;
-      else S.zeta_ip1[j] = 0.0;
-      if (S.zeta_i[j] != 0.0) {
-        S.beta_i[j] = S.beta_i[jl] * S.zeta_ip1[j] / S.zeta_i[j];
-      } else {
-        S.zeta_ip1[j] = 0.0;
-        S.beta_i[j] = 0.0;
-        if (j == now - 1 && j > jl) now--;
-      }
-    }
-    S.num_now = now;
-    // psim_j += beta_j pm_j^(s+m-1), pm_j^(s+m-1) = wa pm_j^(s) + sum_{l<m-1} wc_l r^(s+1+l)
-    for (int j = 0; j < now; j++) {
-      double b = S.beta_i[j];
-      S.wx[j] += b * S.wa[j];
-      for (int l = 0; l < m - 1; l++) S.wb[j][l] += b * S.wc[j][l];
-    }
+    S.num_now = now1;
+  }
+  if (j < now) {
+    S.beta_i[j] = beta;
+    S.zeta_ip1[j] = zip1;
+  }
+  // psim_j += beta_j pm_j^(s+m-1), pm_j^(s+m-1) = wa pm_j^(s) + sum_{l<m-1} wc_l r^(s+1+l)
+  if (j < now1) {
+    S.wx[j] += beta * S.wa[j];
+    for (int l = 0; l < m - 1; l++) S.wb[j][l] += beta * S.wc[j][l];
   }
 }
 
 // convergence, alpha recurrences (ks_multicg_offset.c:358-463), search-direction
 // coefficients of this iteration, scalar scroll
-__global__ void k_bms_alpha(const double* __restrict__ sums, BMSR* __restrict__ s, BMSG* __restrict__ g) {
-  int r = threadIdx.x;
+__global__ void __launch_bounds__(kScalarThreads) k_bms_alpha(const double* __restrict__ sums, BMSR* __restrict__ s,
+                                                              BMSG* __restrict__ g) {
+  const int r = threadIdx.x >> 5, j = threadIdx.x & 31;
   if (g->halt_all) return;
-  if (r < g->nr && !s[r].halt) {
+  const bool live = r < g->nr && !s[r].halt;
+  double rsq = 0, oldrsq = 0, alpha_low = 0, beta_low = 0;
+  int jl = 0, now = 0, m = 0;
+  bool met = false;
+  if (live) {
+    const BMSR& S = s[r];
+    rsq = sums[r];
+    oldrsq = S.rsq;
+    met = S.rsqstop > 0 && rsq <= S.rsqstop;
+    jl = S.j_low;
+    now = S.num_now;
+    m = S.m;
+    alpha_low = rsq / oldrsq;
+    beta_low = S.beta_i[jl];
+  }
+  __syncthreads();
+  if (live) {
     BMSR& S = s[r];
-    const int jl = S.j_low;
-    double rsq = sums[r];
-    S.oldrsq = S.rsq;
-    S.rsq = rsq;
-    if (S.rsqstop > 0 && rsq <= S.rsqstop) {
-      S.halt = 1;
-      S.converged = 1;
-    } else {
-      int now = S.num_now, m = S.m;
-      S.alpha[jl] = rsq / S.oldrsq;
-      for (int j = 0; j < now; j++) {
-        if (j == jl) continue;
-        if (S.zeta_i[j] * S.beta_i[jl] != 0.0)
-          S.alpha[j] = S.alpha[jl] * S.zeta_ip1[j] * S.beta_i[j] / (S.zeta_i[j] * S.beta_i[jl]);
-        else
-          S.alpha[j] = 0.0;
-      }
+    if (!met && j < now) {
+      const double zi = S.zeta_i[j], zip1 = S.zeta_ip1[j], beta = S.beta_i[j];
+      double a = alpha_low;
+      if (j != jl) a = zi * beta_low != 0.0 ? alpha_low * zip1 * beta / (zi * beta_low) : 0.0;
+      S.alpha[j] = a;
       // pm_j = zeta_ip1 r + alpha pm_j
-      for (int j = 0; j < now; j++) {
-        double a = S.alpha[j];
-        S.wa[j] *= a;
-        for (int l = 0; l < m - 1; l++) S.wc[j][l] *= a;
-        S.wc[j][m - 1] = S.zeta_ip1[j];
-      }
-      for (int j = 0; j < now; j++) {
-        S.beta_im1[j] = S.beta_i[j];
-        S.zeta_im1[j] = S.zeta_i[j];
-        S.zeta_i[j] = S.zeta_ip1[j];
-      }
+      S.wa[j] *= a;
+      for (int l = 0; l < m - 1; l++) S.wc[j][l] *= a;
+      S.wc[j][m - 1] = zip1;
+      S.beta_im1[j] = beta;
+      S.zeta_im1[j] = zi;
+      S.zeta_i[j] = zip1;
+    }
+    if (j == 0) {
+      S.oldrsq = oldrsq;
+      S.rsq = rsq;
+      if (met) S.halt = S.converged = 1;
       // the loop of ks_multicg_offset.c ends when iteration reaches niter
-      if (1 + S.iters >= g->max_iter) S.halt = 1;
+      else if (1 + S.iters >= g->max_iter) S.halt = 1;
     }
   }
   __syncthreads();
@@ -579,9 +601,9 @@ int bnorms(const void* f, int prec, int nr, double* sums_dev, double* out) {
   hipLaunchKernelGGL((k_bnorm<R, N>), dim3(rg.nb), dim3(256), 0, c.stream, (const R*)f, rg.nrec, rg.loop, part, \
                      ps)
   if (prec == P_F64) {
-    if (nr == 4) BN_CASE(double, 4); else if (nr == 8) BN_CASE(double, 8); else BN_CASE(double, 16);
+    if (nr == 2) BN_CASE(double, 2); else if (nr == 4) BN_CASE(double, 4); else if (nr == 8) BN_CASE(double, 8); else BN_CASE(double, 16);
   } else {
-    if (nr == 4) BN_CASE(float, 4); else if (nr == 8) BN_CASE(float, 8); else BN_CASE(float, 16);
+    if (nr == 2) BN_CASE(float, 2); else if (nr == 4) BN_CASE(float, 4); else if (nr == 8) BN_CASE(float, 8); else BN_CASE(float, 16);
   }
 #undef BN_CASE
   MH_CHECK(hipGetLastError());
@@ -685,7 +707,7 @@ int bmultishift_nr(const void* b64, const double* offs, int n, const double* res
   // one window: reset, K iterations (ks_multicg_offset.c:291-460), flush
   auto window = [&]() -> int {
     int r2;
-    hipLaunchKernelGGL(k_bms_reset, dim3(1), dim3(64), 0, c.stream, ds, dg);
+    hipLaunchKernelGGL(k_bms_reset, dim3(1), dim3(kScalarThreads), 0, c.stream, ds, dg);
     for (int m = 1; m <= BKW; m++) {
       float* rprev = ring0 + (size_t)(m - 1) * ring_stride;
       float* rcur = ring0 + (size_t)m * ring_stride;
@@ -709,11 +731,11 @@ int bmultishift_nr(const void* b64, const double* offs, int n, const double* res
       int nb2 = 0;
       if ((r2 = bdslash(d2, &nb2))) return r2;
       if ((r2 = breduce(NR, nb2, dsum))) return r2;
-      hipLaunchKernelGGL(k_bms_beta, dim3(1), dim3(64), 0, c.stream, dsum, ds, dg);
+      hipLaunchKernelGGL(k_bms_beta, dim3(1), dim3(kScalarThreads), 0, c.stream, dsum, ds, dg);
       hipLaunchKernelGGL(k_bms_r<NR>, dim3(rg.nb), dim3(256), 0, c.stream, rprev, rcur, (const float*)ttt.p, ds, dg,
                          rg.nrec, rg.loop, part, pstride);
       if ((r2 = breduce(NR, rg.nb, dsum + 32))) return r2;
-      hipLaunchKernelGGL(k_bms_alpha, dim3(1), dim3(64), 0, c.stream, dsum + 32, ds, dg);
+      hipLaunchKernelGGL(k_bms_alpha, dim3(1), dim3(kScalarThreads), 0, c.stream, dsum + 32, ds, dg);
       hipLaunchKernelGGL(k_bms_p<NR>, dim3(rg.nb), dim3(256), 0, c.stream, (float*)p.p, rcur, ds, dg, rg.nrec,
                          rg.loop);
     }
@@ -929,7 +951,8 @@ int bmultishift_sets(const void* b64, int nr, int n, const double* offs, const d
                      const double* refine_resid, const BMSParams& prm, std::vector<void*>& x64, BMSStats& st) {
   int rc;
   st = BMSStats();
-  if (nr == 4) rc = bmultishift_nr<4>(b64, offs, n, stage_resid, prm, x64, st);
+  if (nr == 2) rc = bmultishift_nr<2>(b64, offs, n, stage_resid, prm, x64, st);
+  else if (nr == 4) rc = bmultishift_nr<4>(b64, offs, n, stage_resid, prm, x64, st);
   else if (nr == 8) rc = bmultishift_nr<8>(b64, offs, n, stage_resid, prm, x64, st);
   else if (nr == 16) rc = bmultishift_nr<16>(b64, offs, n, stage_resid, prm, x64, st);
   else return -2;
@@ -977,6 +1000,7 @@ int bmultishift(const void* b64, int nr, const std::vector<double>& offsets, con
 
 int bcg_mixed(const void* b64, void* x64, int nr, const double* offsets, const BCGParams& prm, BCGStats& st) {
   st = BCGStats();
+  if (nr == 2) return bcg_mixed_nr<2>(b64, x64, offsets, prm, st);
   if (nr == 4) return bcg_mixed_nr<4>(b64, x64, offsets, prm, st);
   if (nr == 8) return bcg_mixed_nr<8>(b64, x64, offsets, prm, st);
   if (nr == 16) return bcg_mixed_nr<16>(b64, x64, offsets, prm, st);

@@ -137,7 +137,7 @@ static int rational_solve_all(const std::vector<const VecField*>& src, const std
                               const std::vector<double>& resid, std::vector<std::vector<VecField>>& x, long* iters) {
   const int ns = (int)src.size();
   if (ns < 1 || ns > BNR_MAX || (int)offs.size() != ns || (int)resid.size() != ns) return -2;
-  const int nr = ns <= 4 ? 4 : (ns <= 8 ? 8 : 16);
+  const int nr = batch_width(ns);
   int n = 0;
   for (auto& o : offs) {
     if (o.empty() || (int)o.size() > BMS_MAX) return -2;

@@ -255,3 +255,26 @@ def test_batched_solvers_stop_at_max_iters(l8):
             it, fres = G.ks_congrad_block_parity(srcs, dests, q, 0.05)
             assert it <= cap + 1 and q.converged == 0, (cap, it)
             assert max(fres) > 1e-14
+
+
+@pytest.mark.parametrize("dims", [(4, 4, 4, 4), (6, 4, 8, 6), (8, 6, 4, 10)])
+@pytest.mark.parametrize("nsrc,nshift", [(1, 1), (2, 1), (2, 12), (2, 32), (3, 31)])
+def test_multishift_block_narrow_batches_vs_oracle(dims, nsrc, nshift):
+    """Batches of two (one and two sources) and the next width up, with one
+    shift to the most: solutions against the oracle's multi-shift CG to 1e-13.
+    A shift refined to the true residual r is off by r |b| / (offset |x|) at
+    most, and |x| >= |b| / (offset + 10)."""
+    L, fat, lng = hisq_setup(dims, 1007)
+    offs = [0.04 * 1.3 ** j for j in range(nshift)]
+    resid = 1e-9
+    with mq.Lattice(dims) as G:
+        G.set_links(fat, lng)
+        for parity in (ko.EVEN, ko.ODD):
+            sl = L.parity_slice(parity)
+            srcs = [L.gaussian_vector(720 + s, parity) for s in range(nsrc)]
+            psim, res, _ = G.ks_multicg_offset_block(srcs, offs, parity, 1e-7, resid)
+            assert max(max(r) for r in res) < resid
+            for s in range(nsrc):
+                ref, _, _ = L.multicg_offset(fat, lng, srcs[s], offs, 1e-13, parity=parity, max_iters=3000)
+                for j in range(nshift):
+                    assert rel(psim[s][j][sl], ref[j][sl]) < resid * (offs[j] + 10) / offs[j]

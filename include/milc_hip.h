@@ -455,7 +455,8 @@ int milc_hip_dev_block_dslash(int prec, int nrhs, int variant, int nsrc, const i
  * solutions of the first out_nsrc sources to slots out_slot0 + s * num_offsets + j
  * when out_slot0 >= 0.
  * stats[0..5] = multi-shift iterations, multi-shift seconds, refinement
- * seconds, converged, stencil variant, its time (us); stats[6 + j] = max true
+ * seconds, converged, stencil variant, its time (us; -1 and 0 where the sources
+ * of a small lattice were solved one after another in FP64); stats[6 + j] = max true
  * residual of shift j, stats[6 + num_offsets + j] = its refinement iterations.
  * Returns the multi-shift iteration count. */
 int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int num_offsets, const double* offsets,

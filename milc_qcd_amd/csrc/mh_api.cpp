@@ -1163,6 +1163,51 @@ extern "C" int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int
     if (!slot_ok(src_slots[s], true)) return -2;
   if (out_slot0 >= 0 && (out_nsrc < 0 || out_nsrc > nsrc || out_slot0 + out_nsrc * num_offsets > kSlots)) return -2;
   int rc;
+  if (refine_resid > 0 && max_iters != 1 && block_is_small(nsrc)) {
+    for (int j = 0; j < num_offsets; j++)
+      if (!(offsets[j] > 0)) return -2;
+    auto t0 = std::chrono::steady_clock::now();
+    std::vector<double> offs(offsets, offsets + num_offsets), res(num_offsets, refine_resid), rel(num_offsets);
+    std::vector<double> worst(num_offsets, 0.0);
+    long most = 0;
+    int conv = 1;
+    for (int s = 0; s < nsrc; s++) {
+      std::vector<VecField> xs(num_offsets);
+      VecScope owned;
+      for (auto& v : xs) {
+        owned.add(&v);
+        if ((rc = alloc_vec(v, P_F64, c.stride))) return rc;
+      }
+      long it = 0;
+      int ok = 1;
+      if ((rc = multishift_small(g_slots[src_slots[s]], xs, offs, res.data(), parity, max_iters > 0 ? max_iters : 20000,
+                                 &it, rel.data(), &ok)))
+        return rc;
+      most = std::max(most, it);
+      conv &= ok;
+      for (int j = 0; j < num_offsets; j++) {
+        worst[j] = std::max(worst[j], rel[j]);
+        const int slot = out_slot0 + s * num_offsets + j;
+        if (out_slot0 >= 0 && s < out_nsrc &&
+            ((rc = ensure_slot(slot)) || (rc = vec_copy(xs[j], g_slots[slot], P_F64))))
+          return rc;
+      }
+    }
+    MH_CHECK(hipStreamSynchronize(c.stream));
+    if (stats) {
+      stats[0] = most;
+      stats[1] = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+      stats[2] = 0;
+      stats[3] = conv;
+      stats[4] = -1;
+      stats[5] = 0;
+      for (int j = 0; j < num_offsets; j++) {
+        stats[6 + j] = worst[j];
+        stats[6 + num_offsets + j] = 0;
+      }
+    }
+    return (int)most;
+  }
   if ((rc = ensure_links(P_F32))) return rc;
   const int nr = batch_width(nsrc);
   BBuf b;
@@ -1224,9 +1269,38 @@ extern "C" int milc_hip_multishift_invert_block(int external_precision, int nsrc
   if (parity < 0) return -2;
   int rc;
   if ((rc = refresh_links(external_precision, fatlink, longlink, num_iters))) return rc;
-  if ((rc = ensure_links(P_F32))) return rc;
   const int pb = pbit(parity);
   int total = 0;
+  bool positive = true;
+  for (int j = 0; j < num_offsets; j++) positive = positive && offsets[j] > 0;
+  if (refine_residual > 0 && positive && args.max_iter != 1 && block_is_small(nsrc)) {
+    std::vector<double> offs(offsets, offsets + num_offsets), res(num_offsets, refine_residual), rel(num_offsets);
+    VecField v;
+    std::vector<VecField> xs(num_offsets);
+    VecScope owned{&v};
+    if ((rc = alloc_vec(v, P_F64, c.stride))) return rc;
+    for (auto& f : xs) {
+      owned.add(&f);
+      if ((rc = alloc_vec(f, P_F64, c.stride))) return rc;
+    }
+    for (int s = 0; s < nsrc; s++) {
+      long it = 0;
+      int ok = 1;
+      if ((rc = host_vec_in(external_precision, source[s], v, pb)) ||
+          (rc = multishift_small(v, xs, offs, res.data(), parity, args.max_iter > 0 ? args.max_iter : 20000, &it,
+                                 rel.data(), &ok)))
+        return rc;
+      for (int j = 0; j < num_offsets; j++) {
+        const size_t k = (size_t)s * num_offsets + j;
+        if ((rc = host_vec_out(external_precision, xs[j], pb, solution[k]))) return rc;
+        if (final_residual) final_residual[k] = rel[j];
+      }
+      total = std::max(total, (int)it);
+    }
+    if (num_iters) *num_iters = total;
+    return total;
+  }
+  if ((rc = ensure_links(P_F32))) return rc;
   for (int s0 = 0; s0 < nsrc; s0 += BNR_MAX) {
     int ns = std::min(BNR_MAX, nsrc - s0);
     int nr = batch_width(ns);
@@ -1287,9 +1361,35 @@ extern "C" int milc_hip_invert_block(int external_precision, int nsrc, double ma
   if (parity < 0) return -2;
   int rc;
   if ((rc = refresh_links(external_precision, fatlink, longlink, num_iters))) return rc;
-  if ((rc = ensure_links(P_F32))) return rc;
   const int pb = pbit(parity);
   int total = 0;
+  if (block_is_small(nsrc)) {
+    SolveParams sp;
+    sp.parity = parity;
+    sp.max_iters = args.max_iter > 0 ? args.max_iter : 20000;
+    sp.max_restarts = 1;
+    sp.resid = target_residual;
+    sp.relresid = 0;
+    sp.sloppy_prec = P_F64;
+    sp.delta = kReliableDelta;
+    sp.batch = 16;
+    VecField b, x;
+    VecScope owned{&b, &x};
+    if ((rc = alloc_vec(b, P_F64, c.stride)) || (rc = alloc_vec(x, P_F64, c.stride))) return rc;
+    for (int s = 0; s < nsrc; s++) {
+      SolveStats st;
+      // t_dest is the initial guess (d_congrad5_fn_gpu.c:104-110)
+      if ((rc = host_vec_in(external_precision, source[s], b, pb)) ||
+          (rc = host_vec_in(external_precision, solution[s], x, pb)) || (rc = cg_solve_restarting(b, x, mass, sp, st)) ||
+          (rc = host_vec_out(external_precision, x, pb, solution[s])))
+        return rc;
+      if (final_residual) final_residual[s] = std::sqrt(st.final_rsq);
+      total = std::max(total, st.iters);
+    }
+    if (num_iters) *num_iters = total;
+    return total;
+  }
+  if ((rc = ensure_links(P_F32))) return rc;
   for (int s0 = 0; s0 < nsrc; s0 += BNR_MAX) {
     int ns = std::min(BNR_MAX, nsrc - s0);
     int nr = batch_width(ns);

@@ -1373,6 +1373,13 @@ size_t cg_scratch_bytes(int ps, int Vh, int stride) {
   return 2 * a(P_F64) + 2 * a(ps) + 3 * a(ps == P_H16 ? kH16Arith : P_F32);
 }
 
+// FP64 CG that restarts from the true residual until that meets the target
+// (or max_restarts * max_iters iterations are done).
+int cg_solve_restarting(const VecField& src, VecField& x, double mass, const SolveParams& sp, SolveStats& st) {
+  const long max_cg = (long)sp.max_restarts * sp.max_iters;
+  return cg_solve_f64(src, x, mass, sp, (int)std::min<long>(max_cg, 1L << 30), max_cg, 1 << 30, st);
+}
+
 int cg_solve(const VecField& src, VecField& x, double mass, const SolveParams& sp, SolveStats& st) {
   auto t0 = std::chrono::steady_clock::now();
   int rc;
@@ -1381,7 +1388,7 @@ int cg_solve(const VecField& src, VecField& x, double mass, const SolveParams& s
   // on a small lattice the FP64 loop in one kernel is the fastest solve for
   // any sloppy precision: it restarts until the true residual meets the target
   else if (sp.relresid <= 0 && ctx().Vh <= kPersistMixedSites && persist_shape(ctx().Vh).lps)
-    rc = cg_solve_f64(src, x, mass, sp, (int)std::min<long>(max_cg, 1L << 30), max_cg, 1 << 30, st);
+    rc = cg_solve_restarting(src, x, mass, sp, st);
   else if (sp.sloppy_prec == P_F32) rc = cg_solve_mixed<P_F32, P_F32>(src, x, mass, sp, st);
   else rc = cg_solve_mixed<P_H16, kH16Arith>(src, x, mass, sp, st);
   (void)hipStreamSynchronize(ctx().stream);

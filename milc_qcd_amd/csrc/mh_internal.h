@@ -210,6 +210,7 @@ struct SolveStats {
   double seconds = 0;
 };
 int cg_solve(const VecField& src, VecField& x, double mass, const SolveParams& sp, SolveStats& st);
+int cg_solve_restarting(const VecField& src, VecField& x, double mass, const SolveParams& sp, SolveStats& st);
 // builds the sloppy copy of the FP64 device links in precision prec if absent
 int ensure_links(int prec);
 
@@ -233,6 +234,8 @@ bool multishift_is_small(int sources = 1);
 // target finished by its own CG.  iters, fres and converged as refine_shifts.
 int multishift_small(const VecField& b, std::vector<VecField>& x, const std::vector<double>& offsets,
                      const double* resid, int parity, int max_iters, long* iters, double* fres, int* converged);
+// Whether a block call of `sources` sources solves them one after another.
+bool block_is_small(int sources);
 int shift_residuals(const VecField& b, const std::vector<VecField>& x, const double* offsets, int parity, double* rel);
 
 // ---- force outer products ---------------------------------------------------

@@ -493,10 +493,33 @@ bool multishift_is_small(int sources) {
   return ctx().Vh <= persist_mixed_shift_sites(sources) && persist_shape(ctx().Vh).lps && ctx().links[P_F64].valid;
 }
 
+bool block_is_small(int sources) {
+  return ctx().Vh <= persist_block_sites(sources) && persist_shape(ctx().Vh).lps && ctx().links[P_F64].valid;
+}
+
 int multishift_small(const VecField& b, std::vector<VecField>& x, const std::vector<double>& offsets,
                      const double* resid, int parity, int max_iters, long* iters, double* fres, int* converged) {
   const int n = (int)offsets.size();
   if (n <= 0 || n > MS_MAX) return -2;
+  if (n == 1) {
+    // a CG: one exchange of sums per iteration instead of two
+    SolveParams sp;
+    sp.parity = parity;
+    sp.max_iters = max_iters;
+    sp.max_restarts = 1;
+    sp.resid = resid[0];
+    sp.relresid = 0;
+    sp.sloppy_prec = P_F64;
+    sp.delta = kReliableDelta;
+    sp.batch = 16;
+    SolveStats st;
+    int rc = vec_zero(x[0], P_F64);
+    if (rc || (rc = cg_solve_restarting(b, x[0], 0.5 * std::sqrt(offsets[0]), sp, st))) return rc;
+    *iters += st.iters;
+    *converged = st.converged;
+    if (fres) fres[0] = std::sqrt(st.final_rsq);
+    return 0;
+  }
   int low = 0;
   for (int j = 1; j < n; j++)
     if (offsets[j] < offsets[low]) low = j;

@@ -40,6 +40,14 @@ int cg_persist(VecField& x, VecField& r, VecField (&work)[4], int pb, double msq
 constexpr int persist_mixed_shift_sites(int sources) {
   return sources <= 2 ? 131072 : (sources == 3 ? 65536 : (sources == 4 ? 16384 : (sources <= 6 ? 4096 : 0)));
 }
+// Sites per parity up to which the sources of a block call are solved one after
+// another in one kernel each instead of as a batch (ms of one source here, of
+// batches of 2 / 4 / 8 sources, CG to 1e-9 at m = 0.03: Vh = 2048 0.67, 4.5 /
+// 4.2 / 4.4; 6000 0.93, 5.9 / 5.5 / 6.1; 13824 1.6, 7.7 / 6.9 / 8.6; 32768 3.5,
+// 9.7 / 9.5 / 12.9; 65536 8.3, 18.1 / 20.4 / 27.5; two-shift multi-shifts alike).
+constexpr int persist_block_sites(int sources) {
+  return sources <= 2 ? 65536 : (sources <= 4 ? 16384 : (sources <= 6 ? 8192 : 0));
+}
 
 // What one FP64 multi-shift solve in one kernel takes and gives back (device memory).
 struct MSPersist {

@@ -105,3 +105,37 @@ def test_multishift_one_kernel_shift_counts_and_retirement(n):
             assert qic[0].final_iters == it_ref
             for a, b in zip(x, ref):
                 assert np.linalg.norm(a[s] - b[s]) < 1e-9 * max(np.linalg.norm(b[s]), 1e-300)
+
+
+@pytest.mark.parametrize("dims,nsrc", [((6, 4, 8, 6), 1), ((6, 4, 8, 6), 6), ((6, 4, 8, 6), 7), ((12, 12, 12, 16), 4),
+                                       ((12, 12, 12, 16), 5), ((12, 12, 12, 24), 2), ((12, 12, 12, 24), 3)])
+def test_block_calls_on_both_sides_of_the_dispatch(dims, nsrc):
+    """Block CG (with an initial guess) and block multi-shift of one and three
+    shifts, just where the sources are solved one after another and just where
+    they go as a batch: true residuals and single-source solutions."""
+    resid, mass = 1e-9, 0.1
+    print(f"block calls {dims} x {nsrc}", flush=True)
+    with mq.Lattice(dims) as G:
+        G.dev_gauge_hisq(1410)
+        fat, lng = G.dev_read_links()
+        E = G.parity_slice(mq.EVEN)
+        srcs = []
+        for s in range(nsrc):
+            G.dev_source(1411 + s, mq.EVEN, s)
+            srcs.append(G.dev_read(s, mq.EVEN))
+        G.set_links(fat, lng)
+        qic = mq.QuarkInvertControl(max=3000, nrestart=1, parity=mq.EVEN, resid=resid)
+        dests = [0.3 * v for v in srcs]
+        _, res = G.ks_congrad_block_parity(srcs, dests, qic, mass)
+        assert max(res) < resid
+        for offs in ([4 * mass ** 2], [4 * mass ** 2, 0.3, 2.0]):
+            st = G.dev_multishift_block(list(range(nsrc)), offs, 1e-7, resid, out_slot0=20)
+            assert st["converged"] and max(st["true_rel"]) < resid
+            for s in range(nsrc):
+                for j, o in enumerate(offs):
+                    G.dev_invert(s, 50, 0.5 * o ** 0.5, mq.EVEN, resid / 100, 0)
+                    x = 20 + s * len(offs) + j
+                    assert G.dev_diff(x, 50) < 10 * resid / o
+                    if j == 0:
+                        ref = G.dev_read(50, mq.EVEN)
+                        assert np.linalg.norm(dests[s][E] - ref[E]) < 10 * resid / o * np.linalg.norm(ref[E])

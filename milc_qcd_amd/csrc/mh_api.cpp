@@ -115,26 +115,13 @@ int refresh_links(int ext_prec, const void* fat, const void* lng, int* num_iters
   return 0;
 }
 
-// host MILC vector (float/double) -> device FP64 parity field
-int host_vec_in(int ext_prec, const void* h, VecField& v, int pb) {
-  Context& c = ctx();
-  if (ext_prec == 2) return upload_vec_milc((const double*)h, v, P_F64, pb);
-  std::vector<double> tmp((size_t)2 * c.Vh * 6, 0.0);
-  const float* f = (const float*)h;
-  size_t off = (size_t)pb * c.Vh * 6;
-  for (size_t i = 0; i < (size_t)c.Vh * 6; i++) tmp[off + i] = f[off + i];
-  return upload_vec_milc(tmp.data(), v, P_F64, pb);
+// host MILC vector (float/double) <-> device parity field (FP64 unless prec says otherwise)
+int host_vec_in(int ext_prec, const void* h, VecField& v, int pb, int prec = P_F64) {
+  return ext_prec == 2 ? upload_vec_milc((const double*)h, v, prec, pb)
+                       : upload_vec_milc_f32((const float*)h, v, prec, pb);
 }
-int host_vec_out(int ext_prec, const VecField& v, int pb, void* h) {
-  Context& c = ctx();
-  if (ext_prec == 2) return download_vec_milc(v, P_F64, pb, (double*)h);
-  std::vector<double> tmp((size_t)2 * c.Vh * 6, 0.0);
-  int rc = download_vec_milc(v, P_F64, pb, tmp.data());
-  if (rc) return rc;
-  float* f = (float*)h;
-  size_t off = (size_t)pb * c.Vh * 6;
-  for (size_t i = 0; i < (size_t)c.Vh * 6; i++) f[off + i] = (float)tmp[off + i];
-  return 0;
+int host_vec_out(int ext_prec, const VecField& v, int pb, void* h, int prec = P_F64) {
+  return ext_prec == 2 ? download_vec_milc(v, prec, pb, (double*)h) : download_vec_milc_f32(v, prec, pb, (float*)h);
 }
 
 int sloppy_of(int internal_precision, int mixed) {
@@ -262,19 +249,12 @@ int milc_hip_dslash(int external_precision, int internal_precision, milc_hip_inv
   int prec = internal_precision == 1 ? P_F32 : P_F64;
   if ((rc = ensure_links(prec))) return rc;
   int pb = pbit(parity);
-  VecField s, d, s64, d64;
-  VecScope owned{&s, &d, &s64, &d64};
-  if ((rc = alloc_vec(s64, P_F64, c.stride)) || (rc = alloc_vec(d64, P_F64, c.stride))) return rc;
-  if ((rc = host_vec_in(external_precision, src, s64, pb ^ 1))) return rc;
-  if (prec == P_F64) {
-    rc = dslash(c.links[P_F64], s64, d64, pb, P_F64);
-  } else {
-    if ((rc = alloc_vec(s, prec, c.stride)) || (rc = alloc_vec(d, prec, c.stride))) return rc;
-    if (!(rc = convert_vec(s64, P_F64, s, prec)) && !(rc = dslash(c.links[prec], s, d, pb, prec)))
-      rc = convert_vec(d, prec, d64, P_F64);
-  }
-  if (!rc) rc = host_vec_out(external_precision, d64, pb, dst);
-  return rc;
+  VecField s, d;
+  VecScope owned{&s, &d};
+  if ((rc = alloc_vec(s, prec, c.stride)) || (rc = alloc_vec(d, prec, c.stride)) ||
+      (rc = host_vec_in(external_precision, src, s, pb ^ 1, prec)) || (rc = dslash(c.links[prec], s, d, pb, prec)))
+    return rc;
+  return host_vec_out(external_precision, d, pb, dst, prec);
 }
 
 int milc_hip_dev_source(uint64_t seed, int parity, int slot) {

@@ -252,11 +252,12 @@ static inline int nblocks_for(int n, int block) { return (n + block - 1) / block
 // ===========================================================================
 // Layout kernels: MILC AoS (node_index order) <-> per-parity SoA planes
 // ===========================================================================
-template <int P>
-__global__ void k_vec_from_milc(const double* __restrict__ aos, VecField out, int Vh, int pb) {
+// H: the caller's real type (double, or float of a MILC_PRECISION 1 program)
+template <int P, typename H>
+__global__ void k_vec_from_milc(const H* __restrict__ aos, VecField out, int Vh, int pb) {
   int cb = blockIdx.x * blockDim.x + threadIdx.x;
   if (cb >= Vh) return;
-  const double* s = aos + 6 * ((size_t)pb * Vh + cb);
+  const H* s = aos + 6 * ((size_t)pb * Vh + cb);
   Vec3<typename PrecTraits<P>::Real> v;
 #pragma unroll
   for (int k = 0; k < 3; k++) {
@@ -265,17 +266,17 @@ __global__ void k_vec_from_milc(const double* __restrict__ aos, VecField out, in
   }
   store_vec<P>(out, cb, v);
 }
-template <int P>
-__global__ void k_vec_to_milc(VecField in, double* __restrict__ aos, int Vh, int pb) {
+template <int P, typename H>
+__global__ void k_vec_to_milc(VecField in, H* __restrict__ aos, int Vh, int pb) {
   int cb = blockIdx.x * blockDim.x + threadIdx.x;
   if (cb >= Vh) return;
   Vec3<typename PrecTraits<P>::Real> v;
   load_vec<P>(in, cb, v);
-  double* d = aos + 6 * ((size_t)pb * Vh + cb);
+  H* d = aos + 6 * ((size_t)pb * Vh + cb);
 #pragma unroll
   for (int k = 0; k < 3; k++) {
-    d[2 * k] = (double)v.c[k].re;
-    d[2 * k + 1] = (double)v.c[k].im;
+    d[2 * k] = (H)v.c[k].re;
+    d[2 * k + 1] = (H)v.c[k].im;
   }
 }
 
@@ -470,24 +471,31 @@ __global__ void k_convert_vec(VecField in, VecField out, int Vh) {
     else FN<P_H16>(__VA_ARGS__);                     \
   } while (0)
 
-template <int P>
-static void launch_vec_from_milc(const double* aos, VecField& out, int pb) {
+template <int P, typename H>
+static void launch_vec_from_milc(const H* aos, VecField& out, int pb) {
   Context& c = ctx();
-  hipLaunchKernelGGL(k_vec_from_milc<P>, dim3(nblocks_for(c.Vh, 256)), dim3(256), 0, c.stream, aos, out, c.Vh, pb);
+  hipLaunchKernelGGL((k_vec_from_milc<P, H>), dim3(nblocks_for(c.Vh, 256)), dim3(256), 0, c.stream, aos, out, c.Vh,
+                     pb);
 }
-template <int P>
-static void launch_vec_to_milc(const VecField& in, double* aos, int pb) {
+template <int P, typename H>
+static void launch_vec_to_milc(const VecField& in, H* aos, int pb) {
   Context& c = ctx();
-  hipLaunchKernelGGL(k_vec_to_milc<P>, dim3(nblocks_for(c.Vh, 256)), dim3(256), 0, c.stream, in, aos, c.Vh, pb);
+  hipLaunchKernelGGL((k_vec_to_milc<P, H>), dim3(nblocks_for(c.Vh, 256)), dim3(256), 0, c.stream, in, aos, c.Vh, pb);
 }
 
-int vec_from_milc_dev(const double* dev_aos, VecField& out, int prec, int pb) {
-  DISPATCH_PREC(prec, launch_vec_from_milc, dev_aos, out, pb);
+template <typename H>
+static int vec_from_milc_dev(const H* dev_aos, VecField& out, int prec, int pb) {
+  if (prec == P_F64) launch_vec_from_milc<P_F64, H>(dev_aos, out, pb);
+  else if (prec == P_F32) launch_vec_from_milc<P_F32, H>(dev_aos, out, pb);
+  else launch_vec_from_milc<P_H16, H>(dev_aos, out, pb);
   MH_CHECK(hipGetLastError());
   return 0;
 }
-int vec_to_milc_dev(const VecField& in, int prec, int pb, double* dev_aos) {
-  DISPATCH_PREC(prec, launch_vec_to_milc, in, dev_aos, pb);
+template <typename H>
+static int vec_to_milc_dev(const VecField& in, int prec, int pb, H* dev_aos) {
+  if (prec == P_F64) launch_vec_to_milc<P_F64, H>(in, dev_aos, pb);
+  else if (prec == P_F32) launch_vec_to_milc<P_F32, H>(in, dev_aos, pb);
+  else launch_vec_to_milc<P_H16, H>(in, dev_aos, pb);
   MH_CHECK(hipGetLastError());
   return 0;
 }
@@ -504,25 +512,40 @@ static int ensure_staging(size_t elems) {
   return 0;
 }
 
-int upload_vec_milc(const double* host_aos, VecField& out, int prec, int pb) {
+template <typename H>
+static int upload_vec(const H* host_aos, VecField& out, int prec, int pb) {
   Context& c = ctx();
   int rc = ensure_staging((size_t)2 * c.Vh * 6);
   if (rc) return rc;
   // only the parity half is needed
-  MH_CHECK(hipMemcpyAsync(c.staging + (size_t)pb * c.Vh * 6, host_aos + (size_t)pb * c.Vh * 6,
-                          (size_t)c.Vh * 6 * sizeof(double), hipMemcpyHostToDevice, c.stream));
-  return vec_from_milc_dev(c.staging, out, prec, pb);
+  H* stage = (H*)c.staging;
+  const size_t at = (size_t)pb * c.Vh * 6;
+  MH_CHECK(hipMemcpyAsync(stage + at, host_aos + at, (size_t)c.Vh * 6 * sizeof(H), hipMemcpyHostToDevice, c.stream));
+  return vec_from_milc_dev<H>(stage, out, prec, pb);
 }
-int download_vec_milc(const VecField& in, int prec, int pb, double* host_aos) {
+template <typename H>
+static int download_vec(const VecField& in, int prec, int pb, H* host_aos) {
   Context& c = ctx();
   int rc = ensure_staging((size_t)2 * c.Vh * 6);
   if (rc) return rc;
-  rc = vec_to_milc_dev(in, prec, pb, c.staging);
-  if (rc) return rc;
-  MH_CHECK(hipMemcpyAsync(host_aos + (size_t)pb * c.Vh * 6, c.staging + (size_t)pb * c.Vh * 6,
-                          (size_t)c.Vh * 6 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+  H* stage = (H*)c.staging;
+  const size_t at = (size_t)pb * c.Vh * 6;
+  if ((rc = vec_to_milc_dev<H>(in, prec, pb, stage))) return rc;
+  MH_CHECK(hipMemcpyAsync(host_aos + at, stage + at, (size_t)c.Vh * 6 * sizeof(H), hipMemcpyDeviceToHost, c.stream));
   MH_CHECK(hipStreamSynchronize(c.stream));
   return 0;
+}
+int upload_vec_milc(const double* host_aos, VecField& out, int prec, int pb) {
+  return upload_vec<double>(host_aos, out, prec, pb);
+}
+int download_vec_milc(const VecField& in, int prec, int pb, double* host_aos) {
+  return download_vec<double>(in, prec, pb, host_aos);
+}
+int upload_vec_milc_f32(const float* host_aos, VecField& out, int prec, int pb) {
+  return upload_vec<float>(host_aos, out, prec, pb);
+}
+int download_vec_milc_f32(const VecField& in, int prec, int pb, float* host_aos) {
+  return download_vec<float>(in, prec, pb, host_aos);
 }
 
 static int link_absmax_f64(const LinkField& f, double* out) {

@@ -157,8 +157,9 @@ size_t link_bytes(int prec, int stride);
 // ---- layout ----------------------------------------------------------------
 int upload_vec_milc(const double* host_aos, VecField& out, int prec, int pb);
 int download_vec_milc(const VecField& in, int prec, int pb, double* host_aos);
-int vec_from_milc_dev(const double* dev_aos, VecField& out, int prec, int pb);
-int vec_to_milc_dev(const VecField& in, int prec, int pb, double* dev_aos);
+// the same with MILC_PRECISION 1 host fields, converted on the device
+int upload_vec_milc_f32(const float* host_aos, VecField& out, int prec, int pb);
+int download_vec_milc_f32(const VecField& in, int prec, int pb, float* host_aos);
 int links_from_milc_dev(const double* dev_aos, LinkField& out, int prec);
 int links_to_milc_dev(const LinkField& in, int prec, double* dev_aos);
 int convert_links(const LinkField& in, int pin, LinkField& out, int pout);

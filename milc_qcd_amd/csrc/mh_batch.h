@@ -1,7 +1,7 @@
 // mh_batch.h -- many right-hand sides at once: batched colour-vector fields,
 // the batched fat + Naik stencil and the batched solvers built on it.
 //
-// Batched field of one parity, NR right-hand sides (NR = 2, 4, 8 or 16):
+// Batched field of one parity, NR right-hand sides (NR = 2, 4, 6, 8, 12 or 16):
 //   record (site cb, rhs r) = 6 reals  [re c0, re c1, re c2, im c0, im c1, im c2]
 //   at offset (cb * NR + r) * 6; R = float (F32) or double (F64);
 //   16-bit (P_H16): one int4 per record at cb * NR + r (mh_bkern.h).
@@ -21,7 +21,9 @@ namespace mh {
 // FP64 / 16-bit stencil for 2, 4, 8, 16: 96 / 181 / 57, 116 / 211 / 78,
 // 166 / 310 / 122, 281 / 539 / 212; the solves of a trajectory step pair with
 // two pseudofermions 285 ms in a batch of four, 220 in one of two).
-inline int batch_width(int n) { return n <= 2 ? 2 : (n <= 4 ? 4 : (n <= 8 ? 8 : 16)); }
+inline int batch_width(int n) {
+  return n <= 2 ? 2 : (n <= 4 ? 4 : (n <= 6 ? 6 : (n <= 8 ? 8 : (n <= 12 ? 12 : 16))));
+}
 #define BMS_MAX 32   // shifts per multi-shift solve
 #define BKW 8        // iterations per deferred shift-update window
 

@@ -412,16 +412,21 @@ struct BWork {
   double* partials = nullptr;
   float* W = nullptr;
   unsigned W_version = ~0u;
-  int tuned[3][4];      // [prec][nr index] -> variant, -1 untuned
-  double tuned_us[3][4];
+  int tuned[3][6];      // [prec][nr index] -> variant, -1 untuned
+  double tuned_us[3][6];
   BWork() {
     for (int a = 0; a < 3; a++)
-      for (int b = 0; b < 4; b++) tuned[a][b] = -1, tuned_us[a][b] = 0;
+      for (int b = 0; b < 6; b++) tuned[a][b] = -1, tuned_us[a][b] = 0;
   }
 };
 BWork g_bw;
 
-int nr_index(int nr) { return nr == 4 ? 0 : (nr == 8 ? 1 : (nr == 16 ? 2 : (nr == 2 ? 3 : -1))); }
+int nr_index(int nr) {
+  const int widths[] = {4, 8, 16, 2, 6, 12};
+  for (int i = 0; i < 6; i++)
+    if (nr == widths[i]) return i;
+  return -1;
+}
 
 // site-order block shapes offered to the tuner (index 0: checkerboard order)
 const int kOrders[4][4] = {{0, 0, 0, 0}, {8, 8, 8, 4}, {8, 4, 4, 4}, {4, 4, 4, 4}};
@@ -522,20 +527,17 @@ int launch_h16(const BDOp& op, int block, int loop_min, int order, int* nb_out) 
 
 template <int NR>
 int launch_h16_tps(const BDOp& op, const BVariant& v, int* nb) {
+#define MH_TPS(T)                                                                                     \
+  case T:                                                                                             \
+    if constexpr (NR % T == 0 && NR / T <= 8) return launch_h16<NR, T>(op, v.block, v.loop, v.order, nb); \
+    break
   switch (v.tps) {
-    case 1:
-      if constexpr (NR <= 8) return launch_h16<NR, 1>(op, v.block, v.loop, v.order, nb);
-      break;
-    case 2:
-      if constexpr (NR / 2 <= 8) return launch_h16<NR, 2>(op, v.block, v.loop, v.order, nb);
-      break;
-    case 4:
-      if constexpr (NR >= 4) return launch_h16<NR, 4>(op, v.block, v.loop, v.order, nb);
-      break;
-    case 8:
-      if constexpr (NR >= 8) return launch_h16<NR, 8>(op, v.block, v.loop, v.order, nb);
-      break;
+    MH_TPS(1);
+    MH_TPS(2);
+    MH_TPS(4);
+    MH_TPS(8);
   }
+#undef MH_TPS
   return -2;
 }
 
@@ -576,47 +578,53 @@ int launch_mfma(const BDOp& op, int block, int loop_min, int order, int* nb_out)
 template <int P, int NR>
 int launch_valu_tps(const BDOp& op, const BVariant& v, int* nb) {
   constexpr int RMAX = P == P_F64 ? 4 : 8;  // accumulators per thread (more spill)
+#define MH_TPS(T)                                                                                           \
+  case T:                                                                                                   \
+    if constexpr (NR % T == 0 && NR / T <= RMAX) return launch_valu<P, NR, T>(op, v.block, v.loop, v.order, nb); \
+    break
   switch (v.tps) {
-    case 1:
-      if constexpr (NR <= RMAX) return launch_valu<P, NR, 1>(op, v.block, v.loop, v.order, nb);
-      break;
-    case 2:
-      if constexpr (NR / 2 <= RMAX) return launch_valu<P, NR, 2>(op, v.block, v.loop, v.order, nb);
-      break;
-    case 4:
-      if constexpr (NR >= 4) return launch_valu<P, NR, 4>(op, v.block, v.loop, v.order, nb);
-      break;
-    case 8:
-      if constexpr (NR >= 8) return launch_valu<P, NR, 8>(op, v.block, v.loop, v.order, nb);
-      break;
+    MH_TPS(1);
+    MH_TPS(2);
+    MH_TPS(4);
+    MH_TPS(8);
   }
+#undef MH_TPS
   return -2;
 }
 
 int launch_variant(const BDOp& op, const BVariant& v, int* nb) {
-  if (op.prec == P_H16) {
-    if (v.mfma) return -2;
-    if (op.nr == 2) return launch_h16_tps<2>(op, v, nb);
-    if (op.nr == 4) return launch_h16_tps<4>(op, v, nb);
-    if (op.nr == 8) return launch_h16_tps<8>(op, v, nb);
-    return launch_h16_tps<16>(op, v, nb);
-  }
+#define MH_WIDTHS(CALL)      \
+  switch (op.nr) {           \
+    case 2: return CALL(2);   \
+    case 4: return CALL(4);   \
+    case 6: return CALL(6);   \
+    case 8: return CALL(8);   \
+    case 12: return CALL(12); \
+    case 16: return CALL(16); \
+  }                          \
+  return -2
+#define MH_H16(N) launch_h16_tps<N>(op, v, nb)
+#define MH_F64(N) launch_valu_tps<P_F64, N>(op, v, nb)
+#define MH_F32(N) launch_valu_tps<P_F32, N>(op, v, nb)
   if (v.mfma) {
-    if (op.prec != P_F32 || op.nr < 4) return -2;  // four columns to a block
+    // four columns to a block, whole sites to a wavefront
+    if (op.prec != P_F32) return -2;
     if (op.nr == 4) return launch_mfma<4>(op, v.block, v.loop, v.order, nb);
     if (op.nr == 8) return launch_mfma<8>(op, v.block, v.loop, v.order, nb);
-    return launch_mfma<16>(op, v.block, v.loop, v.order, nb);
+    if (op.nr == 16) return launch_mfma<16>(op, v.block, v.loop, v.order, nb);
+    return -2;
+  }
+  if (op.prec == P_H16) {
+    MH_WIDTHS(MH_H16);
   }
   if (op.prec == P_F64) {
-    if (op.nr == 2) return launch_valu_tps<P_F64, 2>(op, v, nb);
-    if (op.nr == 4) return launch_valu_tps<P_F64, 4>(op, v, nb);
-    if (op.nr == 8) return launch_valu_tps<P_F64, 8>(op, v, nb);
-    return launch_valu_tps<P_F64, 16>(op, v, nb);
+    MH_WIDTHS(MH_F64);
   }
-  if (op.nr == 2) return launch_valu_tps<P_F32, 2>(op, v, nb);
-  if (op.nr == 4) return launch_valu_tps<P_F32, 4>(op, v, nb);
-  if (op.nr == 8) return launch_valu_tps<P_F32, 8>(op, v, nb);
-  return launch_valu_tps<P_F32, 16>(op, v, nb);
+  MH_WIDTHS(MH_F32);
+#undef MH_WIDTHS
+#undef MH_H16
+#undef MH_F64
+#undef MH_F32
 }
 
 }  // namespace
@@ -642,14 +650,14 @@ std::vector<BVariant> bvariants(int prec, int nr) {
     if (order_of(k).on) orders.push_back(k);
   for (int order : orders)
     for (int tps : {1, 2, 4, 8}) {
-      if (tps > nr || nr / tps > rpt_max) continue;
+      if (nr % tps || nr / tps > rpt_max) continue;
       for (int block : {128, 256})
         for (int loop : {1, 2}) {
           if (order && loop > 1) continue;
           v.push_back(BVariant{0, tps, block, loop, order});
         }
     }
-  if (prec == P_F32 && nr >= 4)
+  if (prec == P_F32 && nr >= 4 && nr % 3)
     for (int order : orders)
       for (int block : {128, 256})
         for (int loop : {1, 2, 4}) {
@@ -777,17 +785,23 @@ int bpack(const VecField& in, void* batched, int prec, int nr, int r) {
   if (prec == P_H16) {
     if (nr == 2) hipLaunchKernelGGL((k_bpack_h16<2>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
     else if (nr == 4) hipLaunchKernelGGL((k_bpack_h16<4>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
+    else if (nr == 6) hipLaunchKernelGGL((k_bpack_h16<6>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bpack_h16<8>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
+    else if (nr == 12) hipLaunchKernelGGL((k_bpack_h16<12>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
     else hipLaunchKernelGGL((k_bpack_h16<16>), grid, dim3(256), 0, c.stream, in, (int4*)batched, r, c.Vh);
   } else if (prec == P_F64) {
     if (nr == 2) hipLaunchKernelGGL((k_bpack<double, 2>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
     else if (nr == 4) hipLaunchKernelGGL((k_bpack<double, 4>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
+    else if (nr == 6) hipLaunchKernelGGL((k_bpack<double, 6>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bpack<double, 8>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
+    else if (nr == 12) hipLaunchKernelGGL((k_bpack<double, 12>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
     else hipLaunchKernelGGL((k_bpack<double, 16>), grid, dim3(256), 0, c.stream, in, (double*)batched, r, c.Vh);
   } else {
     if (nr == 2) hipLaunchKernelGGL((k_bpack<float, 2>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
     else if (nr == 4) hipLaunchKernelGGL((k_bpack<float, 4>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
+    else if (nr == 6) hipLaunchKernelGGL((k_bpack<float, 6>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bpack<float, 8>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
+    else if (nr == 12) hipLaunchKernelGGL((k_bpack<float, 12>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
     else hipLaunchKernelGGL((k_bpack<float, 16>), grid, dim3(256), 0, c.stream, in, (float*)batched, r, c.Vh);
   }
   MH_CHECK(hipGetLastError());
@@ -800,17 +814,23 @@ int bunpack(const void* batched, int prec, int nr, int r, VecField& out) {
   if (prec == P_H16) {
     if (nr == 2) hipLaunchKernelGGL((k_bunpack_h16<2>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
     else if (nr == 4) hipLaunchKernelGGL((k_bunpack_h16<4>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
+    else if (nr == 6) hipLaunchKernelGGL((k_bunpack_h16<6>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bunpack_h16<8>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
+    else if (nr == 12) hipLaunchKernelGGL((k_bunpack_h16<12>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
     else hipLaunchKernelGGL((k_bunpack_h16<16>), grid, dim3(256), 0, c.stream, (const int4*)batched, r, out, c.Vh);
   } else if (prec == P_F64) {
     if (nr == 2) hipLaunchKernelGGL((k_bunpack<double, 2>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
     else if (nr == 4) hipLaunchKernelGGL((k_bunpack<double, 4>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
+    else if (nr == 6) hipLaunchKernelGGL((k_bunpack<double, 6>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bunpack<double, 8>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
+    else if (nr == 12) hipLaunchKernelGGL((k_bunpack<double, 12>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
     else hipLaunchKernelGGL((k_bunpack<double, 16>), grid, dim3(256), 0, c.stream, (const double*)batched, r, out, c.Vh);
   } else {
     if (nr == 2) hipLaunchKernelGGL((k_bunpack<float, 2>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
     else if (nr == 4) hipLaunchKernelGGL((k_bunpack<float, 4>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
+    else if (nr == 6) hipLaunchKernelGGL((k_bunpack<float, 6>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
     else if (nr == 8) hipLaunchKernelGGL((k_bunpack<float, 8>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
+    else if (nr == 12) hipLaunchKernelGGL((k_bunpack<float, 12>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
     else hipLaunchKernelGGL((k_bunpack<float, 16>), grid, dim3(256), 0, c.stream, (const float*)batched, r, out, c.Vh);
   }
   MH_CHECK(hipGetLastError());

@@ -200,10 +200,29 @@ __device__ __forceinline__ void bst_blk_h16(int4* __restrict__ f, int cb, int r0
   for (int i = 0; i < RPT; i++) a[i] = h16_pack(v[i]);
 }
 
-// Per-rhs block sums when rhs = lane % NR: written to LDS, then one value per
+// Threads per workgroup of the kernels over (site, rhs) records: a multiple of
+// the batch width, so that thread t of every workgroup has rhs t % NR.
+constexpr int rec_block(int nr) { return nr % 3 == 0 ? 192 : 256; }
+
+// Per-rhs block sums when rhs = thread % NR: written to LDS, then one value per
 // (dot, rhs) channel to partials[ch * pstride + blockIdx.x].
 template <int NV, int NR>
 __device__ __forceinline__ void bsum_lanes(double (&d)[NV], double* __restrict__ partials, int pstride) {
+  if constexpr (NR % 3 == 0) {
+    // a wavefront holds no whole number of sites: every thread's value goes to LDS
+    constexpr int B = rec_block(NR);
+    __shared__ double all[NV][B];
+#pragma unroll
+    for (int v = 0; v < NV; v++) all[v][threadIdx.x] = d[v];
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < NV * NR) {
+      double s = 0;
+      for (int k = 0; k < B / NR; k++) s += all[t / NR][t % NR + k * NR];
+      partials[(size_t)t * pstride + blockIdx.x] = s;
+    }
+    return;
+  }
 #pragma unroll
   for (int v = 0; v < NV; v++)
     for (int off = NR; off < 64; off <<= 1) d[v] += __shfl_xor(d[v], off, 64);

@@ -575,15 +575,15 @@ struct DevBuf {
   ~DevBuf() { dev_free(p); }
 };
 
-// grid of a (site, rhs)-record kernel: at most `cap` blocks of 256 threads
+// grid of a (site, rhs)-record kernel: at most `cap` blocks of `block` threads
 struct RecGrid {
   int nb, loop;
   long nrec;
 };
-RecGrid rec_grid(int nr, int cap) {
+RecGrid rec_grid(int nr, int cap, int block = 256) {
   RecGrid g;
   g.nrec = (long)ctx().Vh * nr;
-  long b1 = (g.nrec + 255) / 256;
+  long b1 = (g.nrec + block - 1) / block;
   g.loop = 1;
   while ((b1 + g.loop - 1) / g.loop > cap) g.loop *= 2;
   g.nb = (int)((b1 + g.loop - 1) / g.loop);
@@ -596,14 +596,16 @@ int bnorms(const void* f, int prec, int nr, double* sums_dev, double* out) {
   double* part;
   int ps, rc;
   if ((rc = bpartials(&part, &ps))) return rc;
-  RecGrid rg = rec_grid(nr, ps);
+  RecGrid rg = rec_grid(nr, ps, rec_block(nr));
 #define BN_CASE(R, N)                                                                                      \
-  hipLaunchKernelGGL((k_bnorm<R, N>), dim3(rg.nb), dim3(256), 0, c.stream, (const R*)f, rg.nrec, rg.loop, part, \
+  hipLaunchKernelGGL((k_bnorm<R, N>), dim3(rg.nb), dim3(rec_block(N)), 0, c.stream, (const R*)f, rg.nrec, rg.loop, part, \
                      ps)
   if (prec == P_F64) {
-    if (nr == 2) BN_CASE(double, 2); else if (nr == 4) BN_CASE(double, 4); else if (nr == 8) BN_CASE(double, 8); else BN_CASE(double, 16);
+    if (nr == 2) BN_CASE(double, 2); else if (nr == 4) BN_CASE(double, 4); else if (nr == 6) BN_CASE(double, 6);
+    else if (nr == 8) BN_CASE(double, 8); else if (nr == 12) BN_CASE(double, 12); else BN_CASE(double, 16);
   } else {
-    if (nr == 2) BN_CASE(float, 2); else if (nr == 4) BN_CASE(float, 4); else if (nr == 8) BN_CASE(float, 8); else BN_CASE(float, 16);
+    if (nr == 2) BN_CASE(float, 2); else if (nr == 4) BN_CASE(float, 4); else if (nr == 6) BN_CASE(float, 6);
+    else if (nr == 8) BN_CASE(float, 8); else if (nr == 12) BN_CASE(float, 12); else BN_CASE(float, 16);
   }
 #undef BN_CASE
   MH_CHECK(hipGetLastError());
@@ -634,7 +636,7 @@ int bmultishift_nr(const void* b64, const double* offs, int n, const double* res
   double* part;
   int pstride;
   if ((rc = bpartials(&part, &pstride))) return rc;
-  const RecGrid rg = rec_grid(NR, pstride);
+  const RecGrid rg = rec_grid(NR, pstride, rec_block(NR));
   // the flush walks float4 words: 6 NR / 4 of them per site
   const RecGrid rf = rec_grid(NR * 6 / 4, 2048);
   int variant;
@@ -732,11 +734,11 @@ int bmultishift_nr(const void* b64, const double* offs, int n, const double* res
       if ((r2 = bdslash(d2, &nb2))) return r2;
       if ((r2 = breduce(NR, nb2, dsum))) return r2;
       hipLaunchKernelGGL(k_bms_beta, dim3(1), dim3(kScalarThreads), 0, c.stream, dsum, ds, dg);
-      hipLaunchKernelGGL(k_bms_r<NR>, dim3(rg.nb), dim3(256), 0, c.stream, rprev, rcur, (const float*)ttt.p, ds, dg,
+      hipLaunchKernelGGL(k_bms_r<NR>, dim3(rg.nb), dim3(rec_block(NR)), 0, c.stream, rprev, rcur, (const float*)ttt.p, ds, dg,
                          rg.nrec, rg.loop, part, pstride);
       if ((r2 = breduce(NR, rg.nb, dsum + 32))) return r2;
       hipLaunchKernelGGL(k_bms_alpha, dim3(1), dim3(kScalarThreads), 0, c.stream, dsum + 32, ds, dg);
-      hipLaunchKernelGGL(k_bms_p<NR>, dim3(rg.nb), dim3(256), 0, c.stream, (float*)p.p, rcur, ds, dg, rg.nrec,
+      hipLaunchKernelGGL(k_bms_p<NR>, dim3(rg.nb), dim3(rec_block(NR)), 0, c.stream, (float*)p.p, rcur, ds, dg, rg.nrec,
                          rg.loop);
     }
     hipLaunchKernelGGL(k_bms_coef, dim3(1), dim3(256), 0, c.stream, ds, dg, (float*)dcoef.p, (int*)dmeta.p);
@@ -799,8 +801,8 @@ int btrue_residual(const void* b64, const void* x64, void* tmp64, void* t64, voi
   d2.p = x64;
   for (int r = 0; r < NR; r++) d2.coef[r] = -offsets[r];
   if ((rc = bdslash(d2, nullptr))) return rc;
-  RecGrid rg = rec_grid(NR, ps);
-  hipLaunchKernelGGL(k_bresid<NR>, dim3(rg.nb), dim3(256), 0, c.stream, (const double*)b64, (const double*)t64,
+  RecGrid rg = rec_grid(NR, ps, rec_block(NR));
+  hipLaunchKernelGGL(k_bresid<NR>, dim3(rg.nb), dim3(rec_block(NR)), 0, c.stream, (const double*)b64, (const double*)t64,
                      (double*)r64, rg.nrec, rg.loop, part, ps);
   MH_CHECK(hipGetLastError());
   if ((rc = breduce(NR, rg.nb, sums_dev))) return rc;
@@ -817,7 +819,7 @@ int bcg_mixed_nr(const void* b64, void* x64, const double* offsets, const BCGPar
   double* part;
   int pstride;
   if ((rc = bpartials(&part, &pstride))) return rc;
-  const RecGrid rg = rec_grid(NR, pstride);
+  const RecGrid rg = rec_grid(NR, pstride, rec_block(NR));
   const int sp = prm.sloppy == P_H16 ? P_H16 : P_F32;  // operator / search-direction precision
   if (sp == P_H16 && (rc = ensure_links(P_H16))) return rc;
   int vs, v64;
@@ -868,10 +870,10 @@ int bcg_mixed_nr(const void* b64, void* x64, const double* offsets, const BCGPar
       if ((r2 = breduce(3 * NR, nb2, dsum))) return r2;
       hipLaunchKernelGGL(k_bcg_scalars, dim3(1), dim3(64), 0, c.stream, dsum, dsum_rr, NR, ds, dg);
       if (sp == P_H16)
-        hipLaunchKernelGGL(k_bcg_update_h16<NR>, dim3(rg.nb), dim3(256), 0, c.stream, (float*)xs.p, (int4*)ps.p,
+        hipLaunchKernelGGL(k_bcg_update_h16<NR>, dim3(rg.nb), dim3(rec_block(NR)), 0, c.stream, (float*)xs.p, (int4*)ps.p,
                            (float*)rs.p, (const float*)ttts.p, ds, dg, rg.nrec, rg.loop, part, pstride);
       else
-        hipLaunchKernelGGL(k_bcg_update<NR>, dim3(rg.nb), dim3(256), 0, c.stream, (float*)xs.p, (float*)ps.p,
+        hipLaunchKernelGGL(k_bcg_update<NR>, dim3(rg.nb), dim3(rec_block(NR)), 0, c.stream, (float*)xs.p, (float*)ps.p,
                            (float*)rs.p, (const float*)ttts.p, ds, dg, rg.nrec, rg.loop, part, pstride);
       if ((r2 = breduce(NR, rg.nb, dsum_rr))) return r2;
     }
@@ -918,10 +920,10 @@ int bcg_mixed_nr(const void* b64, void* x64, const double* offsets, const BCGPar
     hg0.iter_cap = (int)std::min<long>(prm.max_iters - iteration, 1L << 30);
     if ((rc = (int)hipMemcpyAsync(dg, &hg0, sizeof(BCGG), hipMemcpyHostToDevice, c.stream))) break;
     if (sp == P_H16)
-      hipLaunchKernelGGL(k_bru_h16<NR>, dim3(rg.nb), dim3(256), 0, c.stream, (const double*)r64.p, (float*)rs.p,
+      hipLaunchKernelGGL(k_bru_h16<NR>, dim3(rg.nb), dim3(rec_block(NR)), 0, c.stream, (const double*)r64.p, (float*)rs.p,
                          (int4*)ps.p, ds, first ? 1 : 0, rg.nrec, rg.loop, part, pstride);
     else
-      hipLaunchKernelGGL(k_bru<NR>, dim3(rg.nb), dim3(256), 0, c.stream, (const double*)r64.p, (float*)rs.p,
+      hipLaunchKernelGGL(k_bru<NR>, dim3(rg.nb), dim3(rec_block(NR)), 0, c.stream, (const double*)r64.p, (float*)rs.p,
                          (float*)ps.p, ds, first ? 1 : 0, rg.nrec, rg.loop, part, pstride);
     if ((rc = (int)hipGetLastError())) break;
     if ((rc = breduce(NR, rg.nb, dsum_rr))) break;
@@ -953,6 +955,8 @@ int bmultishift_sets(const void* b64, int nr, int n, const double* offs, const d
   st = BMSStats();
   if (nr == 2) rc = bmultishift_nr<2>(b64, offs, n, stage_resid, prm, x64, st);
   else if (nr == 4) rc = bmultishift_nr<4>(b64, offs, n, stage_resid, prm, x64, st);
+  else if (nr == 6) rc = bmultishift_nr<6>(b64, offs, n, stage_resid, prm, x64, st);
+  else if (nr == 12) rc = bmultishift_nr<12>(b64, offs, n, stage_resid, prm, x64, st);
   else if (nr == 8) rc = bmultishift_nr<8>(b64, offs, n, stage_resid, prm, x64, st);
   else if (nr == 16) rc = bmultishift_nr<16>(b64, offs, n, stage_resid, prm, x64, st);
   else return -2;
@@ -1002,6 +1006,8 @@ int bcg_mixed(const void* b64, void* x64, int nr, const double* offsets, const B
   st = BCGStats();
   if (nr == 2) return bcg_mixed_nr<2>(b64, x64, offsets, prm, st);
   if (nr == 4) return bcg_mixed_nr<4>(b64, x64, offsets, prm, st);
+  if (nr == 6) return bcg_mixed_nr<6>(b64, x64, offsets, prm, st);
+  if (nr == 12) return bcg_mixed_nr<12>(b64, x64, offsets, prm, st);
   if (nr == 8) return bcg_mixed_nr<8>(b64, x64, offsets, prm, st);
   if (nr == 16) return bcg_mixed_nr<16>(b64, x64, offsets, prm, st);
   return -2;

@@ -258,10 +258,10 @@ def test_batched_solvers_stop_at_max_iters(l8):
 
 
 @pytest.mark.parametrize("dims", [(4, 4, 4, 4), (6, 4, 8, 6), (8, 6, 4, 10)])
-@pytest.mark.parametrize("nsrc,nshift", [(1, 1), (2, 1), (2, 12), (2, 32), (3, 31)])
-def test_multishift_block_narrow_batches_vs_oracle(dims, nsrc, nshift):
-    """Batches of two (one and two sources) and the next width up, with one
-    shift to the most: solutions against the oracle's multi-shift CG to 1e-13.
+@pytest.mark.parametrize("nsrc,nshift", [(1, 1), (2, 1), (2, 12), (2, 32), (3, 31), (7, 2), (9, 3), (12, 2)])
+def test_multishift_block_widths_vs_oracle(dims, nsrc, nshift):
+    """Batches of every width, full and with padding sources, with one shift to
+    the most: solutions against the oracle's multi-shift CG to 1e-13.
     A shift refined to the true residual r is off by r |b| / (offset |x|) at
     most, and |x| >= |b| / (offset + 10)."""
     L, fat, lng = hisq_setup(dims, 1007)

@@ -62,6 +62,25 @@ def test_mixed_cg_above_the_one_kernel_range():
 OFFSETS = [4 * 0.05 ** 2 + 1e-4 * 10 ** (4 * i / 11) for i in range(12)]
 
 
+# 206, 524 and 512 blocks of 256 sites in the update kernel: remainders over the
+# 8 XCDs with a last block of 8 and of 248 sites; an even split
+@pytest.mark.parametrize("dims", [(18, 18, 18, 18), (18, 18, 18, 46), (16, 16, 32, 32)])
+def test_update_kernel_block_order(dims):
+    """A block order that missed or repeated sites would leave the true residual,
+    which other kernels compute, above the target.  Two solutions lie within
+    the sum of their residuals times the condition number 1 / (4 m^2) (times 10)."""
+    mass, resid = 0.05, 1e-9
+    print(f"update kernel {dims}", flush=True)
+    with mq.Lattice(dims) as G:
+        G.dev_gauge_hisq(1404)
+        G.dev_source(1405, mq.EVEN, 0)
+        G.dev_invert(0, 1, mass, mq.EVEN, resid, 0)
+        for mixed in (1, 2):
+            _, st = G.dev_invert(0, 2, mass, mq.EVEN, resid, mixed)
+            assert st["converged"] and st["resid"] < resid
+            assert G.dev_diff(2, 1) < 10 * 2 * resid / (4 * mass ** 2)
+
+
 @pytest.mark.parametrize("dims", SIZES)
 @pytest.mark.parametrize("mixed", [0, 1])
 def test_multishift_one_kernel(dims, mixed):

@@ -453,7 +453,7 @@ int milc_hip_dev_block_dslash(int prec, int nrhs, int variant, int nsrc, const i
                               const int* dst_slots);
 /* Batched multi-shift on device slots (see milc_hip_multishift_invert_block);
  * solutions of the first out_nsrc sources to slots out_slot0 + s * num_offsets + j
- * when out_slot0 >= 0.
+ * when out_slot0 >= 0; these may be slots of sources, which are all read first.
  * stats[0..5] = multi-shift iterations, multi-shift seconds, refinement
  * seconds, converged, stencil variant, its time (us; -1 and 0 where the sources
  * of a small lattice were solved one after another in FP64); stats[6 + j] = max true

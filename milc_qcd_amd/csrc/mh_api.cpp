@@ -1029,6 +1029,16 @@ int ensure_slot(int s) {
   if (!g_slots[s].data) return alloc_vec(g_slots[s], P_F64, c.stride);
   return 0;
 }
+
+// n FP64 fields, freed with `owned`
+int alloc_fields(std::vector<VecField>& f, int n, VecScope& owned) {
+  f.assign(n, VecField{});
+  for (auto& v : f) {
+    owned.add(&v);
+    if (int rc = alloc_vec(v, P_F64, ctx().stride)) return rc;
+  }
+  return 0;
+}
 }  // namespace
 
 extern "C" int milc_hip_dev_dslash(int prec, int slot_src, int parity_out, int slot_dst) {
@@ -1151,28 +1161,28 @@ extern "C" int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int
     std::vector<double> worst(num_offsets, 0.0);
     long most = 0;
     int conv = 1;
+    // every source is read before a solution is written, as in the batch: the
+    // slots may overlap
+    const int kept = out_slot0 >= 0 ? out_nsrc : 0;
+    std::vector<std::vector<VecField>> xs(kept + (kept < nsrc ? 1 : 0));
+    VecScope owned;
+    for (auto& x : xs)
+      if ((rc = alloc_fields(x, num_offsets, owned))) return rc;
     for (int s = 0; s < nsrc; s++) {
-      std::vector<VecField> xs(num_offsets);
-      VecScope owned;
-      for (auto& v : xs) {
-        owned.add(&v);
-        if ((rc = alloc_vec(v, P_F64, c.stride))) return rc;
-      }
       long it = 0;
       int ok = 1;
-      if ((rc = multishift_small(g_slots[src_slots[s]], xs, offs, res.data(), parity, max_iters > 0 ? max_iters : 20000,
-                                 &it, rel.data(), &ok)))
+      if ((rc = multishift_small(g_slots[src_slots[s]], xs[std::min(s, kept)], offs, res.data(), parity,
+                                 max_iters > 0 ? max_iters : 20000, &it, rel.data(), &ok)))
         return rc;
       most = std::max(most, it);
       conv &= ok;
-      for (int j = 0; j < num_offsets; j++) {
-        worst[j] = std::max(worst[j], rel[j]);
-        const int slot = out_slot0 + s * num_offsets + j;
-        if (out_slot0 >= 0 && s < out_nsrc &&
-            ((rc = ensure_slot(slot)) || (rc = vec_copy(xs[j], g_slots[slot], P_F64))))
-          return rc;
-      }
+      for (int j = 0; j < num_offsets; j++) worst[j] = std::max(worst[j], rel[j]);
     }
+    for (int s = 0; s < kept; s++)
+      for (int j = 0; j < num_offsets; j++) {
+        const int slot = out_slot0 + s * num_offsets + j;
+        if ((rc = ensure_slot(slot)) || (rc = vec_copy(xs[s][j], g_slots[slot], P_F64))) return rc;
+      }
     MH_CHECK(hipStreamSynchronize(c.stream));
     if (stats) {
       stats[0] = most;
@@ -1255,28 +1265,27 @@ extern "C" int milc_hip_multishift_invert_block(int external_precision, int nsrc
   for (int j = 0; j < num_offsets; j++) positive = positive && offsets[j] > 0;
   if (refine_residual > 0 && positive && args.max_iter != 1 && block_is_small(nsrc)) {
     std::vector<double> offs(offsets, offsets + num_offsets), res(num_offsets, refine_residual), rel(num_offsets);
-    VecField v;
-    std::vector<VecField> xs(num_offsets);
-    VecScope owned{&v};
-    if ((rc = alloc_vec(v, P_F64, c.stride))) return rc;
-    for (auto& f : xs) {
-      owned.add(&f);
-      if ((rc = alloc_vec(f, P_F64, c.stride))) return rc;
-    }
+    // every source is read before a solution is written, as in the batch: the
+    // arrays may be the same
+    std::vector<VecField> b;
+    std::vector<std::vector<VecField>> xs(nsrc);
+    VecScope owned;
+    if ((rc = alloc_fields(b, nsrc, owned))) return rc;
+    for (int s = 0; s < nsrc; s++)
+      if ((rc = alloc_fields(xs[s], num_offsets, owned)) || (rc = host_vec_in(external_precision, source[s], b[s], pb)))
+        return rc;
     for (int s = 0; s < nsrc; s++) {
       long it = 0;
       int ok = 1;
-      if ((rc = host_vec_in(external_precision, source[s], v, pb)) ||
-          (rc = multishift_small(v, xs, offs, res.data(), parity, args.max_iter > 0 ? args.max_iter : 20000, &it,
+      if ((rc = multishift_small(b[s], xs[s], offs, res.data(), parity, args.max_iter > 0 ? args.max_iter : 20000, &it,
                                  rel.data(), &ok)))
         return rc;
-      for (int j = 0; j < num_offsets; j++) {
-        const size_t k = (size_t)s * num_offsets + j;
-        if ((rc = host_vec_out(external_precision, xs[j], pb, solution[k]))) return rc;
-        if (final_residual) final_residual[k] = rel[j];
-      }
+      if (final_residual) std::copy(rel.begin(), rel.end(), final_residual + (size_t)s * num_offsets);
       total = std::max(total, (int)it);
     }
+    for (int s = 0; s < nsrc; s++)
+      for (int j = 0; j < num_offsets; j++)
+        if ((rc = host_vec_out(external_precision, xs[s][j], pb, solution[(size_t)s * num_offsets + j]))) return rc;
     if (num_iters) *num_iters = total;
     return total;
   }
@@ -1353,19 +1362,23 @@ extern "C" int milc_hip_invert_block(int external_precision, int nsrc, double ma
     sp.sloppy_prec = P_F64;
     sp.delta = kReliableDelta;
     sp.batch = 16;
-    VecField b, x;
-    VecScope owned{&b, &x};
-    if ((rc = alloc_vec(b, P_F64, c.stride)) || (rc = alloc_vec(x, P_F64, c.stride))) return rc;
+    // every source and initial guess (t_dest, d_congrad5_fn_gpu.c:104-110) is
+    // read before a solution is written, as in the batch: the arrays may be the same
+    std::vector<VecField> b, x;
+    VecScope owned;
+    if ((rc = alloc_fields(b, nsrc, owned)) || (rc = alloc_fields(x, nsrc, owned))) return rc;
+    for (int s = 0; s < nsrc; s++)
+      if ((rc = host_vec_in(external_precision, source[s], b[s], pb)) ||
+          (rc = host_vec_in(external_precision, solution[s], x[s], pb)))
+        return rc;
     for (int s = 0; s < nsrc; s++) {
       SolveStats st;
-      // t_dest is the initial guess (d_congrad5_fn_gpu.c:104-110)
-      if ((rc = host_vec_in(external_precision, source[s], b, pb)) ||
-          (rc = host_vec_in(external_precision, solution[s], x, pb)) || (rc = cg_solve_restarting(b, x, mass, sp, st)) ||
-          (rc = host_vec_out(external_precision, x, pb, solution[s])))
-        return rc;
+      if ((rc = cg_solve_restarting(b[s], x[s], mass, sp, st))) return rc;
       if (final_residual) final_residual[s] = std::sqrt(st.final_rsq);
       total = std::max(total, st.iters);
     }
+    for (int s = 0; s < nsrc; s++)
+      if ((rc = host_vec_out(external_precision, x[s], pb, solution[s]))) return rc;
     if (num_iters) *num_iters = total;
     return total;
   }

@@ -8,6 +8,8 @@ condition number of the operator, 1 / (4 m^2) (times 10); everywhere its true
 residual, which other kernels compute, has to meet the target.  A mixed solve
 on a lattice above the one-kernel range of the mixed CG still goes through the
 sloppy iterations."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -159,3 +161,57 @@ def test_block_calls_on_both_sides_of_the_dispatch(dims, nsrc):
                     if j == 0:
                         ref = G.dev_read(63, mq.EVEN)
                         assert np.linalg.norm(dests[s][E] - ref[E]) < 10 * resid / o * np.linalg.norm(ref[E])
+
+
+@pytest.mark.parametrize("nsrc", [2, 7])
+def test_block_multishift_slots_may_overlap(nsrc):
+    """Solutions over slots of the sources, one source after another (2) and as
+    a batch (7): every source is read before a solution is written, so the
+    solutions are bit for bit those of separate slots."""
+    offs = [0.04, 0.3]
+    with mq.Lattice((6, 4, 8, 6)) as G:
+        G.dev_gauge_hisq(1420)
+        for first in (0, 1):  # solutions from slot `first` on
+            for s in range(nsrc):
+                G.dev_source(1421 + s, mq.EVEN, s)
+            src = list(range(nsrc))
+            G.dev_multishift_block(src, offs, 1e-7, 1e-9, out_slot0=40)
+            G.dev_multishift_block(src, offs, 1e-7, 1e-9, out_slot0=first)
+            for k in range(nsrc * len(offs)):
+                assert G.dev_diff(first + k, 40 + k) == 0.0, (first, k)
+
+
+@pytest.mark.parametrize("nsrc", [2, 7])
+def test_block_calls_on_aliased_host_arrays(nsrc):
+    """The same for host arrays: solution s in the array of source s + 1 (which is
+    then also the CG's initial guess)."""
+    dims, mass = (6, 4, 8, 6), 0.1
+    offs = [4 * mass ** 2, 0.3]
+    with mq.Lattice(dims) as G:
+        G.dev_gauge_hisq(1430)
+        G.set_links(*G.dev_read_links())
+        srcs = []
+        for s in range(nsrc):
+            G.dev_source(1431 + s, mq.EVEN, 0)
+            srcs.append(G.dev_read(0, mq.EVEN))
+        qic = mq.QuarkInvertControl(max=3000, nrestart=1, parity=mq.EVEN, resid=1e-9)
+        ref = [srcs[(s + 1) % nsrc].copy() for s in range(nsrc)]
+        G.ks_congrad_block_parity([v.copy() for v in srcs], ref, qic, mass)
+        a = [v.copy() for v in srcs]
+        G.ks_congrad_block_parity(a, [a[(s + 1) % nsrc] for s in range(nsrc)], qic, mass)
+        for s in range(nsrc):
+            assert np.array_equal(a[(s + 1) % nsrc], ref[s]), s
+
+        ref = G.ks_multicg_offset_block(srcs, offs, mq.EVEN, 1e-7, 1e-9)[0]
+        a = [v.copy() for v in srcs]
+        x = [[a[(s + 1) % nsrc], np.zeros_like(a[0])] for s in range(nsrc)]
+        ptr = lambda fields: (ctypes.c_void_p * len(fields))(*[f.ctypes.data for f in fields])
+        rc = G.lib.milc_hip_multishift_invert_block(
+            2, nsrc, 2, (ctypes.c_double * 2)(*offs), mq.ks.InvArgs(3000, 0, 1, 0.0, 1.0, 0), (ctypes.c_double * 1)(1e-7),
+            1e-9, G.fat.ctypes.data, G.lng.ctypes.data, ptr(a), ptr([f for xs in x for f in xs]),
+            (ctypes.c_double * (2 * nsrc))(), ctypes.byref(ctypes.c_int(0)))
+        assert rc > 0
+        E = G.parity_slice(mq.EVEN)
+        for s in range(nsrc):
+            for j in range(2):
+                assert np.array_equal(x[s][j][E], ref[s][j][E]), (s, j)

@@ -599,8 +599,9 @@ extern "C" int milc_hip_multishift_invert(int external_precision, int internal_p
   if (rc) return rc;
   int pb = pbit(parity);
   bool mixed = args.mixed_precision != 0;
-  bool small = mixed && multishift_is_small() && args.max_iter != 1;
-  for (int j = 0; j < num_offsets; j++) small = small && (target_resid[j] > 0 ? target_resid[j] : target_resid[0]) > 0;
+  std::vector<double> res(num_offsets);
+  for (int j = 0; j < num_offsets; j++) res[j] = target_resid[j] > 0 ? target_resid[j] : target_resid[0];
+  const bool small = mixed && args.max_iter != 1 && multishift_is_small() && multishift_small_takes(res);
   int bulk = (internal_precision == 1 || mixed) ? P_F32 : P_F64;
   if (!small && (rc = ensure_links(bulk))) return rc;
   VecField b;
@@ -621,8 +622,7 @@ extern "C" int milc_hip_multishift_invert(int external_precision, int internal_p
   mp.prec = bulk;
   mp.batch = 16;
   SolveStats st;
-  std::vector<double> fres(num_offsets, 0.0), res(num_offsets);
-  for (int j = 0; j < num_offsets; j++) res[j] = target_resid[j] > 0 ? target_resid[j] : target_resid[0];
+  std::vector<double> fres(num_offsets, 0.0);
   long it = 0;
   int conv = 1;
   if (small) {
@@ -1153,11 +1153,12 @@ extern "C" int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int
     if (!slot_ok(src_slots[s], true)) return -2;
   if (out_slot0 >= 0 && (out_nsrc < 0 || out_nsrc > nsrc || out_slot0 + out_nsrc * num_offsets > kSlots)) return -2;
   int rc;
-  if (refine_resid > 0 && max_iters != 1 && block_is_small(nsrc)) {
+  const std::vector<double> res(num_offsets, refine_resid);
+  if (refine_resid > 0 && max_iters != 1 && block_is_small(nsrc) && multishift_small_takes(res)) {
     for (int j = 0; j < num_offsets; j++)
       if (!(offsets[j] > 0)) return -2;
     auto t0 = std::chrono::steady_clock::now();
-    std::vector<double> offs(offsets, offsets + num_offsets), res(num_offsets, refine_resid), rel(num_offsets);
+    std::vector<double> offs(offsets, offsets + num_offsets), rel(num_offsets);
     std::vector<double> worst(num_offsets, 0.0);
     long most = 0;
     int conv = 1;
@@ -1263,8 +1264,9 @@ extern "C" int milc_hip_multishift_invert_block(int external_precision, int nsrc
   int total = 0;
   bool positive = true;
   for (int j = 0; j < num_offsets; j++) positive = positive && offsets[j] > 0;
-  if (refine_residual > 0 && positive && args.max_iter != 1 && block_is_small(nsrc)) {
-    std::vector<double> offs(offsets, offsets + num_offsets), res(num_offsets, refine_residual), rel(num_offsets);
+  const std::vector<double> res(num_offsets, refine_residual);
+  if (refine_residual > 0 && positive && args.max_iter != 1 && block_is_small(nsrc) && multishift_small_takes(res)) {
+    std::vector<double> offs(offsets, offsets + num_offsets), rel(num_offsets);
     // every source is read before a solution is written, as in the batch: the
     // arrays may be the same
     std::vector<VecField> b;
@@ -1352,7 +1354,9 @@ extern "C" int milc_hip_invert_block(int external_precision, int nsrc, double ma
   if ((rc = refresh_links(external_precision, fatlink, longlink, num_iters))) return rc;
   const int pb = pbit(parity);
   int total = 0;
-  if (block_is_small(nsrc)) {
+  // a target that is never met runs to max_iter as a batch (the one-source solve
+  // takes one whose square is zero for no target at all)
+  if (std::abs(target_residual) > kNoTarget && block_is_small(nsrc)) {
     SolveParams sp;
     sp.parity = parity;
     sp.max_iters = args.max_iter > 0 ? args.max_iter : 20000;

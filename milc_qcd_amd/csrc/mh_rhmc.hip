@@ -101,8 +101,8 @@ static int rational_solve(const VecField& phi, int n, const double* offsets, dou
   for (int t = 0; t < n; t++)
     if ((rc = alloc_vec(x[t], P_F64, c.stride))) return rc;
   std::vector<double> offs(offsets, offsets + n);
-  if (mixed && resid > 0 && multishift_is_small()) {
-    std::vector<double> res(n, resid);
+  const std::vector<double> res(n, resid);
+  if (mixed && multishift_is_small() && multishift_small_takes(res)) {
     long it = 0;
     if ((rc = multishift_small(phi, x, offs, res.data(), parity, 20000, &it, nullptr, &st.converged))) return rc;
     st.iters = (int)it;
@@ -121,7 +121,6 @@ static int rational_solve(const VecField& phi, int n, const double* offsets, dou
   // Refinement of every shift to the FP64 true-residual target from the
   // multi-shift solution: 16-bit sloppy operator, FP64 reliable updates, up to
   // four shifts per batched CG.
-  std::vector<double> res(n, resid);
   long it = 0;
   if ((rc = refine_shifts(phi, x, offs.data(), res.data(), parity, 20000, P_H16, &it, nullptr, &st.converged)))
     return rc;
@@ -143,7 +142,7 @@ static int rational_solve_all(const std::vector<const VecField*>& src, const std
     if (o.empty() || (int)o.size() > BMS_MAX) return -2;
     n = std::max(n, (int)o.size());
   }
-  if (multishift_is_small(ns) && *std::min_element(resid.begin(), resid.end()) > 0) {
+  if (multishift_is_small(ns) && multishift_small_takes(resid)) {
     // one source after another: no padding sources, no refinement
     x.assign(ns, {});
     long it = 0;

@@ -215,3 +215,28 @@ def test_block_calls_on_aliased_host_arrays(nsrc):
         for s in range(nsrc):
             for j in range(2):
                 assert np.array_equal(x[s][j][E], ref[s][j][E]), (s, j)
+
+
+@pytest.mark.parametrize("nsrc", [2, 7])
+def test_block_calls_without_a_target_run_to_the_cap(nsrc):
+    """A target whose square is zero is never met: max_iter iterations and no
+    convergence, on either side of the dispatch."""
+    with mq.Lattice((6, 4, 8, 6)) as G:
+        G.dev_gauge_hisq(1440)
+        G.set_links(*G.dev_read_links())
+        for s in range(nsrc):
+            G.dev_source(1441 + s, mq.EVEN, s)
+        src = G.dev_read(0, mq.EVEN)
+        for resid in (0.0, 1e-170):
+            qic = mq.QuarkInvertControl(max=24, nrestart=1, parity=mq.EVEN, resid=resid)
+            dests = [np.zeros_like(src) for _ in range(nsrc)]
+            it, res = G.ks_congrad_block_parity([src] * nsrc, dests, qic, 0.1)
+            assert 24 <= it <= 25 and qic.converged == 0
+            assert 0 < max(res) < 1e-2
+        st = G.dev_multishift_block(list(range(nsrc)), [0.04, 0.5], 1e-6, 1e-170, max_iters=60, out_slot0=20)
+        assert st["converged"] == 0 and 0 < max(st["true_rel"]) < 1e-9
+        if nsrc == 2:
+            _, _, conv = G.dev_multishift(0, [0.04, 0.5], 1e-170, 1, out_slot0=20)
+            assert not conv
+            G.dev_invert(0, 30, 0.1, mq.EVEN, 1e-12, 0)
+            assert G.dev_diff(20, 30) < 1e-9

@@ -601,7 +601,8 @@ extern "C" int milc_hip_multishift_invert(int external_precision, int internal_p
   bool mixed = args.mixed_precision != 0;
   std::vector<double> res(num_offsets);
   for (int j = 0; j < num_offsets; j++) res[j] = target_resid[j] > 0 ? target_resid[j] : target_resid[0];
-  const bool small = mixed && args.max_iter != 1 && multishift_is_small() && multishift_small_takes(res);
+  const std::vector<double> offs(offsets, offsets + num_offsets);
+  const bool small = mixed && args.max_iter != 1 && multishift_is_small() && multishift_small_takes(offs, res);
   int bulk = (internal_precision == 1 || mixed) ? P_F32 : P_F64;
   if (!small && (rc = ensure_links(bulk))) return rc;
   VecField b;
@@ -612,7 +613,6 @@ extern "C" int milc_hip_multishift_invert(int external_precision, int internal_p
   for (auto& v : xs)
     if ((rc = alloc_vec(v, P_F64, c.stride))) return rc;
   if ((rc = host_vec_in(external_precision, source, b, pb))) return rc;
-  std::vector<double> offs(offsets, offsets + num_offsets);
   MultiParams mp;
   mp.parity = parity;
   mp.max_iters = args.max_iter > 0 ? args.max_iter : 1000;
@@ -1153,13 +1153,10 @@ extern "C" int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int
     if (!slot_ok(src_slots[s], true)) return -2;
   if (out_slot0 >= 0 && (out_nsrc < 0 || out_nsrc > nsrc || out_slot0 + out_nsrc * num_offsets > kSlots)) return -2;
   int rc;
-  const std::vector<double> res(num_offsets, refine_resid);
-  if (refine_resid > 0 && max_iters != 1 && block_is_small(nsrc) && multishift_small_takes(res)) {
-    for (int j = 0; j < num_offsets; j++)
-      if (!(offsets[j] > 0)) return -2;
+  const std::vector<double> offs(offsets, offsets + num_offsets), res(num_offsets, refine_resid);
+  if (refine_resid > 0 && max_iters != 1 && block_is_small(nsrc) && multishift_small_takes(offs, res)) {
     auto t0 = std::chrono::steady_clock::now();
-    std::vector<double> offs(offsets, offsets + num_offsets), rel(num_offsets);
-    std::vector<double> worst(num_offsets, 0.0);
+    std::vector<double> rel(num_offsets), worst(num_offsets, 0.0);
     long most = 0;
     int conv = 1;
     // every source is read before a solution is written, as in the batch: the
@@ -1218,7 +1215,6 @@ extern "C" int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int
   prm.refine_resid = refine_resid;
   prm.delta = kBatchReliableDelta;
   BMSStats st;
-  std::vector<double> offs(offsets, offsets + num_offsets);
   if ((rc = bmultishift(b.p, nr, offs, prm, xp, st))) return rc;
   if (out_slot0 >= 0) {
     for (int s = 0; s < out_nsrc; s++)
@@ -1262,11 +1258,9 @@ extern "C" int milc_hip_multishift_invert_block(int external_precision, int nsrc
   if ((rc = refresh_links(external_precision, fatlink, longlink, num_iters))) return rc;
   const int pb = pbit(parity);
   int total = 0;
-  bool positive = true;
-  for (int j = 0; j < num_offsets; j++) positive = positive && offsets[j] > 0;
-  const std::vector<double> res(num_offsets, refine_residual);
-  if (refine_residual > 0 && positive && args.max_iter != 1 && block_is_small(nsrc) && multishift_small_takes(res)) {
-    std::vector<double> offs(offsets, offsets + num_offsets), rel(num_offsets);
+  const std::vector<double> offs(offsets, offsets + num_offsets), res(num_offsets, refine_residual);
+  if (refine_residual > 0 && args.max_iter != 1 && block_is_small(nsrc) && multishift_small_takes(offs, res)) {
+    std::vector<double> rel(num_offsets);
     // every source is read before a solution is written, as in the batch: the
     // arrays may be the same
     std::vector<VecField> b;
@@ -1318,7 +1312,6 @@ extern "C" int milc_hip_multishift_invert_block(int external_precision, int nsrc
     prm.refine_resid = refine_residual;
     prm.delta = kBatchReliableDelta;
     BMSStats st;
-    std::vector<double> offs(offsets, offsets + num_offsets);
     if ((rc = bmultishift(b.p, nr, offs, prm, xp, st))) {
       free_vec(v);
       return rc;

@@ -229,11 +229,12 @@ int multicg_solve(const VecField& src, std::vector<VecField>& x, const std::vect
                   const MultiParams& mp, SolveStats& st);
 // Whether the mixed multi-shifts of `sources` sources run as multishift_small.
 bool multishift_is_small(int sources = 1);
-// ... and whether their targets allow it: a target whose square times |b|^2 may
+// ... and whether their shifts allow it.  A target whose square times |b|^2 may
 // be zero is never met, which the recurrence of the one-kernel solve does not
-// survive.
+// survive.  A shift that misses its target is finished by a CG of mass
+// sqrt(offset) / 2; the batched refinement takes any offset.
 constexpr double kNoTarget = 1e-100;
-bool multishift_small_takes(const std::vector<double>& resid);
+bool multishift_small_takes(const std::vector<double>& offsets, const std::vector<double>& resid);
 // Multi-shift of a small lattice to each shift's own FP64 true residual
 // target resid[j] (what the FP32 stage and refine_shifts do on larger ones):
 // FP64 in one kernel, every true residual checked, a shift that misses its

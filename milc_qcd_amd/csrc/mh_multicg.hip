@@ -493,7 +493,9 @@ bool multishift_is_small(int sources) {
   return ctx().Vh <= persist_mixed_shift_sites(sources) && persist_shape(ctx().Vh).lps && ctx().links[P_F64].valid;
 }
 
-bool multishift_small_takes(const std::vector<double>& resid) {
+bool multishift_small_takes(const std::vector<double>& offsets, const std::vector<double>& resid) {
+  for (double o : offsets)
+    if (!(o > 0)) return false;
   for (double r : resid)
     if (!(r > kNoTarget)) return false;
   return true;

@@ -240,3 +240,15 @@ def test_block_calls_without_a_target_run_to_the_cap(nsrc):
             assert not conv
             G.dev_invert(0, 30, 0.1, mq.EVEN, 1e-12, 0)
             assert G.dev_diff(20, 30) < 1e-9
+
+
+@pytest.mark.parametrize("nsrc", [2, 7])
+def test_block_multishift_takes_an_offset_of_zero(nsrc):
+    """(-D D) x = b, offset 0, is a positive system too: accepted on either side
+    of the dispatch."""
+    with mq.Lattice((4, 4, 4, 4)) as G:
+        G.dev_gauge_hisq(1450)
+        for s in range(nsrc):
+            G.dev_source(1451 + s, mq.EVEN, s)
+        st = G.dev_multishift_block(list(range(nsrc)), [0.0, 0.5], 1e-6, 1e-9, out_slot0=20)
+        assert st["converged"] and max(st["true_rel"]) < 1e-9

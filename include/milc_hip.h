@@ -339,7 +339,9 @@ int milc_hip_invert_block(int external_precision, int nsrc, double mass, milc_hi
  * runs to target_residual[0] in FP32 with FP64 recurrences; refine_residual > 0
  * then refines every shift to that FP64 true residual (mixed-precision CG,
  * the per-shift refinement of ks_multicg_hybrid_field, ks_multicg.c:170-236).
- * final_residual[s * num_offsets + j] gets the true residuals (after refinement). */
+ * final_residual[s * num_offsets + j] gets the true residuals (after refinement).
+ * Returns the iterations of the multi-shift plus those of every shift's
+ * refinement, each of the source that needs the most. */
 int milc_hip_multishift_invert_block(int external_precision, int nsrc, int num_offsets, const double* offsets,
                                      milc_hip_inv_args args, const double* target_residual, double refine_residual,
                                      const void* fatlink, const void* longlink, void* const* source,

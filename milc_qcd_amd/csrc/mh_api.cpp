@@ -1030,6 +1030,22 @@ int ensure_slot(int s) {
   return 0;
 }
 
+// Iterations of the multi-shifts of one source after another, counted as a
+// batch counts them: those of the source that needs the most, stage and
+// refinement of each shift apart.
+struct BlockCounts {
+  std::vector<int> one, refine;  // refinement of the source at hand, of all so far
+  int stage = 0;
+  explicit BlockCounts(int shifts) : one(shifts, 0), refine(shifts, 0) {}
+  void add(long iters) {
+    for (size_t j = 0; j < one.size(); j++) {
+      iters -= one[j];
+      refine[j] = std::max(refine[j], one[j]);
+    }
+    stage = std::max(stage, (int)iters);
+  }
+};
+
 // n FP64 fields, freed with `owned`
 int alloc_fields(std::vector<VecField>& f, int n, VecScope& owned) {
   f.assign(n, VecField{});
@@ -1157,7 +1173,7 @@ extern "C" int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int
   if (refine_resid > 0 && max_iters != 1 && block_is_small(nsrc) && multishift_small_takes(offs, res)) {
     auto t0 = std::chrono::steady_clock::now();
     std::vector<double> rel(num_offsets), worst(num_offsets, 0.0);
-    long most = 0;
+    BlockCounts counts(num_offsets);
     int conv = 1;
     // every source is read before a solution is written, as in the batch: the
     // slots may overlap
@@ -1170,9 +1186,9 @@ extern "C" int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int
       long it = 0;
       int ok = 1;
       if ((rc = multishift_small(g_slots[src_slots[s]], xs[std::min(s, kept)], offs, res.data(), parity,
-                                 max_iters > 0 ? max_iters : 20000, &it, rel.data(), &ok)))
+                                 max_iters > 0 ? max_iters : 20000, &it, rel.data(), &ok, counts.one.data())))
         return rc;
-      most = std::max(most, it);
+      counts.add(it);
       conv &= ok;
       for (int j = 0; j < num_offsets; j++) worst[j] = std::max(worst[j], rel[j]);
     }
@@ -1183,7 +1199,7 @@ extern "C" int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int
       }
     MH_CHECK(hipStreamSynchronize(c.stream));
     if (stats) {
-      stats[0] = most;
+      stats[0] = counts.stage;
       stats[1] = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
       stats[2] = 0;
       stats[3] = conv;
@@ -1191,10 +1207,10 @@ extern "C" int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int
       stats[5] = 0;
       for (int j = 0; j < num_offsets; j++) {
         stats[6 + j] = worst[j];
-        stats[6 + num_offsets + j] = 0;
+        stats[6 + num_offsets + j] = counts.refine[j];
       }
     }
-    return (int)most;
+    return counts.stage;
   }
   if ((rc = ensure_links(P_F32))) return rc;
   const int nr = batch_width(nsrc);
@@ -1261,6 +1277,7 @@ extern "C" int milc_hip_multishift_invert_block(int external_precision, int nsrc
   const std::vector<double> offs(offsets, offsets + num_offsets), res(num_offsets, refine_residual);
   if (refine_residual > 0 && args.max_iter != 1 && block_is_small(nsrc) && multishift_small_takes(offs, res)) {
     std::vector<double> rel(num_offsets);
+    BlockCounts counts(num_offsets);
     // every source is read before a solution is written, as in the batch: the
     // arrays may be the same
     std::vector<VecField> b;
@@ -1274,11 +1291,13 @@ extern "C" int milc_hip_multishift_invert_block(int external_precision, int nsrc
       long it = 0;
       int ok = 1;
       if ((rc = multishift_small(b[s], xs[s], offs, res.data(), parity, args.max_iter > 0 ? args.max_iter : 20000, &it,
-                                 rel.data(), &ok)))
+                                 rel.data(), &ok, counts.one.data())))
         return rc;
+      counts.add(it);
       if (final_residual) std::copy(rel.begin(), rel.end(), final_residual + (size_t)s * num_offsets);
-      total = std::max(total, (int)it);
     }
+    total = counts.stage;
+    for (int n : counts.refine) total += n;
     for (int s = 0; s < nsrc; s++)
       for (int j = 0; j < num_offsets; j++)
         if ((rc = host_vec_out(external_precision, xs[s][j], pb, solution[(size_t)s * num_offsets + j]))) return rc;

@@ -238,9 +238,11 @@ bool multishift_small_takes(const std::vector<double>& offsets, const std::vecto
 // Multi-shift of a small lattice to each shift's own FP64 true residual
 // target resid[j] (what the FP32 stage and refine_shifts do on larger ones):
 // FP64 in one kernel, every true residual checked, a shift that misses its
-// target finished by its own CG.  iters, fres and converged as refine_shifts.
+// target finished by its own CG.  iters, fres and converged as refine_shifts;
+// refine_iters[j]: what of iters the CG of shift j took.
 int multishift_small(const VecField& b, std::vector<VecField>& x, const std::vector<double>& offsets,
-                     const double* resid, int parity, int max_iters, long* iters, double* fres, int* converged);
+                     const double* resid, int parity, int max_iters, long* iters, double* fres, int* converged,
+                     int* refine_iters = nullptr);
 // Whether a block call of `sources` sources solves them one after another.
 bool block_is_small(int sources);
 int shift_residuals(const VecField& b, const std::vector<VecField>& x, const double* offsets, int parity, double* rel);

@@ -506,9 +506,11 @@ bool block_is_small(int sources) {
 }
 
 int multishift_small(const VecField& b, std::vector<VecField>& x, const std::vector<double>& offsets,
-                     const double* resid, int parity, int max_iters, long* iters, double* fres, int* converged) {
+                     const double* resid, int parity, int max_iters, long* iters, double* fres, int* converged,
+                     int* refine_iters) {
   const int n = (int)offsets.size();
   if (n <= 0 || n > MS_MAX) return -2;
+  if (refine_iters) std::fill(refine_iters, refine_iters + n, 0);
   if (n == 1) {
     // a CG: one exchange of sums per iteration instead of two
     SolveParams sp;
@@ -563,6 +565,7 @@ int multishift_small(const VecField& b, std::vector<VecField>& x, const std::vec
       SolveStats s2;
       if ((rc = ensure_links(P_H16)) || (rc = cg_solve(b, x[j], 0.5 * std::sqrt(offsets[j]), sp, s2))) return rc;
       *iters += s2.iters;
+      if (refine_iters) refine_iters[j] = s2.iters;
       rel[j] = std::sqrt(s2.final_rsq);
       *converged &= s2.converged;
     }

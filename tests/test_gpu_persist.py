@@ -252,3 +252,26 @@ def test_block_multishift_takes_an_offset_of_zero(nsrc):
             G.dev_source(1451 + s, mq.EVEN, s)
         st = G.dev_multishift_block(list(range(nsrc)), [0.0, 0.5], 1e-6, 1e-9, out_slot0=20)
         assert st["converged"] and max(st["true_rel"]) < 1e-9
+
+
+@pytest.mark.parametrize("nsrc", [2, 7])
+def test_block_multishift_counts_stage_and_refinement(nsrc):
+    """On either side of the dispatch the device call counts the multi-shift's
+    iterations and those of each shift's refinement apart and the host call
+    returns their sum.  A target below what FP64 reaches (about 4e-16 |b|) needs
+    refinement, up to the cap."""
+    offs, cap = [0.04, 0.5], 200
+    with mq.Lattice((6, 4, 8, 6)) as G:
+        G.dev_gauge_hisq(1460)
+        for s in range(nsrc):
+            G.dev_source(1461 + s, mq.EVEN, s)
+        st = G.dev_multishift_block(list(range(nsrc)), offs, 1e-6, 1e-16, max_iters=cap)
+        print(st)
+        assert st["converged"] == 0 and max(st["true_rel"]) < 1e-14
+        assert st["iters"] == st["ms_iters"] < cap
+        assert all(cap <= it <= cap + 1 for it in st["refine_iters"])
+        fat, lng = G.dev_read_links()
+        srcs = [G.dev_read(s, mq.EVEN) for s in range(nsrc)]
+        G.set_links(fat, lng)
+        _, _, it = G.ks_multicg_offset_block(srcs, offs, mq.EVEN, 1e-6, 1e-16, max_iter=cap)
+        assert it == st["ms_iters"] + sum(st["refine_iters"])

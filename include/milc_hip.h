@@ -64,6 +64,15 @@ typedef struct {
 int milc_hip_init(const int dims[4], int device);
 /* Replaces qudaFinalize (ks_imp_rhmc/control.c:189). */
 int milc_hip_finalize(void);
+/* Form of the solves on small lattices of the current context: 1 (default, set
+ * by milc_hip_init) = the Krylov loop in one kernel and few sources one after
+ * another, where that is faster; 0 = launch by launch and batched, as on large
+ * lattices; 2 = as 1, but the kernels give up at once and their solves go on
+ * launch by launch, as they do when the kernel's workgroups are not resident
+ * together (the card shared with another process).  Same results within the
+ * solves' targets.  Returns -2 for another value.  No counterpart in the
+ * reference. */
+int milc_hip_set_small_lattice_form(int form);
 /* Library version string. */
 const char* milc_hip_version(void);
 

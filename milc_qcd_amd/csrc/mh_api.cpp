@@ -150,12 +150,12 @@ int milc_hip_init(const int dims[4], int device) {
   c.geom = make_geom(dims);
   c.Vh = c.geom.Vh;
   c.stride = plane_stride(c.Vh);
+  c.small_form = 1;
   MH_CHECK(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
   c.ws.max_blocks = (c.Vh + 255) / 256 + 1024;
   rc = dev_alloc((void**)&c.ws.partials, (size_t)c.ws.max_blocks * 4 * 2 * sizeof(double));
   if (rc) return rc;
   if ((rc = dev_alloc((void**)&c.ws.scal, sizeof(CGScalars)))) return rc;
-  if ((rc = dev_alloc((void**)&c.ws.flags, kPersistFlagBytes))) return rc;
   MH_CHECK(hipHostMalloc((void**)&c.ws.scal_host, sizeof(CGScalars), hipHostMallocDefault));
   // pinned read-back space for one partial record per block (vec_norm2)
   if (!pinned_scratch((size_t)c.ws.max_blocks * 4 * sizeof(double))) return -5;
@@ -183,7 +183,6 @@ int milc_hip_finalize(void) {
   c.thin_valid = false;
   dev_free(c.ws.partials);
   dev_free(c.ws.scal);
-  dev_free(c.ws.flags);
   if (c.ws.scal_host) (void)hipHostFree(c.ws.scal_host);
   if (c.ws.pinned) (void)hipHostFree(c.ws.pinned);
   dev_free(c.staging);
@@ -195,6 +194,14 @@ int milc_hip_finalize(void) {
   c.stream = nullptr;
   c.link_key = c.link_key2 = nullptr;
   c.initialised = false;
+  return 0;
+}
+
+int milc_hip_set_small_lattice_form(int form) {
+  Context& c = ctx();
+  if (!c.initialised) return -1;
+  if (form < 0 || form > 2) return -2;
+  c.small_form = form;
   return 0;
 }
 

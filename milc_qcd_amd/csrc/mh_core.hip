@@ -1141,7 +1141,7 @@ static int cg_solve_f64(const VecField& src, VecField& x, double mass, const Sol
     st.converged = 1;
     return vec_zero(x, P_F64);
   }
-  const bool one_kernel = !rel && persist_shape(c.Vh).lps > 0;
+  bool one_kernel = !rel && persist_shape(c.Vh).lps > 0;
   VecField ttt, p, r, tmp, extra;
   VecScope owned{&ttt, &p, &r, &tmp, &extra};
   if ((rc = alloc_vec(ttt, P_F64, c.stride)) || (rc = alloc_vec(p, P_F64, c.stride)) ||
@@ -1178,11 +1178,15 @@ static int cg_solve_f64(const VecField& src, VecField& x, double mass, const Sol
     left = std::min(left, max_cg - iteration);
     if (one_kernel) {
       VecField work[4] = {p, tmp, ttt, extra};
-      if ((rc = cg_persist(x, r, work, pb, msq_x4, (int)std::min<long>(left, 1L << 30)))) break;
-      if ((rc = read_scalars(&h))) break;
-      if (h.iters < 0) {
-        rc = -8;
-        break;
+      if ((rc = cg_persist(x, r, work, pb, msq_x4, (int)std::min<long>(left, 1L << 30))) < 0) break;
+      if (!rc && (rc = read_scalars(&h))) break;
+      if (rc || h.gone) {
+        // not launched, or given up: the launches below, from this restart on
+        rc = 0;
+        one_kernel = false;
+        iteration--;
+        nrestart--;
+        continue;
       }
       iteration += h.iters;
       size_r = h.rsq / source_norm;

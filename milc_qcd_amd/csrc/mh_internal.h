@@ -30,6 +30,9 @@ struct CGScalars {
   int go;              // written by every scalar step: 1 if this iteration's
                        // vector update must run
   int iters;           // scalar steps executed since the last reset
+  // set when a workgroup of the one-kernel solve gave up waiting; in a cache
+  // line of its own, which kernels touch with agent-scope accesses only
+  alignas(256) unsigned gone;
 };
 
 // Reduction scratch: partial sums per block (FP64) and the scalar block.
@@ -38,7 +41,6 @@ struct Workspace {
   int max_blocks = 0;
   CGScalars* scal = nullptr;   // device
   CGScalars* scal_host = nullptr;  // pinned host mirror
-  unsigned* flags = nullptr;       // barrier words of the one-kernel solvers
   void* pinned = nullptr;          // pinned host scratch for small read-backs
   size_t pinned_bytes = 0;
 };
@@ -79,6 +81,10 @@ struct Context {
   double* staging = nullptr;   // FP64 AoS staging buffer, 4*V*18 doubles
   size_t staging_elems = 0;
   int block = 256;
+  // 1: Krylov loops of small lattices in one kernel; 0: launch by launch and
+  // batched on every lattice; 2: as 1 with a poll limit of one, so that those
+  // kernels give up and the launches take over
+  int small_form = 1;
   bool initialised = false;
 };
 

@@ -413,7 +413,8 @@ static int multicg_run(const VecField& src64, std::vector<VecField>& x64, const 
   return 0;
 }
 
-// The FP64 solve of a small lattice in one kernel.
+// The FP64 solve of a small lattice in one kernel.  1: not done (the launch was
+// refused, or a workgroup gave up waiting), to be solved launch by launch.
 static int multicg_one_kernel(const VecField& src64, std::vector<VecField>& x64, const std::vector<double>& offsets,
                               const MultiParams& mp, SolveStats& st) {
   Context& c = ctx();
@@ -471,7 +472,7 @@ static int multicg_one_kernel(const VecField& src64, std::vector<VecField>& x64,
   if ((rc = ms_persist(src64, (const VecField*)(dev + head), work, pbit(mp.parity), (MSPersist*)dev))) return rc;
   MH_CHECK(hipMemcpyAsync(&h, dev, sizeof h, hipMemcpyDeviceToHost, c.stream));
   MH_CHECK(hipStreamSynchronize(c.stream));
-  if (h.iters < 0) return -8;
+  if (h.gone) return 1;
   st.iters = 1 + h.iters;
   st.converged = h.converged;
   st.final_rsq = st.size_r = h.rsq / source_norm;
@@ -481,9 +482,11 @@ static int multicg_one_kernel(const VecField& src64, std::vector<VecField>& x64,
 int multicg_solve(const VecField& src, std::vector<VecField>& x, const std::vector<double>& offsets,
                   const MultiParams& mp, SolveStats& st) {
   auto t0 = std::chrono::steady_clock::now();
-  int rc = mp.prec == P_F64 && mp.max_iters > 1 && persist_shape(ctx().Vh).lps
-               ? multicg_one_kernel(src, x, offsets, mp, st)
-           : mp.prec == P_F64 ? multicg_run<P_F64>(src, x, offsets, mp, st) : multicg_run<P_F32>(src, x, offsets, mp, st);
+  int rc = 1;
+  if (mp.prec == P_F64 && mp.max_iters > 1 && persist_shape(ctx().Vh).lps)
+    rc = multicg_one_kernel(src, x, offsets, mp, st);
+  if (rc == 1)
+    rc = mp.prec == P_F64 ? multicg_run<P_F64>(src, x, offsets, mp, st) : multicg_run<P_F32>(src, x, offsets, mp, st);
   (void)hipStreamSynchronize(ctx().stream);
   st.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   return rc;

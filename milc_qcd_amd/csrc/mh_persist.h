@@ -5,11 +5,10 @@
 namespace mh {
 
 constexpr int kPersistMaxBlocks = 256;
-constexpr size_t kPersistFlagBytes = 256;
 
 // Lanes per site, threads per workgroup and workgroups (one per CU, so that
 // the grid is resident at once) for Vh sites of a parity; lps = 0: the lattice
-// does not fit.
+// does not fit, or one-kernel solves are switched off.
 struct PersistShape {
   int lps, threads, blocks;
 };
@@ -22,8 +21,11 @@ PersistShape persist_shape(int Vh);
 constexpr int kPersistMixedSites = 49152;
 
 // FP64 CG iterations from a restart (r the residual, |r|^2 in the context's
-// CGScalars); x and the scalars are updated (iters = -1: a workgroup gave up
-// waiting), the work fields are scratch.
+// CGScalars); x and the scalars are updated, the work fields are scratch.
+// Returns 1 when the device refuses the launch.  With `gone` set in the
+// scalars a workgroup gave up waiting, and x holds a mixture of the guess and
+// iterates: either way the solve has to go on launch by launch from the true
+// residual.
 int cg_persist(VecField& x, VecField& r, VecField (&work)[4], int pb, double msq_x4, int max_it);
 
 // Multi-shift CG: most shifts of a solve, iterations of a window of deferred
@@ -55,10 +57,11 @@ struct MSPersist {
   double stop[MS_MAX];    // |r_j|^2 below which shift j (not the smallest) is done; 0: never
   double source_norm, rsqstop, rsq;
   int n, j_low, max_iter, iters, converged;
+  alignas(256) unsigned gone;  // as in CGScalars
 };
 // tab (device memory): psim_j in [0, n), pm_j in [MS_MAX, MS_MAX + n), the
-// residuals of a window in [2 MS_MAX, 2 MS_MAX + MS_KW); iters = -1 in io: a
-// workgroup gave up waiting.
+// residuals of a window in [2 MS_MAX, 2 MS_MAX + MS_KW).  Returns 1 when the
+// device refuses the launch; with `gone` set in io the solutions are void.
 int ms_persist(const VecField& src, const VecField* tab, VecField (&work)[4], int pb, MSPersist* io);
 
 }  // namespace mh

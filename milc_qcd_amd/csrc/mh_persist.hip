@@ -47,21 +47,27 @@ __device__ __forceinline__ bool empty(double v) { return (unsigned long long)__d
 
 // Polls of one word before the kernel gives up: seconds, against the
 // microseconds an exchange takes.  `gone` is the give-up word of the launch.
+// The workgroups are resident at once when the launch has the card to itself;
+// beside the kernels of another process they need not be, and the host then
+// finishes the solve with launches that wait for nobody.
 constexpr unsigned kMaxPolls = 4u << 20;
 
 struct Waiter {
   unsigned* gone;
+  unsigned limit;
   bool dead;
   // another poll (true) or give up (false)
   __device__ __forceinline__ bool again(unsigned& polls) {
     if (dead) return false;
-    if (++polls >= kMaxPolls ||
-        ((polls & 1023u) == 0 && __hip_atomic_load(gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+    if (++polls >= limit || ((polls & 1023u) == 0 && anybody_gone())) {
       __hip_atomic_store(gone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       dead = true;
       return false;
     }
     return true;
+  }
+  __device__ __forceinline__ bool anybody_gone() const {
+    return __hip_atomic_load(gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
   }
 };
 
@@ -325,6 +331,7 @@ struct Exchange {
   VecField p[2], tmp[2];
   double* rec;       // 3 * nb records of 4 doubles
   unsigned* gone;
+  unsigned polls;    // poll limit
 };
 
 // FP64 CG from a restart (p = r, |r|^2 in the scalars) to the recurrence
@@ -345,7 +352,7 @@ k_cg_persist(Geom g, LinkField fat, LinkField lng, VecField x, VecField r, Excha
   const bool on = cb < g.Vh;
   Vec3<double> xv, rv, pv, tv;
   SiteStencil<LPS, BS> st;
-  Waiter w{ex.gone, false};
+  Waiter w{ex.gone, ex.polls, false};
   zero(xv);
   zero(rv);
   if (on) {
@@ -358,7 +365,6 @@ k_cg_persist(Geom g, LinkField fat, LinkField lng, VecField x, VecField r, Excha
   double pkp = 0.0, c_tr = 0.0, c_tt = 0.0;
   const double stop = sc->rsq_stop;
   int it = 0, halt = 0;
-  bool ok = true;
   while (it < max_it && !halt) {
     const int e = it & 1;
     double s[4] = {0, 0, 0, rr_here};
@@ -379,7 +385,7 @@ k_cg_persist(Geom g, LinkField fat, LinkField lng, VecField x, VecField r, Excha
     }
     double* rec = ex.rec + (size_t)(it % 3) * 4 * nb;
     publish_sums<4, BS>(s, rec, sm);
-    if (!(ok = collect_sums<4, BS>(s, rec, nb, sm, &lds_dead, w))) break;
+    if (!collect_sums<4, BS>(s, rec, nb, sm, &lds_dead, w)) break;
     if (on) {
       empty_vec<LPS>(ex.p[e], cb, sub);
       empty_vec<LPS>(ex.tmp[e], cb, sub);
@@ -411,7 +417,10 @@ k_cg_persist(Geom g, LinkField fat, LinkField lng, VecField x, VecField r, Excha
       if (LPS > 1 && sub != 0) rr_here = 0.0;
     }
   }
-  if (on && sub == 0) store_vec<P_F64>(x, cb, xv);
+  // A thread that gives up publishes the sums of what it did not get (NaN) only
+  // after its give-up word: whoever collected those sums finds the word set, and
+  // leaves x as it was.
+  if (on && sub == 0 && !w.anybody_gone()) store_vec<P_F64>(x, cb, xv);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     sc->rsq = rsq;
     sc->oldrsq = oldrsq;
@@ -422,7 +431,7 @@ k_cg_persist(Geom g, LinkField fat, LinkField lng, VecField x, VecField r, Excha
     sc->a = a;
     sc->b = b;
     sc->rsq_max = rsq_max;
-    sc->iters = ok ? it : -1;
+    sc->iters = it;
     sc->halt = halt;
     sc->go = 0;
   }
@@ -462,7 +471,7 @@ k_ms_persist(Geom g, LinkField fat, LinkField lng, VecField src, const VecField*
   const double stop_shift = tid < n && tid != jl ? io->stop[tid] : 0.0;
   Vec3<double> rv, pv, tv;
   SiteStencil<LPS, BS> st;
-  Waiter w{ex.gone, false};
+  Waiter w{ex.gone, ex.polls, false};
   zero(rv);
   if (on) {
     load_vec<P_F64>(src, cb, rv);
@@ -473,7 +482,7 @@ k_ms_persist(Geom g, LinkField fat, LinkField lng, VecField src, const VecField*
   pv = rv;
   double rsq = io->source_norm, alpha_low = 0.0, beta_low_1 = -1.0;
   int it = 0, now = n, now_ws = n, m = 0, halt = 0, converged = 0;
-  bool first = true, ok = true;
+  bool first = true;
   __syncthreads();
   while (!halt) {
     const int e = it & 1;
@@ -504,7 +513,7 @@ k_ms_persist(Geom g, LinkField fat, LinkField lng, VecField src, const VecField*
     double* const rec_a = ex.rec + (size_t)e * 4 * nb;
     double* const rec_b = ex.rec + (size_t)(2 + e) * 4 * nb;
     publish_sums<1, BS>(s, rec_a, sm);
-    if (!(ok = collect_sums<1, BS>(s, rec_a, nb, sm, &lds_dead, w))) break;
+    if (!collect_sums<1, BS>(s, rec_a, nb, sm, &lds_dead, w)) break;
     if (on) {
       empty_vec<LPS>(ex.p[e], cb, sub);
       empty_vec<LPS>(ex.tmp[e], cb, sub);
@@ -552,7 +561,7 @@ k_ms_persist(Geom g, LinkField fat, LinkField lng, VecField src, const VecField*
       if (LPS > 1 && sub != 0) s[0] = 0.0;
     }
     publish_sums<1, BS>(s, rec_b, sm);
-    if (!(ok = collect_sums<1, BS>(s, rec_b, nb, sm, &lds_dead, w))) break;
+    if (!collect_sums<1, BS>(s, rec_b, nb, sm, &lds_dead, w)) break;
     if (tid == 0) st_empty(rec_a + 4 * blockIdx.x);
     const double oldrsq = rsq;
     rsq = s[0];
@@ -627,7 +636,7 @@ k_ms_persist(Geom g, LinkField fat, LinkField lng, VecField src, const VecField*
   }
   if (blockIdx.x == 0 && tid == 0) {
     io->rsq = rsq;
-    io->iters = ok ? it : -1;
+    io->iters = it;
     io->converged = converged;
   }
 }
@@ -664,6 +673,7 @@ int empty_words(void* p, size_t bytes) {
 // 6.3 / 22; 2048 8.1 / 30; 6000 8.1 / 38; 13824 12.8 / 52; 32768 27.8 / 60;
 // 65536 42 / 69; 73728 55 / 89; 131072 95 / 113.
 PersistShape persist_shape(int Vh) {
+  if (!ctx().small_form) return PersistShape{0, 0, 0};
   const int cus = std::min(cu_count(), kPersistMaxBlocks);
   constexpr PersistShape shapes[] = {{16, 256, 0}, {8, 256, 0}, {4, 256, 0}, {1, 256, 0}, {1, 512, 0}};
   for (PersistShape s : shapes) {
@@ -673,8 +683,8 @@ PersistShape persist_shape(int Vh) {
   return PersistShape{0, 0, 0};
 }
 
-// The exchange of a launch, all words empty.
-static int start_exchange(const VecField (&work)[4], int nb, int records, Exchange& ex) {
+// The exchange of a launch, all words empty; gone: its give-up word, zero.
+static int start_exchange(const VecField (&work)[4], int nb, int records, unsigned* gone, Exchange& ex) {
   Context& c = ctx();
   int rc;
   for (int k = 0; k < 4; k++) {
@@ -682,9 +692,21 @@ static int start_exchange(const VecField (&work)[4], int nb, int records, Exchan
     if ((rc = empty_words(work[k].data, vec_bytes(P_F64, work[k].stride)))) return rc;
   }
   ex.rec = c.ws.partials;
-  ex.gone = c.ws.flags;
-  if ((rc = empty_words(ex.rec, (size_t)records * 4 * nb * sizeof(double)))) return rc;
-  MH_CHECK(hipMemsetAsync(ex.gone, 0, kPersistFlagBytes, c.stream));
+  ex.gone = gone;
+  ex.polls = c.small_form == 2 ? 1u : kMaxPolls;
+  return empty_words(ex.rec, (size_t)records * 4 * nb * sizeof(double));
+}
+
+// 0: enqueued; 1: the device cannot hold the grid at once, or knows no such
+// launches.
+static int launch_persist(const void* kernel, const PersistShape& sh, void** args) {
+  const hipError_t e =
+      hipLaunchCooperativeKernel(kernel, dim3(sh.blocks), dim3(sh.threads), args, 0, ctx().stream);
+  if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported) {
+    (void)hipGetLastError();  // answered here
+    return 1;
+  }
+  MH_CHECK(e);
   return 0;
 }
 
@@ -700,16 +722,14 @@ int cg_persist(VecField& x, VecField& r, VecField (&work)[4], int pb, double msq
   const DevLinks& L = c.links[P_F64];
   const PersistShape sh = persist_shape(c.Vh);
   if (!L.valid || !sh.lps) return -3;
-  const int nb = sh.blocks;
   Exchange ex;
-  int rc = start_exchange(work, nb, 3, ex);
+  CGScalars* sc = c.ws.scal;
+  int rc = start_exchange(work, sh.blocks, 3, &sc->gone, ex);
   if (rc) return rc;
   Geom g = c.geom;
   LinkField fat = L.fat, lng = L.lng;
-  CGScalars* sc = c.ws.scal;
   void* args[] = {&g, &fat, &lng, &x, &r, &ex, &pb, &msq_x4, &max_it, &sc};
-  MH_CHECK(hipLaunchCooperativeKernel(PERSIST_KERNEL(k_cg_persist, sh), dim3(nb), dim3(sh.threads), args, 0, c.stream));
-  return 0;
+  return launch_persist(PERSIST_KERNEL(k_cg_persist, sh), sh, args);
 }
 
 int ms_persist(const VecField& src, const VecField* tab, VecField (&work)[4], int pb, MSPersist* io) {
@@ -718,15 +738,13 @@ int ms_persist(const VecField& src, const VecField* tab, VecField (&work)[4], in
   const PersistShape sh = persist_shape(c.Vh);
   if (!L.valid || !sh.lps) return -3;
   Exchange ex;
-  int rc = start_exchange(work, sh.blocks, 4, ex);
+  int rc = start_exchange(work, sh.blocks, 4, &io->gone, ex);
   if (rc) return rc;
   Geom g = c.geom;
   LinkField fat = L.fat, lng = L.lng;
   VecField s = src;
   void* args[] = {&g, &fat, &lng, &s, &tab, &ex, &pb, &io};
-  MH_CHECK(hipLaunchCooperativeKernel(PERSIST_KERNEL(k_ms_persist, sh), dim3(sh.blocks), dim3(sh.threads), args, 0,
-                                      c.stream));
-  return 0;
+  return launch_persist(PERSIST_KERNEL(k_ms_persist, sh), sh, args);
 }
 
 }  // namespace mh

@@ -53,7 +53,7 @@ EXPORTS = [
     "milc_hip_dev_block_dslash_bench", "milc_hip_dev_block_dslash", "milc_hip_dev_multishift_block",
     "milc_hip_dev_block_describe",
     "milc_hip_dev_multishift", "milc_hip_dev_hmc_step", "milc_hip_hisq_force", "milc_hip_eo_fermion_force_multi",
-    "milc_hip_set_force_form", "milc_hip_dev_rhmc_trajectory", "milc_hip_gauge_force", "milc_hip_gauge_action",
+    "milc_hip_set_force_form", "milc_hip_set_small_lattice_form", "milc_hip_dev_rhmc_trajectory", "milc_hip_gauge_force", "milc_hip_gauge_action",
     "milc_hip_update_u", "milc_hip_mom_action", "milc_hip_dev_load_thin_links", "milc_hip_dev_read_thin_links",
     "milc_hip_dev_dslash", "milc_hip_set_link_compression", "milc_hip_link_compression", "milc_hip_dev_hisq_force",
     "milc_hip_reunitarize", "milc_hip_dev_seed_rng", "milc_hip_dev_ranmom", "milc_hip_dev_gaussian_source",
@@ -218,6 +218,7 @@ def load_library(path=LIB_PATH):
     L.milc_hip_hisq_force.argtypes = [I, I, I, D, ctypes.POINTER(PD), ctypes.POINTER(P), PD, PD, P, P, P, P]
     L.milc_hip_eo_fermion_force_multi.argtypes = [I, D, PD, ctypes.POINTER(P), I, P, P]
     L.milc_hip_set_force_form.argtypes = [I]
+    L.milc_hip_set_small_lattice_form.argtypes = [I]
     L.milc_hip_dev_rhmc_trajectory.argtypes = [ctypes.POINTER(RhmcParams), ctypes.POINTER(D)]
     L.milc_hip_debug_fail_trajectory.argtypes = [I]
     L.milc_hip_dev_seed_rng.argtypes = [I, I]
@@ -624,6 +625,13 @@ class Lattice:
         _check(self.lib.milc_hip_reunitarize(2, tolerance, _p(links), int(bool(phases_in)), ctypes.byref(md),
                                              ctypes.byref(ne)), "milc_hip_reunitarize")
         return ne.value, md.value
+
+    def set_small_lattice_form(self, form):
+        """1 (default of a new context): one-kernel solves on small lattices; 0:
+        launch by launch and batched, as on large ones; 2: as 1, given up at once
+        and finished launch by launch"""
+        self._activate()
+        _check(self.lib.milc_hip_set_small_lattice_form(form), "milc_hip_set_small_lattice_form")
 
     def set_force_form(self, form):
         """0: path-table gather; 1 (default): staple form, for any links; 2:

@@ -275,3 +275,35 @@ def test_block_multishift_counts_stage_and_refinement(nsrc):
         G.set_links(fat, lng)
         _, _, it = G.ks_multicg_offset_block(srcs, offs, mq.EVEN, 1e-6, 1e-16, max_iter=cap)
         assert it == st["ms_iters"] + sum(st["refine_iters"])
+
+
+@pytest.mark.parametrize("dims", [(4, 4, 4, 4), (10, 10, 10, 12), (18, 6, 14, 28), (16, 16, 16, 32)])
+def test_given_up_solves_go_on_launch_by_launch(dims):
+    """A one-kernel solve that gives up waiting (form 2: a poll limit of one) is
+    finished by the loops of larger lattices (form 0), with the restarts and
+    iterations of those: bit for bit the same solutions and counts."""
+    print(f"given up {dims}", flush=True)
+    offs = OFFSETS[::4]
+    out = []
+    with mq.Lattice(dims) as G:
+        G.dev_gauge_hisq(1470)
+        G.dev_source(1471, mq.EVEN, 0)
+        for k, form in enumerate((0, 2)):
+            G.set_small_lattice_form(form)
+            it, st = G.dev_invert(0, 1 + k, 0.1, mq.EVEN, 1e-10, 0)
+            itc, stc = G.dev_invert(0, 3 + k, 0.1, mq.EVEN, 1e-10, 0, max_iter=7)
+            itm, _, conv = G.dev_multishift(0, offs, 1e-9, 0, out_slot0=10 + 4 * k)
+            assert st["converged"] and conv and st["resid"] < 1e-10
+            out.append((it, st["reliable_updates"], itc, stc["converged"], itm))
+        assert out[0] == out[1]
+        for a in (1, 3):
+            assert G.dev_diff(a, a + 1) == 0.0
+        for j in range(len(offs)):
+            assert G.dev_diff(10 + j, 14 + j) == 0.0
+        # where the small lattice's form is chosen for a mixed solve
+        it, st = G.dev_invert(0, 3, 0.1, mq.EVEN, 1e-10, 2)
+        assert st["converged"] and st["resid"] < 1e-10
+        itm, _, conv = G.dev_multishift(0, offs, 1e-9, 1, out_slot0=20)
+        assert conv
+        for j in range(len(offs)):
+            assert G.dev_diff(20 + j, 10 + j) < 10 * 2e-9 / offs[j]

@@ -1670,7 +1670,7 @@ int mom_action_dev(const double* mom_dev, double* action) {
 //
 // The Lepage term.  For unitary links it is cl S_nu(S_nu(L_mu)) with -6 cl on
 // the one-link term (the retracing paths of the double staple equal L_mu), and
-// takes no pass of its own beside 7-staples: its FA part is c7's, already in
+// takes no pass of its own beside 7-staples of its size: its FA part is c7's, already in
 // G2[nu], so G1[nu] starts as (c3 - cl c5 / c7) F + (cl / c7) G2[nu], and its
 // FU part rides on the 7-staples' (argument + (cl / c7) S1[rho]).  For links
 // that need not be unitary it is the path itself, the upper half of S_nu of the
@@ -1685,8 +1685,13 @@ static int smear_adjoint_dev(const LinkField& L, const LinkField& F1, const Link
   const double c1 = coeff[0] - (split ? 0.0 : 6.0 * cl);
   const bool staples = c3 != 0.0 || cl != 0.0 || c5 != 0.0 || c7 != 0.0;
   const bool five = c5 != 0.0 || c7 != 0.0, seven = c7 != 0.0;
-  const bool ride = cl != 0.0 && !split && seven;  // Lepage term on the 7-staples' passes
-  const bool double_staple = cl != 0.0 && !split && !seven;
+  // Lepage term on the 7-staples' passes.  Its parts of F, cl c5 / c7 in G1 and
+  // in (cl / c7) G2, cancel: they stay of the size of the one-link term's 6 cl
+  // only while c7 is not small beside c5 and cl (c5 / c7 and cl / c7 are 6 and
+  // 48 in the HISQ smearing, 6 u0^2 and 24 u0^2 in asqtad; with c7 a thousandth
+  // of asqtad's the momentum lost two digits)
+  const bool ride = cl != 0.0 && !split && std::abs(cl) <= 64.0 * std::abs(c7) && std::abs(c5) <= 8.0 * std::abs(c7);
+  const bool double_staple = cl != 0.0 && !split && !ride;
   // buffers by slot of the three other directions
   double2 *F = nullptr, *SS = nullptr, *S1[3] = {}, *G1[3] = {}, *G2[3] = {}, *H[4] = {};
   OnExit bufs([&] {

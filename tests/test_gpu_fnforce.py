@@ -125,3 +125,28 @@ def test_staple_form_against_the_path_table(have, dims):
                 assert err < 1e-13
         finally:
             G.set_force_form(1)
+
+
+@pytest.mark.parametrize("c7_factor", [1.0, 0.55, 0.54, 0.1, 1e-3, 1e-9, 1e-300])
+def test_staple_form_with_a_small_seven_staple_term(c7_factor):
+    """The Lepage term of unitary links takes the 7-staples' passes only beside
+    7-staples of its size (the line lies between factors 0.55 and 0.54 of
+    asqtad's coefficient at this u0); below, no digits are lost against the path
+    table (1e-13, as above)."""
+    dims = (4, 6, 4, 10)
+    c = list(ko.asqtad_coeffs(0.85))
+    c[4] *= c7_factor
+    L = ko.Lattice(dims)
+    U = L.rephase(L.gauge_random(1031))
+    xs = [L.gaussian_vector(1033 + t, ko.EVENANDODD) for t in range(2)]
+    with mq.Lattice(dims) as G:
+        try:
+            mom = [np.zeros((L.V, 4, 10)), np.zeros((L.V, 4, 10))]
+            for m, f in zip(mom, (0, 2)):
+                G.set_force_form(f)
+                G.fermion_force_fn_multi(0.1, [0.7, -0.4], xs, c, U, m)
+            err = np.linalg.norm(mom[1] - mom[0]) / np.linalg.norm(mom[0])
+            print(f"{c7_factor}: {err:.1e}", flush=True)
+            assert err < 1e-13
+        finally:
+            G.set_force_form(1)

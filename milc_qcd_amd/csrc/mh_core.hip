@@ -1400,7 +1400,8 @@ int cg_iteration_profile(const VecField& src, double mass, int parity, int reps,
 // The work vectors cg_solve_f64 / cg_solve_mixed allocate, 256-byte aligned.
 size_t cg_scratch_bytes(int ps, int Vh, int stride) {
   auto a = [&](int prec) { return (vec_bytes(prec, stride) + 255) & ~(size_t)255; };
-  if (ps == P_F64 || Vh <= kPersistMixedSites) return (persist_shape(Vh).lps ? 5 : 4) * a(P_F64);
+  const bool one_kernel = persist_shape(Vh).lps > 0;
+  if (ps == P_F64 || (one_kernel && Vh <= kPersistMixedSites)) return (one_kernel ? 5 : 4) * a(P_F64);
   return 2 * a(P_F64) + 2 * a(ps) + 3 * a(ps == P_H16 ? kH16Arith : P_F32);
 }
 

@@ -1105,7 +1105,7 @@ extern "C" int milc_hip_dev_block_tune(int prec, int nrhs, int* variant, double*
   if (!c.initialised || !c.links[P_F64].valid) return -1;
   int ip = block_prec(prec);
   if (ip != P_F64 && ensure_links(ip)) return -3;
-  if (nrhs != 4 && nrhs != 8 && nrhs != 16) return -2;
+  if (!is_batch_width(nrhs)) return -2;
   int v;
   double us;
   int rc = btune(ip, nrhs, &v, &us);
@@ -1138,7 +1138,7 @@ extern "C" int milc_hip_dev_block_dslash(int prec, int nrhs, int variant, int ns
                                          int out_parity, const int* dst_slots) {
   Context& c = ctx();
   if (!c.initialised || !c.links[P_F64].valid) return -1;
-  if (nsrc <= 0 || nsrc > nrhs || (nrhs != 4 && nrhs != 8 && nrhs != 16)) return -2;
+  if (nsrc <= 0 || nsrc > nrhs || !is_batch_width(nrhs)) return -2;
   int ip = block_prec(prec);
   int rc;
   if (ip != P_F64 && (rc = ensure_links(ip))) return rc;

@@ -24,6 +24,7 @@ namespace mh {
 inline int batch_width(int n) {
   return n <= 2 ? 2 : (n <= 4 ? 4 : (n <= 6 ? 6 : (n <= 8 ? 8 : (n <= 12 ? 12 : 16))));
 }
+inline bool is_batch_width(int nr) { return nr > 0 && nr <= BNR_MAX && batch_width(nr) == nr; }
 #define BMS_MAX 32   // shifts per multi-shift solve
 #define BKW 8        // iterations per deferred shift-update window
 

@@ -13,6 +13,14 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "slow: longer CPU oracle checks")
 
 
+@pytest.fixture(params=[1, 0], ids=["small-lattice-form", "large-lattice-form"])
+def small_form(request):
+    """Both forms of the solves on a small lattice, for Lattice.set_small_lattice_form:
+    a lattice that the oracle solves quickly takes the one-kernel solves (1); the
+    launch-by-launch and batched ones of larger lattices are tested on it too (0)."""
+    return request.param
+
+
 @pytest.fixture(scope="session")
 def oracle():
     import ks_oracle

@@ -125,14 +125,16 @@ def oracle_multishift(L, fat, lng, srcs, parity):
 
 
 @pytest.mark.parametrize("parity", [ko.EVEN, ko.ODD])
-def test_multishift_block_refined_vs_oracle(l8, parity):
-    """3 sources (padded to a batch of 4), 4 shifts; FP32 multi-shift then
-    per-shift refinement to a 1e-10 FP64 true residual."""
+def test_multishift_block_refined_vs_oracle(l8, parity, small_form):
+    """3 sources, 4 shifts, every shift to a 1e-10 FP64 true residual; as a batch
+    of 4 with a padding source (large-lattice form) by an FP32 multi-shift and
+    per-shift refinement."""
     L, fat, lng = l8
     srcs = [L.gaussian_vector(800 + s, parity) for s in range(3)]
     ref = oracle_multishift(L, fat, lng, srcs, parity)
     sl = L.parity_slice(parity)
     with mq.Lattice(L.dims) as G:
+        G.set_small_lattice_form(small_form)
         G.dev_load_links(fat, lng)
         for s, v in enumerate(srcs):
             G.dev_write(s, parity, v)
@@ -172,10 +174,10 @@ def test_multishift_block_fp32_stage_vs_oracle(l8):
         assert np.array_equal(a, G.dev_read(16, ko.EVEN))
 
 
-def test_multishift_block_seven_shifts_refined_from_1e4_vs_oracle(l8):
-    """2 sources (a batch of 4) and 7 shifts, the FP32 stage stopped at 1e-4 so
-    that every shift's refinement runs sloppy phases and reliable updates down to
-    a 1e-10 FP64 true residual."""
+def test_multishift_block_seven_shifts_refined_from_1e4_vs_oracle(l8, small_form):
+    """2 sources and 7 shifts to a 1e-10 FP64 true residual; as a batch (large-
+    lattice form) with the FP32 stage stopped at 1e-4, so that every shift's
+    refinement runs sloppy phases and reliable updates."""
     L, fat, lng = l8
     offs = [4 * 0.05 ** 2 + s for s in (3e-4, 1e-3, 3e-3, 1e-2, 3e-2, 0.1, 1.0)]
     srcs = [L.gaussian_vector(1200 + s, ko.EVEN) for s in range(2)]
@@ -185,6 +187,7 @@ def test_multishift_block_seven_shifts_refined_from_1e4_vs_oracle(l8):
         ref.append(xs)
     sl = L.parity_slice(ko.EVEN)
     with mq.Lattice(L.dims) as G:
+        G.set_small_lattice_form(small_form)
         G.dev_load_links(fat, lng)
         for s, v in enumerate(srcs):
             G.dev_write(s, ko.EVEN, v)
@@ -198,13 +201,14 @@ def test_multishift_block_seven_shifts_refined_from_1e4_vs_oracle(l8):
                 assert rel(got[sl], ref[s][j][sl]) < 1e-7, (s, j)
 
 
-def test_multishift_invert_block_host_abi(l8):
+def test_multishift_invert_block_host_abi(l8, small_form):
     """milc_hip_multishift_invert_block with MILC-layout host arrays."""
     L, fat, lng = l8
     srcs = [L.gaussian_vector(1100 + s, ko.ODD) for s in range(5)]
     ref = oracle_multishift(L, fat, lng, srcs, ko.ODD)
     sl = L.parity_slice(ko.ODD)
     with mq.Lattice(L.dims) as G:
+        G.set_small_lattice_form(small_form)
         G.set_links(fat, lng)
         psim, res, it = G.ks_multicg_offset_block(srcs, OFFS, ko.ODD, 1e-5, 1e-10)
     for s in range(5):
@@ -215,7 +219,7 @@ def test_multishift_invert_block_host_abi(l8):
             assert not other.any()  # only the solve parity is written
 
 
-def test_invert_block_vs_oracle(l8):
+def test_invert_block_vs_oracle(l8, small_form):
     """ks_congrad_block_parity form: 6 sources, one with a nonzero initial guess."""
     L, fat, lng = l8
     m = 0.05
@@ -224,6 +228,7 @@ def test_invert_block_vs_oracle(l8):
     dests[2][:] = 0.3 * L.gaussian_vector(1300, ko.EVEN)
     sl = L.parity_slice(ko.EVEN)
     with mq.Lattice(L.dims) as G:
+        G.set_small_lattice_form(small_form)
         G.set_links(fat, lng)
         q = mq.QuarkInvertControl(max=2000, nrestart=5, parity=ko.EVEN, resid=1e-10)
         it, fres = G.ks_congrad_block_parity(srcs, dests, q, m)
@@ -233,7 +238,7 @@ def test_invert_block_vs_oracle(l8):
         assert rel(dests[s][sl], x[sl]) < 1e-8, s
 
 
-def test_batched_solvers_stop_at_max_iters(l8):
+def test_batched_solvers_stop_at_max_iters(l8, small_form):
     """The iteration cap holds inside the captured windows: the batched
     multi-shift stops at max_iters (ks_multicg_offset.c counts the set-up as
     one), the batched CG at max_iters plus the closing true-residual
@@ -243,6 +248,7 @@ def test_batched_solvers_stop_at_max_iters(l8):
     L, fat, lng = l8
     srcs = [L.gaussian_vector(1400 + s, ko.EVEN) for s in range(4)]
     with mq.Lattice(L.dims) as G:
+        G.set_small_lattice_form(small_form)
         G.dev_load_links(fat, lng)
         for s, v in enumerate(srcs):
             G.dev_write(s, ko.EVEN, v)
@@ -259,16 +265,19 @@ def test_batched_solvers_stop_at_max_iters(l8):
 
 
 @pytest.mark.parametrize("dims", [(4, 4, 4, 4), (6, 4, 8, 6), (8, 6, 4, 10)])
-@pytest.mark.parametrize("nsrc,nshift", [(1, 1), (2, 1), (2, 12), (2, 32), (3, 31), (7, 2), (9, 3), (12, 2)])
-def test_multishift_block_widths_vs_oracle(dims, nsrc, nshift):
-    """Batches of every width, full and with padding sources, with one shift to
-    the most: solutions against the oracle's multi-shift CG to 1e-13.
+@pytest.mark.parametrize("nsrc,nshift", [(1, 1), (2, 1), (2, 12), (2, 32), (3, 31), (4, 3), (5, 2), (6, 12), (7, 2),
+                                         (9, 3), (12, 2), (13, 1)])
+def test_multishift_block_widths_vs_oracle(dims, nsrc, nshift, small_form):
+    """One shift to the most, for source counts that make batches of every width,
+    full and with padding sources, in the large-lattice form; in the other up to
+    six sources are solved one after another.  Solutions against the oracle's multi-shift CG to 1e-13.
     A shift refined to the true residual r is off by r |b| / (offset |x|) at
     most, and |x| >= |b| / (offset + 10)."""
     L, fat, lng = hisq_setup(dims, 1007)
     offs = [0.04 * 1.3 ** j for j in range(nshift)]
     resid = 1e-9
     with mq.Lattice(dims) as G:
+        G.set_small_lattice_form(small_form)
         G.set_links(fat, lng)
         for parity in (ko.EVEN, ko.ODD):
             sl = L.parity_slice(parity)

@@ -58,7 +58,7 @@ def test_hmc_step_48x48x48x96_mixed_vs_fp64_force():
         assert st["S"] > 0
 
 
-def test_hmc_step_vs_oracle_8x8x8x8():
+def test_hmc_step_vs_oracle_8x8x8x8(small_form):
     dims = (8, 8, 8, 8)
     L = ko.Lattice(dims)
     U = L.rephase(L.gauge_random(1010))
@@ -75,6 +75,7 @@ def test_hmc_step_vs_oracle_8x8x8x8():
         tot = tot + r * x
     act_ref = float(np.sum(tot[E] ** 2))
     with mq.Lattice(dims) as G:
+        G.set_small_lattice_form(small_form)
         G.dev_load_links(fat, lng)
         G.dev_write(0, ko.EVEN, phi)
         st = G.dev_hmc_step(0, offs, res, 1e-11, mixed=1, compare_fp64=True)

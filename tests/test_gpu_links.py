@@ -76,20 +76,26 @@ def test_non_unitary_long_links_keep_nine_elements(hisq):
             assert rel(got, ref) < 5e-4
 
 
-def test_mixed_cg_on_two_row_links_reaches_target(hisq):
-    """the mixed 16-bit CG on two-row long links: FP64 true residual 1e-10 and
-    the solution within 1e-8 of the oracle's"""
+@pytest.mark.parametrize("compressed", [1, 0])
+def test_mixed_cg_on_two_row_links_reaches_target(hisq, small_form, compressed):
+    """the mixed 16-bit CG (large-lattice form) on two-row and on nine-element long
+    links: FP64 true residual 1e-10 and the solution within 1e-8 of the oracle's"""
     L, fat, lng = hisq
     m = 0.05
     src = L.gaussian_vector(1403, ko.EVEN)
     ref, _, _ = L.congrad(fat, lng, src, m, 1e-14, parity=ko.EVEN, max_iters=5000, nrestart=5)
     sl = L.parity_slice(ko.EVEN)
     with mq.Lattice(DIMS) as G:
-        G.dev_load_links(fat, lng)
-        assert G.link_compression(2) == 1
-        G.dev_write(0, ko.EVEN, src)
-        it, st = G.dev_invert(0, 1, m, mq.EVEN, 1e-10, 2)
-        print(it, st)
-        x = G.dev_read(1, ko.EVEN)
+        G.set_small_lattice_form(small_form)
+        G.set_link_compression(compressed)  # process-wide setting: restored below
+        try:
+            G.dev_load_links(fat, lng)
+            assert G.link_compression(2) == compressed
+            G.dev_write(0, ko.EVEN, src)
+            it, st = G.dev_invert(0, 1, m, mq.EVEN, 1e-10, 2)
+            print(it, st)
+            x = G.dev_read(1, ko.EVEN)
+        finally:
+            G.set_link_compression(1)
     assert st["converged"] == 1 and st["resid"] < 1e-10
     assert rel(x[sl], ref[sl]) < 1e-8

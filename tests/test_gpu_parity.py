@@ -38,6 +38,13 @@ def gpu8(hisq8):
     G.close()
 
 
+@pytest.fixture
+def solver8(gpu8, small_form):
+    gpu8.set_small_lattice_form(small_form)
+    yield gpu8
+    gpu8.set_small_lattice_form(1)
+
+
 def test_library_exports():
     lib = mq.load_library()
     for name in mq.EXPORTS:
@@ -67,14 +74,14 @@ def test_dslash_f32(hisq8, gpu8):
     assert rel(out[s], ref[s]) < 1e-5
 
 
-def test_cg_f64_matches_oracle_iteration_for_iteration(hisq8, gpu8):
+def test_cg_f64_matches_oracle_iteration_for_iteration(hisq8, solver8):
     """Same restart cadence, same iteration count, solution to 1e-12 (m = 0.5, well conditioned)."""
     L, U, fat, lng, W, _ = hisq8
     src = L.gaussian_vector(2000, ko.EVEN)
     ref, it_ref, q_ref = L.congrad(fat, lng, src, 0.5, 1e-14, parity=ko.EVEN, max_iters=40, nrestart=10)
     x = np.zeros_like(src)
     qic = mq.QuarkInvertControl(max=40, nrestart=10, parity=mq.EVEN, resid=1e-14)
-    it = gpu8.ks_congrad_parity(src, x, qic, 0.5)
+    it = solver8.ks_congrad_parity(src, x, qic, 0.5)
     s = L.parity_slice(ko.EVEN)
     print(f"cg f64: iters gpu {it} oracle {it_ref}; rel {rel(x[s], ref[s]):.3e}")
     assert abs(it - it_ref) <= 1
@@ -82,13 +89,13 @@ def test_cg_f64_matches_oracle_iteration_for_iteration(hisq8, gpu8):
     assert np.all(x[L.parity_slice(ko.ODD)] == 0)
 
 
-def test_cg_f64_light_mass(hisq8, gpu8):
+def test_cg_f64_light_mass(hisq8, solver8):
     L, U, fat, lng, W, _ = hisq8
     src = L.gaussian_vector(2001, ko.ODD)
     ref, it_ref, q_ref = L.congrad(fat, lng, src, 0.05, 1e-12, parity=ko.ODD, max_iters=300, nrestart=5)
     x = np.zeros_like(src)
     qic = mq.QuarkInvertControl(max=300, nrestart=5, parity=mq.ODD, resid=1e-12)
-    it = gpu8.ks_congrad_parity(src, x, qic, 0.05)
+    it = solver8.ks_congrad_parity(src, x, qic, 0.05)
     s = L.parity_slice(ko.ODD)
     # FP64 true residual recomputed by the oracle
     r = src - L.mdagm(fat, lng, 4 * 0.05 ** 2, x, ko.ODD)
@@ -100,13 +107,13 @@ def test_cg_f64_light_mass(hisq8, gpu8):
 
 
 @pytest.mark.parametrize("mixed,tol", [(1, 1e-10), (2, 1e-10)])
-def test_cg_mixed_reaches_fp64_residual(hisq8, gpu8, mixed, tol):
+def test_cg_mixed_reaches_fp64_residual(hisq8, solver8, mixed, tol):
     L, U, fat, lng, W, _ = hisq8
     src = L.gaussian_vector(2002, ko.EVEN)
     ref, it_ref, _ = L.congrad(fat, lng, src, 0.05, 1e-13, parity=ko.EVEN, max_iters=1000, nrestart=5)
     x = np.zeros_like(src)
     qic = mq.QuarkInvertControl(max=4000, nrestart=1, parity=mq.EVEN, resid=tol, mixed=mixed)
-    it = gpu8.ks_congrad_parity(src, x, qic, 0.05)
+    it = solver8.ks_congrad_parity(src, x, qic, 0.05)
     r = src - L.mdagm(fat, lng, 4 * 0.05 ** 2, x, ko.EVEN)
     tr = np.sqrt(L.norm2(r, ko.EVEN) / L.norm2(src, ko.EVEN))
     s = L.parity_slice(ko.EVEN)
@@ -147,7 +154,7 @@ def test_device_source_matches_oracle():
     assert rel(v[s], ref[s]) < 1e-14
 
 
-def test_multishift_f64_matches_oracle(hisq8, gpu8):
+def test_multishift_f64_matches_oracle(hisq8, solver8):
     L, U, fat, lng, W, _ = hisq8
     src = L.gaussian_vector(3000, ko.EVEN)
     m = 0.05
@@ -155,7 +162,7 @@ def test_multishift_f64_matches_oracle(hisq8, gpu8):
     ref, it_ref, _ = L.multicg_offset(fat, lng, src, offsets, 1e-12, parity=ko.EVEN, max_iters=2000, nrestart=1)
     ksp = [mq.KsParam(offset=o) for o in offsets]
     qic = [mq.QuarkInvertControl(max=2000, nrestart=1, parity=mq.EVEN, resid=1e-12) for _ in offsets]
-    xs = gpu8.ks_multicg_offset_field(src, ksp, qic, mixed=0, prec=2)
+    xs = solver8.ks_multicg_offset_field(src, ksp, qic, mixed=0, prec=2)
     s = L.parity_slice(ko.EVEN)
     for j, o in enumerate(offsets):
         e = rel(xs[j][s], ref[j][s])
@@ -165,10 +172,11 @@ def test_multishift_f64_matches_oracle(hisq8, gpu8):
 
 
 @pytest.mark.parametrize("mixed,parity", [(1, ko.EVEN), (2, ko.EVEN), (2, ko.ODD)])
-def test_multishift_mixed_per_shift_residuals(hisq8, gpu8, mixed, parity):
-    """FP32 bulk, then every shift refined to its own FP64 target with an FP32
-    (mixed 1) or 16-bit (mixed 2) sloppy operator; six shifts are refined as a
-    batched group of four and one of two (two unused slots)."""
+def test_multishift_mixed_per_shift_residuals(hisq8, solver8, mixed, parity):
+    """Every shift to its own FP64 target.  Large-lattice form: FP32 bulk, then
+    every shift refined with an FP32 (mixed 1) or 16-bit (mixed 2) sloppy
+    operator; six shifts are refined as a batched group of four and one of two
+    (two unused slots)."""
     L, U, fat, lng, W, _ = hisq8
     src = L.gaussian_vector(3001, parity)
     m = 0.02
@@ -176,7 +184,7 @@ def test_multishift_mixed_per_shift_residuals(hisq8, gpu8, mixed, parity):
     targets = [1e-9, 1e-9, 3e-9, 1e-8, 1e-8, 3e-8]
     ksp = [mq.KsParam(offset=o) for o in offsets]
     qic = [mq.QuarkInvertControl(max=3000, nrestart=1, parity=parity, resid=t) for t in targets]
-    xs = gpu8.ks_multicg_offset_field(src, ksp, qic, mixed=mixed, prec=1)
+    xs = solver8.ks_multicg_offset_field(src, ksp, qic, mixed=mixed, prec=1)
     bn = np.sqrt(L.norm2(src, parity))
     for j, o in enumerate(offsets):
         r = src - L.mdagm(fat, lng, o, xs[j], parity)
@@ -188,9 +196,9 @@ def test_multishift_mixed_per_shift_residuals(hisq8, gpu8, mixed, parity):
 
 
 @pytest.mark.parametrize("nshift", [1, 5, 9])
-def test_multishift_mixed_group_edges(hisq8, gpu8, nshift):
-    """Shift counts at the edges of the grouped refinement: one shift (the
-    one-source mixed CG alone), five (a group of four and a lone shift) and
+def test_multishift_mixed_group_edges(hisq8, solver8, nshift):
+    """Shift counts at the edges of the large-lattice form's grouped refinement:
+    one shift (the one-source mixed CG alone), five (a group of four and a lone shift) and
     nine (two groups and a lone shift); every shift to its FP64 target."""
     L, U, fat, lng, W, _ = hisq8
     src = L.gaussian_vector(3100 + nshift, ko.EVEN)
@@ -198,7 +206,7 @@ def test_multishift_mixed_group_edges(hisq8, gpu8, nshift):
     offsets = [4 * m * m + s for s in np.geomspace(3e-4, 0.5, nshift)] if nshift > 1 else [4 * m * m + 1e-3]
     ksp = [mq.KsParam(offset=o) for o in offsets]
     qic = [mq.QuarkInvertControl(max=3000, nrestart=1, parity=ko.EVEN, resid=1e-9) for _ in offsets]
-    xs = gpu8.ks_multicg_offset_field(src, ksp, qic, mixed=2, prec=1)
+    xs = solver8.ks_multicg_offset_field(src, ksp, qic, mixed=2, prec=1)
     bn = np.sqrt(L.norm2(src, ko.EVEN))
     for j, o in enumerate(offsets):
         tr = np.sqrt(L.norm2(src - L.mdagm(fat, lng, o, xs[j], ko.EVEN), ko.EVEN)) / bn

@@ -105,8 +105,8 @@ def test_multishift_one_kernel(dims, mixed):
 
 
 @pytest.mark.parametrize("n", [1, 2, 31, 32])
-def test_multishift_one_kernel_shift_counts_and_retirement(n):
-    """Shift counts at the ends of the table, the smallest offset last or first,
+def test_multishift_one_kernel_shift_counts_and_retirement(n, small_form):
+    """In one kernel and launch by launch: shift counts at the ends of the table, the smallest offset last or first,
     heavy shifts whose zeta underflows (retired), and iteration caps inside and
     at the edge of a window, against the oracle's multi-shift CG."""
     dims = (6, 4, 8, 6)
@@ -117,6 +117,7 @@ def test_multishift_one_kernel_shift_counts_and_retirement(n):
     offs = [0.04 * 1.9 ** (j if n % 2 else n - 1 - j) for j in range(n)]
     s = L.parity_slice(ko.EVEN)
     with mq.Lattice(dims) as G:
+        G.set_small_lattice_form(small_form)
         G.set_links(fat, lng)
         for cap in (3000, 2, 9, 10):
             ref, it_ref, _ = L.multicg_offset(fat, lng, src, offs, 1e-10, max_iters=cap, nrestart=1)

@@ -82,7 +82,7 @@ MILC_RESID = [(5e-4, 1e-4, 1e-4)] + [(5e-6, 1e-6, 1e-6)] * 3
 
 
 @pytest.mark.parametrize("mixed", [0, 1])
-def test_milc_su3_rhmc_hisq_trajectory(mixed):
+def test_milc_su3_rhmc_hisq_trajectory(mixed, small_form):
     links, info = lio.reload_lattice(os.path.join(HERE, "golden", "io", "lat.sample.l6666.hisq"))
     assert info["checksum_ok"]
     dims = (6, 6, 6, 6)
@@ -92,6 +92,7 @@ def test_milc_su3_rhmc_hisq_trajectory(mixed):
     assert len(pfs) == 4
     coeff = mq.gauge_loop_coeffs(0.89, 3)
     with mq.Lattice(dims) as G:
+        G.set_small_lattice_form(small_form)
         G.dev_load_thin_links(links, phases_in=False)
         G.dev_seed_rng(MILC_ISEED, precision=1)
         st = G.dev_rhmc_trajectory(10, 0.02, 7.4, coeff, pfs, integrator=mq.INT_3G1F, mixed_md=mixed,
@@ -434,26 +435,30 @@ def test_multi_timescale_integrators(alg, ngauge):
     assert abs(a["dH"]) < abs(lf["dH"])
 
 
-def test_mixed_md_solves_track_fp64():
+def test_mixed_md_solves_track_fp64(small_form):
     """mixed-precision MD solves (FP32 multi-shift + 16-bit refinement, links
     rebuilt each step) give the FP64-solve trajectory's dH to the solver
     tolerance"""
     with mq.Lattice(DIMS) as G:
+        G.set_small_lattice_form(small_form)
         G.dev_gauge_hisq(1200, 0.4)
         a = traj(G, 4, 0.05)
         b = traj(G, 4, 0.05, mixed_md=1, resid_md=1e-10)
     assert abs(a["dH"] - b["dH"]) < 1e-5 * max(1.0, abs(a["dH"]))
 
 
-def test_batched_pseudofermion_solves_match_one_source_solves():
-    """three pseudofermions with different masses and rational orders: the
-    batched multi-shift with a shift set per source (heatbath, MD and action
-    solves) reproduces the one-source FP64 solves' actions and dH"""
+@pytest.mark.parametrize("n", [2, 3, 5])
+def test_batched_pseudofermion_solves_match_one_source_solves(n, small_form):
+    """two, three and five pseudofermions with different masses and rational orders:
+    the solves of all of them (heatbath, MD and action; batched, with a shift set
+    per source, in the large-lattice form) reproduce the one-source FP64 solves'
+    actions and dH"""
     def pfs(resid):
         return [mq.Pseudofermion(mass=m, md=rat(MD), gr=rat(g), fa=rat(MD), resid_md=resid, resid_gr=resid,
                                  resid_fa=resid)
-                for m, g in ((0.1, GR), (0.3, ([0.2, 0.4], [0.5, 1.5], 1.0)), (0.05, GR))]
+                for m, g in ((0.1, GR), (0.3, ([0.2, 0.4], [0.5, 1.5], 1.0)), (0.05, GR), (0.2, GR), (0.4, GR))[:n]]
     with mq.Lattice(DIMS) as G:
+        G.set_small_lattice_form(small_form)
         G.dev_gauge_hisq(1200, 0.4)
         a = G.dev_rhmc_trajectory(4, 0.05, BETA, COEFF, pfs(1e-12), integrator=mq.INT_LEAPFROG, mixed_md=0,
                                   mixed_action=0, action_from_md=False, accept=2, seed=11)

@@ -6,7 +6,8 @@ kernels in the same order, so on the same links and source their solutions,
 iteration counts and residuals must agree (bar: 1e-14 relative on the
 solution, equal iteration counts).  Two calls in a row through the C ABI, the
 second on a smaller lattice (the scratch then holds the first call's data),
-each in FP64 and in 16-bit mixed precision.  Also: the size limit and the
+each in FP64 and in FP32 and 16-bit mixed precision, in the one-kernel and in
+the launch-by-launch form of small lattices.  Also: the size limit and the
 preconditions are reported as errors, not allocations.
 """
 import ctypes
@@ -27,9 +28,10 @@ def _noalloc(G, slot_b, slot_x, mass, parity, resid, mixed, max_iter=2000):
     return rc, {"resid": st[0], "converged": int(st[3]), "iters": int(st[4]), "final_rsq": st[5]}
 
 
-def _compare_on(dims, seed):
-    print(f"noalloc vs allocating solve on {dims}", flush=True)
+def _compare_on(dims, seed, form):
+    print(f"noalloc vs allocating solve on {dims}, form {form}", flush=True)
     with mq.Lattice(dims) as G:
+        G.set_small_lattice_form(form)
         lib = G.lib
         lib.milc_hip_dev_invert_noalloc.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_double, ctypes.c_int,
                                                     ctypes.c_double, ctypes.c_int, ctypes.c_int,
@@ -39,7 +41,7 @@ def _compare_on(dims, seed):
         # slot 2 does not exist yet: the allocation-free call must refuse it
         rc, _ = _noalloc(G, 0, 2, 0.05, mq.EVEN, 1e-10, 0)
         assert rc == -3
-        for mixed in (0, 2):
+        for mixed in (0, 1, 2):
             it_a, st_a = G.dev_invert(0, 1, 0.05, mq.EVEN, 1e-10, mixed)
             # give slot 2 stale contents: the solve must zero it itself
             G.dev_write(2, mq.EVEN, np.full((G.V, 3, 2), 7.0))
@@ -57,10 +59,10 @@ def _compare_on(dims, seed):
         assert rc == -2
 
 
-def test_noalloc_matches_allocating_solve_two_calls():
-    _compare_on((8, 8, 8, 16), 1201)
+def test_noalloc_matches_allocating_solve_two_calls(small_form):
+    _compare_on((8, 8, 8, 16), 1201, small_form)
     # second call: a smaller lattice, the scratch still holds the first call's fields
-    _compare_on((4, 4, 4, 8), 1301)
+    _compare_on((4, 4, 4, 8), 1301, small_form)
 
 
 def test_noalloc_rejects_lattice_beyond_scratch():

@@ -1154,6 +1154,7 @@ static int cg_solve_f64(const VecField& src, VecField& x, double mass, const Sol
   h.rsq_stop = rsqmin * source_norm;
   h.relrsq_stop = relrsqmin;
   h.rel_mode = rel ? 1 : 0;
+  h.gone = c.small_form == 2;
   if ((rc = write_scalars(&h))) return rc;
   long iteration = 0;
   int nrestart = 0;

@@ -82,8 +82,8 @@ struct Context {
   size_t staging_elems = 0;
   int block = 256;
   // 1: Krylov loops of small lattices in one kernel; 0: launch by launch and
-  // batched on every lattice; 2: as 1 with a poll limit of one, so that those
-  // kernels give up and the launches take over
+  // batched on every lattice; 2: as 1 with the give-up word set before the
+  // launch, so that those kernels give up and the launches take over
   int small_form = 1;
   bool initialised = false;
 };

@@ -468,6 +468,7 @@ static int multicg_one_kernel(const VecField& src64, std::vector<VecField>& x64,
   h.source_norm = source_norm;
   h.rsqstop = mp.resid * mp.resid * source_norm;
   h.max_iter = (int)std::min<long>(mp.max_iters, 1L << 30);
+  h.gone = c.small_form == 2;
   MH_CHECK(hipMemcpyAsync(dev, hp, bytes, hipMemcpyHostToDevice, c.stream));
   if ((rc = ms_persist(src64, (const VecField*)(dev + head), work, pbit(mp.parity), (MSPersist*)dev))) return rc;
   MH_CHECK(hipMemcpyAsync(&h, dev, sizeof h, hipMemcpyDeviceToHost, c.stream));

@@ -280,7 +280,7 @@ def test_block_multishift_counts_stage_and_refinement(nsrc):
 
 @pytest.mark.parametrize("dims", [(4, 4, 4, 4), (10, 10, 10, 12), (18, 6, 14, 28), (16, 16, 16, 32)])
 def test_given_up_solves_go_on_launch_by_launch(dims):
-    """A one-kernel solve that gives up waiting (form 2: a poll limit of one) is
+    """A one-kernel solve that gives up waiting (form 2: at the first poll) is
     finished by the loops of larger lattices (form 0), with the restarts and
     iterations of those: bit for bit the same solutions and counts."""
     print(f"given up {dims}", flush=True)

@@ -106,9 +106,10 @@ int milc_hip_invert(int external_precision, int internal_precision, double mass,
  * refined to its own FP64 true residual target_resid[j] (the per-shift CG of
  * ks_multicg_hybrid_field), up to four consecutive shifts in one batched mixed
  * CG with an FP32 (mixed_precision 1) or 16-bit (mixed_precision 2) sloppy
- * operator; final_resid[j] is then that true |r|/|b|.  Up to 131072 sites per
- * parity such a call runs the multi-shift in FP64 to the targets and checks
- * every true residual instead.
+ * operator; final_resid[j] is then that true |r|/|b|.  Up to 65536 sites per
+ * parity with one shift, 98304 with up to four, 131072 with more, such a call
+ * runs the multi-shift in FP64 to the targets and checks every true residual
+ * instead.
  * A nonzero target_relresid[j] returns -4: the multi-shift solve has no
  * relative-residual test (the reference glue stops on it,
  * ks_multicg_offset_gpu.c:55-58). */

@@ -609,7 +609,7 @@ extern "C" int milc_hip_multishift_invert(int external_precision, int internal_p
   std::vector<double> res(num_offsets);
   for (int j = 0; j < num_offsets; j++) res[j] = target_resid[j] > 0 ? target_resid[j] : target_resid[0];
   const std::vector<double> offs(offsets, offsets + num_offsets);
-  const bool small = mixed && args.max_iter != 1 && multishift_is_small() && multishift_small_takes(offs, res);
+  const bool small = mixed && args.max_iter != 1 && solved_one_by_one(1, num_offsets) && multishift_small_takes(offs, res);
   int bulk = (internal_precision == 1 || mixed) ? P_F32 : P_F64;
   if (!small && (rc = ensure_links(bulk))) return rc;
   VecField b;
@@ -1177,7 +1177,7 @@ extern "C" int milc_hip_dev_multishift_block(int nsrc, const int* src_slots, int
   if (out_slot0 >= 0 && (out_nsrc < 0 || out_nsrc > nsrc || out_slot0 + out_nsrc * num_offsets > kSlots)) return -2;
   int rc;
   const std::vector<double> offs(offsets, offsets + num_offsets), res(num_offsets, refine_resid);
-  if (refine_resid > 0 && max_iters != 1 && block_is_small(nsrc) && multishift_small_takes(offs, res)) {
+  if (refine_resid > 0 && max_iters != 1 && solved_one_by_one(nsrc, num_offsets) && multishift_small_takes(offs, res)) {
     auto t0 = std::chrono::steady_clock::now();
     std::vector<double> rel(num_offsets), worst(num_offsets, 0.0);
     BlockCounts counts(num_offsets);
@@ -1282,7 +1282,8 @@ extern "C" int milc_hip_multishift_invert_block(int external_precision, int nsrc
   const int pb = pbit(parity);
   int total = 0;
   const std::vector<double> offs(offsets, offsets + num_offsets), res(num_offsets, refine_residual);
-  if (refine_residual > 0 && args.max_iter != 1 && block_is_small(nsrc) && multishift_small_takes(offs, res)) {
+  if (refine_residual > 0 && args.max_iter != 1 && solved_one_by_one(nsrc, num_offsets) &&
+      multishift_small_takes(offs, res)) {
     std::vector<double> rel(num_offsets);
     BlockCounts counts(num_offsets);
     // every source is read before a solution is written, as in the batch: the
@@ -1375,7 +1376,7 @@ extern "C" int milc_hip_invert_block(int external_precision, int nsrc, double ma
   int total = 0;
   // a target that is never met runs to max_iter as a batch (the one-source solve
   // takes one whose square is zero for no target at all)
-  if (std::abs(target_residual) > kNoTarget && block_is_small(nsrc)) {
+  if (std::abs(target_residual) > kNoTarget && solved_one_by_one(nsrc, 0)) {
     SolveParams sp;
     sp.parity = parity;
     sp.max_iters = args.max_iter > 0 ? args.max_iter : 20000;

@@ -233,9 +233,10 @@ struct MultiParams {
 };
 int multicg_solve(const VecField& src, std::vector<VecField>& x, const std::vector<double>& offsets,
                   const MultiParams& mp, SolveStats& st);
-// Whether the mixed multi-shifts of `sources` sources run as multishift_small.
-bool multishift_is_small(int sources = 1);
-// ... and whether their shifts allow it.  A target whose square times |b|^2 may
+// Whether the mixed multi-shifts of `sources` sources run as multishift_small,
+// and block CGs (shifts = 0) in one kernel, one source after another.
+bool solved_one_by_one(int sources, int shifts);
+// ... and whether the shifts allow it.  A target whose square times |b|^2 may
 // be zero is never met, which the recurrence of the one-kernel solve does not
 // survive.  A shift that misses its target is finished by a CG of mass
 // sqrt(offset) / 2; the batched refinement takes any offset.
@@ -249,8 +250,6 @@ bool multishift_small_takes(const std::vector<double>& offsets, const std::vecto
 int multishift_small(const VecField& b, std::vector<VecField>& x, const std::vector<double>& offsets,
                      const double* resid, int parity, int max_iters, long* iters, double* fres, int* converged,
                      int* refine_iters = nullptr);
-// Whether a block call of `sources` sources solves them one after another.
-bool block_is_small(int sources);
 int shift_residuals(const VecField& b, const std::vector<VecField>& x, const double* offsets, int parity, double* rel);
 
 // ---- force outer products ---------------------------------------------------

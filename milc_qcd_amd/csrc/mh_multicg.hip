@@ -493,8 +493,8 @@ int multicg_solve(const VecField& src, std::vector<VecField>& x, const std::vect
   return rc;
 }
 
-bool multishift_is_small(int sources) {
-  return ctx().Vh <= persist_mixed_shift_sites(sources) && persist_shape(ctx().Vh).lps && ctx().links[P_F64].valid;
+bool solved_one_by_one(int sources, int shifts) {
+  return ctx().Vh <= persist_sites(sources, shifts) && persist_shape(ctx().Vh).lps && ctx().links[P_F64].valid;
 }
 
 bool multishift_small_takes(const std::vector<double>& offsets, const std::vector<double>& resid) {
@@ -503,10 +503,6 @@ bool multishift_small_takes(const std::vector<double>& offsets, const std::vecto
   for (double r : resid)
     if (!(r > kNoTarget)) return false;
   return true;
-}
-
-bool block_is_small(int sources) {
-  return ctx().Vh <= persist_block_sites(sources) && persist_shape(ctx().Vh).lps && ctx().links[P_F64].valid;
 }
 
 int multishift_small(const VecField& b, std::vector<VecField>& x, const std::vector<double>& offsets,

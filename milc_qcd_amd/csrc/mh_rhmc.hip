@@ -102,7 +102,7 @@ static int rational_solve(const VecField& phi, int n, const double* offsets, dou
     if ((rc = alloc_vec(x[t], P_F64, c.stride))) return rc;
   std::vector<double> offs(offsets, offsets + n);
   const std::vector<double> res(n, resid);
-  if (mixed && multishift_is_small() && multishift_small_takes(offs, res)) {
+  if (mixed && solved_one_by_one(1, n) && multishift_small_takes(offs, res)) {
     long it = 0;
     if ((rc = multishift_small(phi, x, offs, res.data(), parity, 20000, &it, nullptr, &st.converged))) return rc;
     st.iters = (int)it;
@@ -142,7 +142,7 @@ static int rational_solve_all(const std::vector<const VecField*>& src, const std
     if (o.empty() || (int)o.size() > BMS_MAX) return -2;
     n = std::max(n, (int)o.size());
   }
-  bool small = multishift_is_small(ns);
+  bool small = solved_one_by_one(ns, n);
   for (int r = 0; r < ns; r++) small = small && multishift_small_takes(offs[r], {resid[r]});
   if (small) {
     // one source after another: no padding sources, no refinement

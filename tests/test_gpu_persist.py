@@ -129,9 +129,11 @@ def test_multishift_one_kernel_shift_counts_and_retirement(n, small_form):
                 assert np.linalg.norm(a[s] - b[s]) < 1e-9 * max(np.linalg.norm(b[s]), 1e-300)
 
 
-@pytest.mark.parametrize("dims,nsrc", [((6, 4, 8, 6), 1), ((6, 4, 8, 6), 6), ((6, 4, 8, 6), 7), ((12, 12, 12, 16), 4),
-                                       ((12, 12, 12, 16), 5), ((12, 12, 12, 16), 6), ((6, 4, 8, 6), 9),
-                                       ((6, 4, 8, 6), 12), ((12, 12, 12, 24), 2), ((12, 12, 12, 24), 3)])
+@pytest.mark.parametrize("dims,nsrc", [((6, 4, 8, 6), 1), ((6, 4, 8, 6), 4), ((6, 4, 8, 6), 5), ((6, 4, 8, 6), 6),
+                                       ((6, 4, 8, 6), 7), ((8, 8, 16, 16), 4), ((8, 8, 16, 16), 5), ((8, 8, 16, 16), 6),
+                                       ((12, 12, 12, 16), 3), ((12, 12, 12, 16), 4), ((12, 12, 12, 16), 5),
+                                       ((12, 12, 12, 16), 6), ((6, 4, 8, 6), 9), ((6, 4, 8, 6), 12),
+                                       ((12, 12, 12, 24), 2), ((12, 12, 12, 24), 3), ((16, 16, 16, 24), 2)])
 def test_block_calls_on_both_sides_of_the_dispatch(dims, nsrc):
     """Block CG (with an initial guess) and block multi-shift of one and three
     shifts, just where the sources are solved one after another and just where

@@ -39,7 +39,8 @@ int cg_persist(VecField& x, VecField& r, VecField (&work)[4], int pb, double msq
 // stage and grouped refinement).  ms here / there at the line and beyond it, to
 // a true residual of 1e-6 and to one of 1e-9 (m = 0.03; beyond the line, the
 // sources times the time of one).  The looser target needs less refinement and
-// decides where both matter; tight ones would gain further out.
+// decides, except for two to four shifts of four sources, where the line is even
+// between the two; tight ones alone would gain further out.
 //   1 source, 1 shift    65536  5.1 / 6.0,   7.7 / 9.4    131072 11.7 / 9.5,  18.3 / 15.3
 //             2          98304  9.1 / 9.7,  13.6 / 15.9   131072 12.5 / 10.9, 19.5 / 20.0
 //             9, 12     131072 13.8 / 14.3, 21.6 / 34.2
@@ -50,7 +51,7 @@ int cg_persist(VecField& x, VecField& r, VecField (&work)[4], int pb, double msq
 //             2          16384  4.6 / 5.7,   6.7 / 9.4     24696  7.5 / 6.0,  11.0 / 10.1
 //             9          65536 18.8 / 18.5, 27.8 / 49.7    98304 30.4 / 24.3, 44.1 / 68.9
 //   4         CG, 1      16384  5.4 / 5.4,   7.4 / 7.6     24696  9.8 / 6.5,  13.9 / 8.9
-//             2           8192  5.0 / 5.5,   6.9 / 8.9     13824  6.1 / 5.6,   8.5 / 8.9
+//             2          16384  6.3 / 5.7,   8.9 / 9.3     24696 10.0 / 5.9,  14.6 / 10.0
 //             5, 9       16384  6.9 / 7.6,   9.6 / 15.4    24696 11.8 / 9.9,  17.4 / 25.4
 //   5         CG          8192  5.3 / 5.5,   7.1 / 7.9     13824  6.4 / 6.2,   8.5 / 8.1
 //             2           8192  6.2 / 7.3,   8.6 / 11.8    13824  7.6 / 7.3,  10.6 / 11.3
@@ -61,7 +62,7 @@ constexpr int persist_sites(int sources, int shifts) {
     case 1: return shifts <= 1 ? 65536 : (shifts <= 4 ? 98304 : 131072);
     case 2: return shifts == 0 ? 49152 : (shifts < 9 ? 65536 : 98304);
     case 3: return shifts < 9 ? 16384 : 65536;
-    case 4: return shifts >= 2 && shifts <= 4 ? 8192 : 16384;
+    case 4: return 16384;
     case 5: return 8192;
     case 6: return shifts == 0 ? 0 : 8192;
   }

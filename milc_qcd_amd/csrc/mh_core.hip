@@ -855,8 +855,9 @@ __global__ void k_cg_relcheck(const double* __restrict__ partials_rr, int nblock
 // updated fields go to the second record slot (d_congrad5_fn_milc.c:351-352).
 // Bound by HBM (152 B per site with a 16-bit p).  Site blocks in the stencils'
 // XCD order, so that a block's p is written through the L2 that reads it in the
-// next stencil: 32^3x64 mixed CG 94.18 -> 93.56 ms (1.006 to 1.007 in three
-// comparisons, runs of one side within 0.3%) against the plain block order.
+// next stencil: 32^3x64 mixed CG 94.18 -> 93.56 ms against the plain block order
+// (1.006 to 1.007 in four comparisons, sides in turn; less than the same build
+// differs by between cards).
 template <int PP, int PA, int REL>
 __global__ void __launch_bounds__(256) k_cg_update(VecField x, VecField p, VecField r, VecField ttt, int Vh,
                                                    const CGScalars* __restrict__ sc, double* __restrict__ partials_rr) {

@@ -882,9 +882,11 @@ __device__ __forceinline__ void sf_term(const LinkField& U, const SfSites& n, in
 }
 // The two 5-staples whose outer direction is nu and the 7-staples' FU part of
 // the same direction (argument SS, force F), one update of FU (48^3x96, pairs
-// without / with t: 6.7 / 8.1 ms against 6.9 / 8.4 in three passes, though it
-// moves a quarter less: the L2 misses of the neighbour reads bound it, and two
-// or one workgroup fewer per CU did not help):
+// without / with t: 6.7 / 8.1 ms against 6.9 / 8.4 in three passes).  Bound by
+// the L2 misses of the neighbour reads: its algorithmic bytes are a quarter
+// fewer, but 51.5 / 57.1 GB leave the L2s (2.6 / 2.9 times the algorithmic, at
+// 7.7 / 7.1 TB/s) where the three passes moved 43.8 / 53.5; two or one
+// workgroup fewer per CU did not help.
 //   FA_k (+)= cg FA_nu(Gs_k),  FU += cg sum_k FU_nu(A_k, Gs_k) + c7 FU_nu(SS, F)
 template <int MU, int NU, int TT>
 __global__ void __launch_bounds__(128) k_sf_adj5(Geom g, LinkField U, SfTerm s0, SfTerm s1, double cg, MF F,

@@ -8,7 +8,10 @@
 // the site of the same index of the other parity, and keeps r, x, p of the
 // site and as many of its links as fit in registers and LDS over all
 // iterations; only the two stencil sources (p, D p) and one record of partial
-// sums per workgroup go through memory.
+// sums per workgroup go through memory.  Bound by the latency of the exchanges
+// on the smallest lattices (8^4: 1.5 MB out of the L2s in 7.7 us) and by the
+// links that do not fit the CU on the largest (16^3x32: 263 MB per iteration,
+// 25 of a site's 32 matrices, from the Infinity Cache at 6.2 TB/s).
 //
 // Exchange without barriers: a shared value is one 8-byte word, written and
 // read with relaxed agent-scope accesses (they meet in the memory-side cache,

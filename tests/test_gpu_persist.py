@@ -310,3 +310,21 @@ def test_given_up_solves_go_on_launch_by_launch(dims):
         assert conv
         for j in range(len(offs)):
             assert G.dev_diff(20 + j, 10 + j) < 10 * 2e-9 / offs[j]
+
+
+def test_small_lattice_form_is_checked_and_belongs_to_the_context():
+    """Values other than 0, 1 and 2 are refused, and a new context starts with 1:
+    a single source's block multi-shift has no stencil variant (-1) there."""
+    dims, variant = (4, 4, 4, 4), []
+    for form in (0, None):
+        with mq.Lattice(dims) as G:
+            assert G.lib.milc_hip_set_small_lattice_form(3) == -2
+            assert G.lib.milc_hip_set_small_lattice_form(-1) == -2
+            if form is not None:
+                G.set_small_lattice_form(form)
+            G.dev_gauge_hisq(1480)
+            G.dev_source(1481, mq.EVEN, 0)
+            st = G.dev_multishift_block([0], [0.1, 0.5], 1e-6, 1e-9)
+            assert st["converged"]
+            variant.append(st["variant"])
+    assert variant[0] >= 0 and variant[1] == -1
